@@ -982,7 +982,7 @@ struct SphAdj {
     if (do_split || do_merge) {  // the energy decides split and merge (SPH-3D-2/sph_system.cpp:356)
       launch_make_erec(S, cap, aux.erec, st, nd);
       launch_energy(SPH_V3D2, P, S, t.cs, t.ce, cap, st, nullptr, kEnergyListDefault,
-                    do_split ? flag_by_slot : nullptr, aux.erec, nd);
+                    do_split ? flag_by_slot : nullptr, aux.erec, nd, aux.fine_energy);
     }
     if (do_split) {
       sph_exclusive_scan(flag_by_slot, rank_by_slot, nd, cap, &cnt->scan_total, scan_tmp, st);
@@ -1103,6 +1103,7 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
             a->alloc(a->B.vbar, cap) && a->alloc(a->B.ebar, cap) && a->alloc(a->B.rbar, cap) &&
             a->alloc(a->aos_dev, cap * sizeof(SphParticle3D));
   a->aux.nbl_stride = (uint)cap;
+  a->aux.choose_forms(SPH_V3D2, false, flags & SPH_STEP_SPLIT ? 2 * n : n);
   a->sc.scan_tmp = a->scan_tmp;
   a->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && hipHostMalloc((void **)&a->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess) ok = false;

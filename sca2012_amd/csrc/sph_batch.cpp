@@ -382,6 +382,7 @@ struct SphBatch {
     const uint mb = dev ? (uint)phys_cap : m;  // entries, removed ones included
     const uint *n_live = dev ? &cnt->n : nullptr;   // live entries at the start of the step
     const uint *n_pre = dev ? &cnt->n_pre : nullptr;  // the same, once split has moved n
+    aux.choose_forms(v, true, M);  // M: the live count at the call's start, also for a graph
     launch_batch_begin(bv, cnt, st);
     pbegin(SPH_P_HASH);
     launch_hash(v, P0, cur, &cnt->m, mb, keys, s2p_hash, cnt, st, &bv, grid);
@@ -417,7 +418,8 @@ struct SphBatch {
     DevParams Pe = P0;  // the energy kernel's unit-length path only if every scene takes it
     Pe.energy_unit = energy_unit_all() ? 1 : 0;
     auto energy = [&](int c) {
-      launch_energy(v, Pe, cur, cstart, cend, Mb, st, &bv, c, split_flags, aux.erec, n_live);
+      launch_energy(v, Pe, cur, cstart, cend, Mb, st, &bv, c, split_flags, aux.erec, n_live,
+                    aux.fine_energy);
     };
     if (dev) energy(le);
     else tune.run(1, st, energy);
@@ -448,9 +450,10 @@ struct SphBatch {
   // The graph of one step with this shape, flags and state-buffer parity (captured on first
   // use). Returns nullptr if capture or instantiation failed.
   hipGraphExec_t graph_for(uint flags, const int shape[3]) {
+    aux.choose_forms(variant, true, M);
     const uint key = (flags & 3u) | ((uint)shape[0] << 2) | ((uint)shape[1] << 4) |
                      ((uint)shape[2] << 6) | ((parity ? 1u : 0u) << 8) |
-                     ((energy_unit_all() ? 1u : 0u) << 9);
+                     ((energy_unit_all() ? 1u : 0u) << 9) | (aux.forms() << 10);
     for (auto &g : graphs)
       if (g.key == key) return g.exec;
     const uint grid = kGridPerCU[shape[0]] * num_cu;

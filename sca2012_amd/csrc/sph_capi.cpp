@@ -473,6 +473,7 @@ struct SphCtx {
   }
   void q_density() {
     pbegin(SPH_P_DENSITY);
+    aux.choose_forms(variant, false, n);
     launch_density(variant, P, cur, aux, cstart, cend, n, st);
     pend();
     nbl_ok = true;
@@ -481,6 +482,7 @@ struct SphCtx {
   void q_force(bool tuned = false) {
     pbegin(SPH_P_FORCE);
     const bool use = nbl_ok;
+    aux.choose_forms(variant, false, n);
     auto go = [&](int c) {
       launch_force(variant, P, cur, aux, cstart, cend, n, st, nullptr, c, nullptr, use);
     };
@@ -503,8 +505,10 @@ struct SphCtx {
       launch_make_erec(cur, n, aux.erec, st);
       erec_ok = true;
     }
+    aux.choose_forms(variant, false, n);
     auto go = [&](int c) {
-      launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, flags, aux.erec);
+      launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, flags, aux.erec, nullptr,
+                    aux.fine_energy);
     };
     if (tuned) tune.run(1, st, go);
     else go(tune.energy);

@@ -87,6 +87,30 @@ struct Aux {
   uint *nbl = nullptr;
   uint *nbl_cnt = nullptr;
   uint nbl_stride = 0;
+  // which form of the neighbour kernels runs (choose_forms): several lanes per particle
+  // (sph_fine.hip) or one thread (sph_kernels.hip)
+  bool fine_density = false, fine_force = false, fine_energy = false;
+
+  // For n live particles of a scene or of a batch's scenes together. Several lanes per
+  // particle shorten the chain of dependent loads and cost more instructions, so density and
+  // energy are chosen by whether n threads fill the GPU. Measured (one thread -> several
+  // lanes, us): density 3D-2 25k particles 70 -> 28, 118k 73 -> 63, 206k 80 -> 99; 3D-4 64k
+  // 100 -> 80, 214k 133 -> 222; 2D 17k 19 -> 12, 66k 19 -> 24. Energy 3D-2 25k 88 -> 26, 206k
+  // 100 -> 87, 330k 112 -> 123; 3D-4 64k 174 -> 91, 214k 215 -> 248; 2D 66k 25 -> 17, 264k
+  // 28 -> 42. Force evaluates the same pairs either way, with one pair's registers instead of
+  // four: 3D-2 25k 36 -> 15, 498k 107 -> 91; 3D-4 506k 219 -> 134, 1.7M 501 -> 392, 4.2M
+  // shrinking to 2M 732 -> 717; 2D 66k 15 -> 13, 264k 24 -> 30; in a batch, whose lanes each
+  // load their scene's parameters, 126k 49 -> 39, 400k 41 -> 52.
+  void choose_forms(int variant, bool batch, uint n) {
+    const bool d3 = variant != SPH_V2D;
+    fine_density = n <= (d3 ? 100000u : 32000u);
+    fine_energy = n <= (d3 ? 180000u : 128000u);
+    fine_force = n <= (d3 ? (batch ? 150000u : 6000000u) : 100000u);
+  }
+  // the forms as bits (a captured step depends on them)
+  uint forms() const {
+    return (fine_density ? 1u : 0u) | (fine_force ? 2u : 0u) | (fine_energy ? 4u : 0u);
+  }
 };
 
 struct DevState {
@@ -376,7 +400,19 @@ void launch_integrate(int variant, const DevParams &P, DevState s, uint n, hipSt
 // integrate kernel, or by launch_make_erec), read for the neighbours' pair terms
 void launch_energy(int variant, const DevParams &P, DevState s, const uint *cstart,
                    const uint *cend, uint n, hipStream_t st, const BatchView *bv, int cfg,
-                   uint *flag_by_slot, const float4 *erec, const uint *n_dev = nullptr);
+                   uint *flag_by_slot, const float4 *erec, const uint *n_dev = nullptr,
+                   bool fine = false);
+// the same phases in several lanes per particle (launch_density, launch_force and launch_energy
+// call these as Aux::choose_forms says)
+void launch_density_fine(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
+                         const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                         const uint *n_dev);
+void launch_force_fine(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
+                       const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                       const uint *n_dev, bool use_nbl);
+void launch_energy_fine(int variant, const DevParams &P, DevState s, const uint *cstart,
+                        const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                        uint *flag_by_slot, const float4 *erec, const uint *n_dev);
 void launch_make_erec(DevState s, uint n, float4 *erec, hipStream_t st,
                       const uint *n_dev = nullptr);
 void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *flag_by_slot,
