@@ -864,6 +864,7 @@ struct SphAdj {
   Aux aux{};
   uint *keys = nullptr, *vals = nullptr, *skeys = nullptr, *svals = nullptr;
   SortScratch sc{};
+  BinScratch bins{};
   uint *s2p_hash = nullptr, *s2p_cell = nullptr, *cs_scr = nullptr, *ce_scr = nullptr;
   uint *flag_by_slot = nullptr, *rank_by_slot = nullptr, *alive_by_slot = nullptr;
   uint *newslot = nullptr, *status = nullptr;
@@ -965,16 +966,27 @@ struct SphAdj {
     return hipMemcpyAsync(dst, src, sizeof(Counters), hipMemcpyDeviceToDevice, st);
   }
 
+  // state S (counters in cnt) into cell order: T, lists cs, ce (sph_bins.hip)
+  void bin(DevState S, DevState T, uint *cs, uint *ce, int par, bool keep_err, bool set_m) {
+    launch_bin_count(SPH_V3D2, P, S, bins, cnt, cap, par, st);
+    launch_bin_table(bins, cells, cs, ce, cnt, par, st, true, keep_err);
+    launch_bin_place(S, bins, cs, cnt, cap, st);
+    launch_bin_reorder(S, T, bins, cs, ce, sc.keys_alt, sc.vals_alt, s2p_cell, cnt, cap, st, true, set_m);
+  }
   // one forward step of state S (counters in cnt): cell order into the tape entry, next
   // state back into S; no host round trip
-  void fwd_step(DevState S, const Tape &t) {
+  void fwd_step(DevState S, const Tape &t, uint step) {
     const uint *nd = &cnt->n;
-    launch_begin_step(cnt, st);  // n_pre = n, split and merge counters cleared
-    launch_hash(SPH_V3D2, P, S, &cnt->m, cap, keys, s2p_hash, cnt, st);
-    sph_radix_sort(keys, vals, cap, kbits, sc, &skeys, &svals, st, nd);
-    sph_fill_cells(t.cs, t.ce, cells, st);
-    launch_cell_bounds(skeys, cap, cells, t.cs, t.ce, st, nd);
-    launch_reorder(S, t.T, svals, s2p_hash, cap, s2p_cell, st, cnt, true, nd);  // and m = n
+    if (bins.ccount) {
+      bin(S, t.T, t.cs, t.ce, (int)(step & 1u), false, true);  // and m = n, n_pre = n, ...
+    } else {
+      launch_begin_step(cnt, st);  // n_pre = n, split and merge counters cleared
+      launch_hash(SPH_V3D2, P, S, &cnt->m, cap, keys, s2p_hash, cnt, st);
+      sph_radix_sort(keys, vals, cap, kbits, sc, &skeys, &svals, st, nd);
+      sph_fill_cells(t.cs, t.ce, cells, st);
+      launch_cell_bounds(skeys, cap, cells, t.cs, t.ce, st, nd);
+      launch_reorder(S, t.T, svals, s2p_hash, cap, s2p_cell, st, cnt, true, nd);  // and m = n
+    }
     launch_density(SPH_V3D2, P, t.T, aux, t.cs, t.ce, cap, st, nullptr, nd);
     launch_force(SPH_V3D2, P, t.T, aux, t.cs, t.ce, cap, st, nullptr, kForceListDefault, nd, true);
     k_adj_integrate_fwd<<<agrid(cap), ABLK, 0, st>>>(P, theta, nf, t.T, S, nd, cap);
@@ -1021,14 +1033,18 @@ struct SphAdj {
     k_adj_density_bwd<<<g, ABLK, 0, st>>>(P, t.T, t.cs, t.ce, B, ap, av, ae, t.tc, cap);
   }
   // final state -> cell order in scratch (lists cs_scr/ce_scr), sample, loss
-  void final_sample() {
+  void final_sample(uint step) {
     const uint *nd = &cnt->n;
-    launch_hash(SPH_V3D2, P, cur, &cnt->m, cap, keys, s2p_hash, cnt, st);
-    sph_radix_sort(keys, vals, cap, kbits, sc, &skeys, &svals, st, nd);
-    sph_fill_cells(cs_scr, ce_scr, cells, st);
-    launch_cell_bounds(skeys, cap, cells, cs_scr, ce_scr, st, nd);
     // cnt->m keeps the entries of cur (merged-away ones included)
-    launch_reorder(cur, scratch, svals, s2p_hash, cap, s2p_cell, st, nullptr, true, nd);
+    if (bins.ccount) {
+      bin(cur, scratch, cs_scr, ce_scr, (int)(step & 1u), true, false);
+    } else {
+      launch_hash(SPH_V3D2, P, cur, &cnt->m, cap, keys, s2p_hash, cnt, st);
+      sph_radix_sort(keys, vals, cap, kbits, sc, &skeys, &svals, st, nd);
+      sph_fill_cells(cs_scr, ce_scr, cells, st);
+      launch_cell_bounds(skeys, cap, cells, cs_scr, ce_scr, st, nd);
+      launch_reorder(cur, scratch, svals, s2p_hash, cap, s2p_cell, st, nullptr, true, nd);
+    }
     k_adj_sample<<<dim3(nvb), ABLK, 0, st>>>(P, ns, scratch.pos, cs_scr, ce_scr, target, sample,
                                              resid, part);
     k_adj_loss_sum<<<1, ABLK, 0, st>>>(part, nvb, loss_dev);
@@ -1106,6 +1122,13 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
   a->aux.choose_forms(SPH_V3D2, false, flags & SPH_STEP_SPLIT ? 2 * n : n);
   a->sc.scan_tmp = a->scan_tmp;
   a->sc.max_tiles = sph_sort_tiles(cap);
+  if (ok && sph_use_bins(a->cells, cap)) {
+    a->bins.hkey = a->keys;
+    a->bins.rank = a->vals;
+    a->bins.bslot = a->s2p_hash;
+    ok = a->alloc(a->bins.ccount, a->cells) && a->alloc(a->bins.tmp, sph_bin_tiles(a->cells));
+    if (ok) sph_fill_u32(a->bins.ccount, 0u, a->cells, a->st);
+  }
   if (ok && hipHostMalloc((void **)&a->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess) ok = false;
   if (ok && hipHostMalloc((void **)&a->loss_host, sizeof(float), hipHostMallocDefault) != hipSuccess) ok = false;
   if (ok && (hipEventCreate(&a->e0) != hipSuccess || hipEventCreate(&a->e1) != hipSuccess)) ok = false;
@@ -1182,11 +1205,11 @@ int sph_adj_forward(SphAdj *a, const float *theta_dev, uint32_t steps, float *sa
         return SPH_EHIP;
     }
     const SphAdj::Tape &tp = record ? a->tape[t] : a->tape[0];
-    a->fwd_step(a->cur, tp);
+    a->fwd_step(a->cur, tp, t);
     if (hipMemcpyAsync(a->topo_dev + t, tp.tc, sizeof(TapeCnt), hipMemcpyDeviceToDevice, st) != hipSuccess)
       return SPH_EHIP;
   }
-  a->final_sample();
+  a->final_sample(steps);
   if (sample_dev &&
       hipMemcpyAsync(sample_dev, a->sample, sizeof(float) * a->nvox, hipMemcpyDefault, st) != hipSuccess)
     return SPH_EHIP;
@@ -1230,7 +1253,7 @@ int sph_adj_backward(SphAdj *a, float *dtheta_dev) {
       const SphAdj::Ckpt &c = a->ckpts[seg];
       if (a->copy_state(a->scratch, c.S, false) != hipSuccess || a->copy_cnt(a->cnt, c.c) != hipSuccess)
         return SPH_EHIP;
-      for (uint j = 0; j < len; j++) a->fwd_step(a->scratch, a->tape[j]);
+      for (uint j = 0; j < len; j++) a->fwd_step(a->scratch, a->tape[j], t0 + j);
       for (uint j = len; j-- > 0;) a->bwd_step(a->tape[j]);
     }
   }

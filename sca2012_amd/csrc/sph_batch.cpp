@@ -206,6 +206,7 @@ struct SphBatch {
   Aux aux{};
   uint *keys = nullptr, *vals = nullptr;
   SortScratch sc{};
+  BinScratch bins{};
   uint *skeys = nullptr, *svals = nullptr;
   uint *s2p_hash = nullptr, *s2p_cell = nullptr;
   uint *cstart = nullptr, *cend = nullptr;
@@ -384,20 +385,38 @@ struct SphBatch {
     const uint *n_pre = dev ? &cnt->n_pre : nullptr;  // the same, once split has moved n
     aux.choose_forms(v, true, M);  // M: the live count at the call's start, also for a graph
     launch_batch_begin(bv, cnt, st);
-    pbegin(SPH_P_HASH);
-    launch_hash(v, P0, cur, &cnt->m, mb, keys, s2p_hash, cnt, st, &bv, grid);
-    pend();
-    pbegin(SPH_P_SORT);
-    sph_radix_sort(keys, vals, Mb, kbits, sc, &skeys, &svals, st, n_live, grid);
-    pend();
-    pbegin(SPH_P_CELLS);
-    sph_fill_cells(cstart, cend, total_cell, st);
-    launch_cell_bounds(skeys, Mb, total_cell, cstart, cend, st, n_live, grid);
-    pend();
-    pbegin(SPH_P_REORDER);
-    // and m = n; acc, dp and energy are recomputed by the step's kernels below
-    launch_reorder(cur, alt, svals, s2p_hash, Mb, s2p_cell, st, cnt, false, n_live, grid);
-    pend();
+    if (bins.ccount) {
+      skeys = sc.keys_alt;
+      svals = sc.vals_alt;
+      pbegin(SPH_P_HASH);
+      launch_bin_count(v, P0, cur, bins, cnt, mb, 0, st, &bv, grid);
+      pend();
+      pbegin(SPH_P_CELLS);
+      launch_bin_table(bins, total_cell, cstart, cend, cnt, 0, st, false);
+      pend();
+      pbegin(SPH_P_SORT);
+      launch_bin_place(cur, bins, cstart, cnt, mb, st, grid);
+      pend();
+      pbegin(SPH_P_REORDER);
+      // and m = n; acc, dp and energy are recomputed by the step's kernels below
+      launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, mb, st, false, true,
+                         &bv, grid);
+      pend();
+    } else {
+      pbegin(SPH_P_HASH);
+      launch_hash(v, P0, cur, &cnt->m, mb, keys, s2p_hash, cnt, st, &bv, grid);
+      pend();
+      pbegin(SPH_P_SORT);
+      sph_radix_sort(keys, vals, Mb, kbits, sc, &skeys, &svals, st, n_live, grid);
+      pend();
+      pbegin(SPH_P_CELLS);
+      sph_fill_cells(cstart, cend, total_cell, st);
+      launch_cell_bounds(skeys, Mb, total_cell, cstart, cend, st, n_live, grid);
+      pend();
+      pbegin(SPH_P_REORDER);
+      launch_reorder(cur, alt, svals, s2p_hash, Mb, s2p_cell, st, cnt, false, n_live, grid);
+      pend();
+    }
     swap_state();
     pbegin(SPH_P_DENSITY);
     launch_density(v, P0, cur, aux, cstart, cend, Mb, st, &bv, n_live);
@@ -592,6 +611,13 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
             b->alloc(b->scan_tmp, sph_scan_tmp_elems(scan_n)) && b->alloc(b->sc.len_dev, 1);
   b->aux.nbl_stride = (uint)cap;
   b->sc.scan_tmp = b->scan_tmp;
+  if (ok && sph_use_bins(b->total_cell, cap)) {
+    b->bins.hkey = b->keys;
+    b->bins.rank = b->vals;
+    b->bins.bslot = b->s2p_hash;
+    ok = b->alloc(b->bins.ccount, b->total_cell) && b->alloc(b->bins.tmp, sph_bin_tiles(b->total_cell));
+    if (ok) sph_fill_u32(b->bins.ccount, 0u, b->total_cell, b->st);
+  }
   b->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && hipHostMalloc((void **)&b->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
     ok = false;

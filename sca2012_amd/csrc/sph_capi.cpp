@@ -295,6 +295,8 @@ struct SphCtx {
   std::vector<void *> allocs;
   uint *keys = nullptr, *vals = nullptr;
   SortScratch sc{};
+  BinScratch bins{};
+  int par = 0;  // parity of the step (counting path)
   uint *s2p_hash = nullptr, *s2p_cell = nullptr;
   uint *cstart = nullptr, *cend = nullptr;
   uint *flag_by_slot = nullptr, *rank_by_slot = nullptr, *alive_by_slot = nullptr;
@@ -470,6 +472,36 @@ struct SphCtx {
     DevState t = cur;
     cur = alt;
     alt = t;
+  }
+  // hash, sort, cell ranges and reorder of a step: by counting where the grid suits it
+  void q_bin_step() {
+    if (!bins.ccount || !sph_use_bins(P.total_cell, n)) {
+      q_hash();
+      q_sort();
+      q_cells(true);
+      return;
+    }
+    nbl_ok = false;
+    erec_ok = false;
+    cells_keys = nullptr;  // every table entry is written again
+    cells_clean = false;
+    par ^= 1;
+    skeys = sc.keys_alt;
+    svals = sc.vals_alt;
+    n_sorted = n;
+    pbegin(SPH_P_HASH);
+    launch_bin_count(variant, P, cur, bins, cnt, m, par, st);
+    pend();
+    pbegin(SPH_P_CELLS);
+    launch_bin_table(bins, P.total_cell, cstart, cend, cnt, par, st);
+    pend();
+    pbegin(SPH_P_SORT);
+    launch_bin_place(cur, bins, cstart, cnt, m, st);
+    pend();
+    pbegin(SPH_P_REORDER);
+    launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, m, st, false);
+    pend();
+    std::swap(cur, alt);
   }
   void q_density() {
     pbegin(SPH_P_DENSITY);
@@ -654,6 +686,14 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
   size_t scan_elems = sph_scan_tmp_elems(std::max(scan_n, c->ncube));
   ok = ok && c->alloc(c->scan_tmp, scan_elems);
   c->sc.scan_tmp = c->scan_tmp;
+  if (ok && sph_use_bins(c->P.total_cell, cap)) {
+    c->bins.hkey = c->keys;
+    c->bins.rank = c->vals;
+    c->bins.bslot = c->s2p_hash;
+    ok = c->alloc(c->bins.ccount, c->P.total_cell) &&
+         c->alloc(c->bins.tmp, sph_bin_tiles(c->P.total_cell));
+    if (ok) sph_fill_u32(c->bins.ccount, 0u, c->P.total_cell, c->st);
+  }
   c->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && hipHostMalloc((void **)&c->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
     ok = false;
@@ -857,9 +897,7 @@ int sph_marching_cubes(SphCtx *ctx, uint32_t *n_tri) {
 int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
   CHECK_CTX(ctx);
   if (ctx->n == 0) return SPH_EEMPTY;
-  ctx->q_hash();
-  ctx->q_sort();
-  ctx->q_cells(true);
+  ctx->q_bin_step();
   ctx->q_density();
   ctx->q_force(true);
   ctx->q_integrate();

@@ -1,5 +1,6 @@
-// Device helpers shared by the step's kernel files (sph_kernels.hip, sph_fine.hip): work-item
-// mapping, the variants' compile-time properties, cell arithmetic and the neighbour order.
+// Device helpers shared by the step's kernel files (sph_kernels.hip, sph_fine.hip, sph_bins.hip,
+// sph_prims.hip): work-item mapping, the variants' compile-time properties, cell arithmetic, the
+// neighbour order and block scans.
 #ifndef SPH_DEVICE_H
 #define SPH_DEVICE_H
 
@@ -148,6 +149,32 @@ __device__ inline void nb_range(const DevParams &P, int o, const uint c[3],
 // pairs are summed, so every length gives the same bits; the autotuner picks one per
 // kernel (sph_internal.h: kForceLists, kEnergyLists).
 __device__ inline uint pack_entry(int o, uint j) { return ((uint)o << 27) | j; }
+
+__device__ inline uint wave_incl_scan(uint x, int lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    uint y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  return x;
+}
+
+// Exclusive scan of one value per thread across the block; returns the block total.
+__device__ inline uint block_excl_scan(uint x, uint *lds_waves, uint &total) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  uint inc = wave_incl_scan(x, lane);
+  if (lane == 63) lds_waves[w] = inc;
+  __syncthreads();
+  uint before = 0, tot = 0;
+  for (int k = 0; k < (int)(blockDim.x >> 6); k++) {
+    uint v = lds_waves[k];
+    if (k < w) before += v;
+    tot += v;
+  }
+  __syncthreads();
+  total = tot;
+  return before + inc - x;
+}
 
 }  // namespace
 

@@ -10,7 +10,7 @@
 // All integer work, no floating point, results independent of scheduling.
 #include <mutex>
 
-#include "sph_internal.h"
+#include "sph_device.h"
 
 namespace {
 
@@ -25,32 +25,6 @@ constexpr int SORT_THREADS = 256;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
 constexpr int SORT_ITEMS = 4;
 constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;  // 1024 keys per tile (more tiles fill the GPU)
-
-__device__ inline uint wave_incl_scan(uint x, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    uint y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  return x;
-}
-
-// Exclusive scan of one value per thread across the block; returns the block total.
-__device__ inline uint block_excl_scan(uint x, uint *lds_waves, uint &total) {
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  uint inc = wave_incl_scan(x, lane);
-  if (lane == 63) lds_waves[w] = inc;
-  __syncthreads();
-  uint before = 0, tot = 0;
-  for (int k = 0; k < (int)(blockDim.x >> 6); k++) {
-    uint v = lds_waves[k];
-    if (k < w) before += v;
-    tot += v;
-  }
-  __syncthreads();
-  total = tot;
-  return before + inc - x;
-}
 
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const uint *__restrict__ in,
                                                               const uint *n_dev, uint n_host,
