@@ -24,13 +24,23 @@ constexpr uint CS_TILE = BLK * CS_ITEMS;    // 2048 cells per block
 constexpr uint SCAN1_THREADS = 1024, SCAN1_TILE = SCAN1_THREADS * CS_ITEMS;
 constexpr uint SCAN1_CELLS = SCAN1_TILE;  // a second round costs more than a second launch (7.2 us at 13,824)
 
+// A block's entries are counted in LDS first, in a hash table of their cells, so the cell
+// counters see one atomic per block and cell instead of one per entry: consecutive entries were
+// neighbours a step ago. Atomics that return a value ran at 12.5 G/s whatever the order of the
+// blocks: 498k particles 38.7 -> 17.7 us, 3.2M in a batch 75 -> 48 us, 14k 4.9 -> 4.6 us. Four
+// entries per thread (a table of 2048 places) were slower, 22.6 and 62 us.
+constexpr uint CT = 2 * BLK;  // table places; at most BLK are taken, so every search ends
+static_assert(CT == 512, "k_bin_count's hash gives 9 bits");
+
 template <int V, bool B>
 __global__ __launch_bounds__(BLK) void k_bin_count(DevParams P0, const DevParams *__restrict__ Ptab,
                                                    SceneCnt *scn, const float4 *__restrict__ pos,
                                                    const uint *__restrict__ slot, uint m_host,
                                                    uint *__restrict__ hkey, uint *__restrict__ rank,
                                                    uint *__restrict__ ccount, Counters *cnt, int par) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  __shared__ uint tcell[CT], tcnt[CT];
+  const uint t = threadIdx.x;
+  if (blockIdx.x == 0 && t == 0) {
     cnt->m_in = cnt->m;  // the entries of this step: m itself changes in k_bin_reorder
     if (!B) {            // the step's counters start over (no thread here reads them)
       cnt->n_pre = cnt->n;
@@ -38,26 +48,47 @@ __global__ __launch_bounds__(BLK) void k_bin_count(DevParams P0, const DevParams
       cnt->err2[par ^ 1] = 0u;
     }
   }
-  for_each_item<false>(min(cnt->m, m_host), [&](const uint k) {
-    const uint w = slot[k];
-    if (w == SPH_DEAD) return;
-    const DevParams &P = scene_params<B>(P0, Ptab, w);
-    const float4 p = pos[k];
-    uint c[3];
-    uint h = P.cell_base;
-    if (cell_of<V>(P, p.x, p.y, p.z, c)) {
-      h += c[2] * P.ncell[0] * P.ncell[1] + c[1] * P.ncell[0] + c[0];
-    } else {  // the scene's cell 0 keeps every later access in bounds
-      if (B) {
-        atomicOr(&cnt->err, 1u);
-        atomicOr(&scn[w >> SPH_SCENE_SHIFT].err, 1u);
-      } else {
-        atomicOr(&cnt->err2[par], 1u);
+  const uint m = min(cnt->m, m_host), nvb = (m + BLK - 1) / BLK;
+  for (uint vb = blockIdx.x; vb < nvb; vb += gridDim.x) {
+    const uint k = vb * BLK + t;
+    const uint w = k < m ? slot[k] : SPH_DEAD;
+    const bool live = w != SPH_DEAD;
+    tcell[t] = tcell[t + BLK] = SPH_EMPTY;
+    tcnt[t] = tcnt[t + BLK] = 0u;
+    uint h = 0u, at = 0u, r = 0u;
+    if (live) {
+      const DevParams &P = scene_params<B>(P0, Ptab, w);
+      const float4 p = pos[k];
+      uint c[3];
+      h = P.cell_base;
+      if (cell_of<V>(P, p.x, p.y, p.z, c)) {
+        h += c[2] * P.ncell[0] * P.ncell[1] + c[1] * P.ncell[0] + c[0];
+      } else {  // the scene's cell 0 keeps every later access in bounds
+        if (B) {
+          atomicOr(&cnt->err, 1u);
+          atomicOr(&scn[w >> SPH_SCENE_SHIFT].err, 1u);
+        } else {
+          atomicOr(&cnt->err2[par], 1u);
+        }
       }
+      hkey[k] = h;
     }
-    hkey[k] = h;
-    rank[k] = atomicAdd(&ccount[h], 1u);
-  });
+    __syncthreads();
+    if (live) {
+      at = (h * 0x9e3779b1u) >> 23;  // the top 9 bits: CT places
+      for (;; at = (at + 1u) % CT) {
+        const uint was = atomicCAS(&tcell[at], SPH_EMPTY, h);
+        if (was == SPH_EMPTY || was == h) break;
+      }
+      r = atomicAdd(&tcnt[at], 1u);
+    }
+    __syncthreads();
+    for (uint x = t; x < CT; x += BLK)
+      if (tcnt[x]) tcnt[x] = atomicAdd(&ccount[tcell[x]], tcnt[x]);
+    __syncthreads();
+    if (live) rank[k] = tcnt[at] + r;
+    __syncthreads();  // the table starts over
+  }
 }
 
 // counts [c, c + 8) of the table, cleared for the next step; 0 past its end
@@ -184,7 +215,9 @@ __global__ __launch_bounds__(BLK) void k_bin_reorder(DevState src, DevState dst,
                                                      bool all, bool set_m, uint *__restrict__ init0,
                                                      uint *__restrict__ init1) {
   if (set_m && blockIdx.x == 0 && threadIdx.x == 0) cnt->m = cnt->n;  // physical == live
-  for_each_item<false>(min(cnt->m_in, m_host), [&](const uint k) {
+  // XCD-contiguous blocks keep a single scene's destinations in one L2 (498k: 24.4 -> 22 us); a
+  // batch's were slower that way (81 -> 96 us)
+  for_each_item<!B>(min(cnt->m_in, m_host), [&](const uint k) {
     const uint w = src.slot[k];
     if (w == SPH_DEAD) return;
     const float4 p = src.pos[k], v = src.vel[k], e = src.ev[k];
