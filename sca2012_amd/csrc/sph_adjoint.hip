@@ -214,23 +214,6 @@ __global__ void k_adj_rec_counts(const Counters *cnt, TapeCnt *tc) {
   tc->groups = cnt->groups;
 }
 
-// split child of entry k (cell order, k < n_pre): the parent of split rank r writes its
-// child at n_pre + r (the 1 -> 2 split, SPH-3D-2/sph_system.cu:1576-1615)
-__global__ __launch_bounds__(ABLK) void k_adj_rec_split(DevState S, const uint *__restrict__ flag_by_slot,
-                                                        const uint *__restrict__ rank_by_slot,
-                                                        const Counters *cnt, uint *__restrict__ child,
-                                                        uint cap) {
-  const uint k = blockIdx.x * ABLK + threadIdx.x;
-  if (k >= cap) return;
-  const uint n_pre = min(cnt->n_pre, cap);
-  uint c = SPH_DEAD;
-  if (k < n_pre) {
-    const uint w = S.slot[k];
-    if (flag_by_slot[w] && rank_by_slot[w] < cnt->s_done) c = n_pre + rank_by_slot[w];
-  }
-  child[k] = c;
-}
-
 // ---- density sample and loss (fp32, fixed-order reductions) ----
 __device__ inline void sample_point(const DevParams &P, int ns, uint v, float x[3]) {
   const uint vv[3] = {v % (uint)ns, v / (uint)ns % (uint)ns, v / ((uint)ns * (uint)ns)};
@@ -866,8 +849,7 @@ struct SphAdj {
   SortScratch sc{};
   BinScratch bins{};
   uint *s2p_hash = nullptr, *s2p_cell = nullptr, *cs_scr = nullptr, *ce_scr = nullptr;
-  uint *flag_by_slot = nullptr, *rank_by_slot = nullptr, *alive_by_slot = nullptr;
-  uint *newslot = nullptr, *status = nullptr;
+  SlotBits sb{};
   uint *scan_tmp = nullptr;
   Counters *cnt = nullptr;
   Counters *cnt_host = nullptr;
@@ -967,18 +949,23 @@ struct SphAdj {
   }
 
   // state S (counters in cnt) into cell order: T, lists cs, ce (sph_bins.hip)
-  void bin(DevState S, DevState T, uint *cs, uint *ce, int par, bool keep_err, bool set_m) {
+  // the step's split and merge records (child, partner) start empty
+  void bin(DevState S, DevState T, uint *cs, uint *ce, int par, bool keep_err, bool set_m,
+           uint *child = nullptr, uint *partner = nullptr) {
     launch_bin_count(SPH_V3D2, P, S, bins, cnt, cap, par, st);
     launch_bin_table(bins, cells, cs, ce, cnt, par, st, true, keep_err);
-    launch_bin_place(S, bins, cs, cnt, cap, st);
-    launch_bin_reorder(S, T, bins, cs, ce, sc.keys_alt, sc.vals_alt, s2p_cell, cnt, cap, st, true, set_m);
+    launch_bin_place(S, bins, cs, cnt, cap, st, 0, child ? sb.split : nullptr, partner ? sb.dead : nullptr, 1u,
+                     (uint)sph_bit_words(cap));
+    launch_bin_reorder(S, T, bins, cs, ce, sc.keys_alt, sc.vals_alt, s2p_cell, cnt, cap, st, true, set_m,
+                       nullptr, 0, child, partner);
   }
   // one forward step of state S (counters in cnt): cell order into the tape entry, next
   // state back into S; no host round trip
   void fwd_step(DevState S, const Tape &t, uint step) {
     const uint *nd = &cnt->n;
     if (bins.ccount) {
-      bin(S, t.T, t.cs, t.ce, (int)(step & 1u), false, true);  // and m = n, n_pre = n, ...
+      // and m = n, n_pre = n, ...
+      bin(S, t.T, t.cs, t.ce, (int)(step & 1u), false, true, t.child, t.partner);
     } else {
       launch_begin_step(cnt, st);  // n_pre = n, split and merge counters cleared
       launch_hash(SPH_V3D2, P, S, &cnt->m, cap, keys, s2p_hash, cnt, st);
@@ -986,6 +973,10 @@ struct SphAdj {
       sph_fill_cells(t.cs, t.ce, cells, st);
       launch_cell_bounds(skeys, cap, cells, t.cs, t.ce, st, nd);
       launch_reorder(S, t.T, svals, s2p_hash, cap, s2p_cell, st, cnt, true, nd);  // and m = n
+      sph_fill_u32(t.child, SPH_DEAD, cap, st);
+      sph_fill_u32(t.partner, SPH_DEAD, cap, st);
+      sph_fill_u32(sb.split, 0u, sph_bit_words(cap), st);
+      sph_fill_u32(sb.dead, 0u, sph_bit_words(cap), st);
     }
     launch_density(SPH_V3D2, P, t.T, aux, t.cs, t.ce, cap, st, nullptr, nd);
     launch_force(SPH_V3D2, P, t.T, aux, t.cs, t.ce, cap, st, nullptr, kForceListDefault, nd, true);
@@ -994,23 +985,13 @@ struct SphAdj {
     if (do_split || do_merge) {  // the energy decides split and merge (SPH-3D-2/sph_system.cpp:356)
       launch_make_erec(S, cap, aux.erec, st, nd);
       launch_energy(SPH_V3D2, P, S, t.cs, t.ce, cap, st, nullptr, kEnergyListDefault,
-                    do_split ? flag_by_slot : nullptr, aux.erec, nd, aux.fine_energy);
+                    do_split ? sb.split : nullptr, nullptr, aux.erec, nd, aux.fine_energy);
     }
-    if (do_split) {
-      sph_exclusive_scan(flag_by_slot, rank_by_slot, nd, cap, &cnt->scan_total, scan_tmp, st);
-      launch_split(SPH_V3D2, P, S, cap, flag_by_slot, rank_by_slot, cnt, status, st, nullptr,
-                   &cnt->n_pre);
-      k_adj_rec_split<<<agrid(cap), ABLK, 0, st>>>(S, flag_by_slot, rank_by_slot, cnt, t.child, cap);
-    } else {
-      sph_fill_u32(t.child, SPH_DEAD, cap, st);
-    }
-    sph_fill_u32(t.partner, SPH_DEAD, cap, st);
+    if (do_split) launch_split(SPH_V3D2, P, S, cap, sb, s2p_cell, cnt, st, false, nullptr, t.child);
     if (do_merge) {
-      launch_merge(SPH_V3D2, P, S, t.cs, t.ce, nullptr, status, cnt, st, nullptr, nullptr, 0,
+      launch_merge(SPH_V3D2, P, S, t.cs, t.ce, nullptr, sb.dead, cnt, st, nullptr, nullptr, 0,
                    nullptr, t.partner);
-      launch_alive_by_slot(S, status, cnt, cap, alive_by_slot, st);
-      sph_exclusive_scan(alive_by_slot, newslot, &cnt->n, cap, &cnt->scan_total, scan_tmp, st);
-      launch_renumber(S, status, newslot, cnt, cap, st);  // and n = survivors
+      launch_renumber(SPH_V3D2, S, cap, sb, s2p_cell, false, cnt, st);  // and n = survivors
     }
     (void)hipMemcpyAsync(t.slot_after, S.slot, 4 * (size_t)cap, hipMemcpyDeviceToDevice, st);
     k_adj_rec_counts<<<1, 1, 0, st>>>(cnt, t.tc);
@@ -1105,8 +1086,8 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
             a->alloc(a->sc.len_dev, 1) && a->alloc(a->scan_tmp, sph_scan_tmp_elems(scan_n)) &&
             a->alloc(a->s2p_hash, cap) && a->alloc(a->s2p_cell, cap) &&
             a->alloc(a->cs_scr, a->cells) && a->alloc(a->ce_scr, a->cells) &&
-            a->alloc(a->flag_by_slot, cap) && a->alloc(a->rank_by_slot, cap) &&
-            a->alloc(a->alive_by_slot, cap) && a->alloc(a->newslot, cap) && a->alloc(a->status, cap) &&
+            a->alloc(a->sb.split, sph_bit_words(cap)) && a->alloc(a->sb.dead, sph_bit_words(cap)) &&
+            a->alloc(a->sb.toff, sph_bit_tiles(cap)) &&
             a->alloc(a->cnt, 1) && a->alloc(a->aux.frec, 3 * cap) && a->alloc(a->aux.erec, cap) &&
             a->alloc(a->aux.nbl, (size_t)SPH_NBL_K * cap) && a->alloc(a->aux.nbl_cnt, cap) &&
             a->alloc(a->theta, nth) && a->alloc(a->dtheta, nth) && a->alloc(a->th_part, iblocks * nth) &&
@@ -1120,7 +1101,7 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
             a->alloc(a->aos_dev, cap * sizeof(SphParticle3D));
   a->aux.nbl_stride = (uint)cap;
   a->aux.choose_forms(SPH_V3D2, false, flags & SPH_STEP_SPLIT ? 2 * n : n);
-  a->sc.scan_tmp = a->scan_tmp;
+  a->sc.scan_tmp = a->sb.scan_tmp = a->scan_tmp;
   a->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && sph_use_bins(a->cells, cap)) {
     a->bins.hkey = a->keys;

@@ -210,8 +210,8 @@ struct SphBatch {
   uint *skeys = nullptr, *svals = nullptr;
   uint *s2p_hash = nullptr, *s2p_cell = nullptr;
   uint *cstart = nullptr, *cend = nullptr;
-  uint *flag_by_slot = nullptr, *rank_by_slot = nullptr, *alive_by_slot = nullptr;
-  uint *newslot = nullptr, *status = nullptr, *scan_tmp = nullptr;
+  SlotBits sb{};
+  uint *newslot = nullptr, *scan_tmp = nullptr;
   unsigned char *aos_dev = nullptr;
   int kbits = 1;
   uint M = 0;      // live particles of all scenes
@@ -351,8 +351,8 @@ struct SphBatch {
 
   // the removed entries of [0, m) are dropped: live entries move to the front, in order
   int pack() {
-    uint *flags = flag_by_slot, *pos = rank_by_slot;
-    launch_pack_live(cur, alt, m, flags, pos, scan_tmp, &cnt->scan_total, st);
+    // keys and vals are scratch between steps
+    launch_pack_live(cur, alt, m, keys, vals, scan_tmp, &cnt->scan_total, st);
     swap_state();
     m = M;
     return SPH_OK;
@@ -381,6 +381,10 @@ struct SphBatch {
     const int v = variant;
     const uint Mb = dev ? (uint)phys_cap : M;  // live entries: host count or bound
     const uint mb = dev ? (uint)phys_cap : m;  // entries, removed ones included
+    const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
+    const uint per_split = v == SPH_V3D4 ? 3u : 1u;
+    // entries that the split can leave
+    const uint Ma = (uint)std::min<uint64_t>((uint64_t)Mb * (1u + per_split), phys_cap);
     const uint *n_live = dev ? &cnt->n : nullptr;   // live entries at the start of the step
     const uint *n_pre = dev ? &cnt->n_pre : nullptr;  // the same, once split has moved n
     aux.choose_forms(v, true, M);  // M: the live count at the call's start, also for a graph
@@ -395,7 +399,8 @@ struct SphBatch {
       launch_bin_table(bins, total_cell, cstart, cend, cnt, 0, st, false);
       pend();
       pbegin(SPH_P_SORT);
-      launch_bin_place(cur, bins, cstart, cnt, mb, st, grid);
+      launch_bin_place(cur, bins, cstart, cnt, mb, st, grid, do_split ? sb.split : nullptr,
+                       do_merge ? sb.dead : nullptr, per_split, (uint)sph_bit_words(phys_cap));
       pend();
       pbegin(SPH_P_REORDER);
       // and m = n; acc, dp and energy are recomputed by the step's kernels below
@@ -415,6 +420,8 @@ struct SphBatch {
       pend();
       pbegin(SPH_P_REORDER);
       launch_reorder(cur, alt, svals, s2p_hash, Mb, s2p_cell, st, cnt, false, n_live, grid);
+      if (do_split) sph_fill_u32(sb.split, 0u, sph_bit_words(Mb), st);
+      if (do_merge) sph_fill_u32(sb.dead, 0u, sph_bit_words(Ma), st);
       pend();
     }
     swap_state();
@@ -431,37 +438,30 @@ struct SphBatch {
     pbegin(SPH_P_INTEGRATE);
     launch_integrate(v, P0, cur, Mb, st, &bv, aux.erec, n_live, grid);
     pend();
-    const bool do_split = (flags & SPH_STEP_SPLIT) != 0;
     pbegin(SPH_P_ENERGY);
-    uint *split_flags = do_split ? flag_by_slot : nullptr;  // the energy kernel decides splits
+    uint *split_bits = do_split ? sb.split : nullptr;  // the energy kernel decides splits
+    uint *qual = do_merge && !aux.fine_energy ? sb.qual : nullptr;
     DevParams Pe = P0;  // the energy kernel's unit-length path only if every scene takes it
     Pe.energy_unit = energy_unit_all() ? 1 : 0;
     auto energy = [&](int c) {
-      launch_energy(v, Pe, cur, cstart, cend, Mb, st, &bv, c, split_flags, aux.erec, n_live,
+      launch_energy(v, Pe, cur, cstart, cend, Mb, st, &bv, c, split_bits, qual, aux.erec, n_live,
                     aux.fine_energy);
     };
     if (dev) energy(le);
     else tune.run(1, st, energy);
     pend();
     pbegin(SPH_P_SPLIT);
-    if (do_split)
-      sph_exclusive_scan(flag_by_slot, rank_by_slot, n_live, Mb, &cnt->scan_total, scan_tmp, st);
-    launch_batch_split_plan(v, bv, rank_by_slot, Mb, do_split, cnt, st, n_pre);
-    if (do_split)
-      launch_split(v, P0, cur, Mb, flag_by_slot, rank_by_slot, cnt, status, st, &bv, n_pre, grid);
+    launch_batch_split_plan(v, bv, cnt, st);
+    if (do_split) launch_split(v, P0, cur, Mb, sb, s2p_cell, cnt, st, qual != nullptr, &bv);
     pend();
-    if (flags & SPH_STEP_MERGE) {
+    if (do_merge) {
       pbegin(SPH_P_MERGE);
-      // flag_by_slot (the split's flags, consumed by now) is the qualification bits' scratch
-      launch_merge(v, P0, cur, cstart, cend, nullptr, status, cnt, st, &bv, skeys, Mb, n_pre,
-                   nullptr, flag_by_slot, phys_cap);
+      launch_merge(v, P0, cur, cstart, cend, nullptr, sb.dead, cnt, st, &bv, skeys, Mb, n_pre,
+                   nullptr, qual, true);
       pend();
       pbegin(SPH_P_COMPACT);
-      const uint bound = (uint)phys_cap;  // entries after split: device count, host bound
-      launch_alive_by_slot(cur, status, cnt, bound, alive_by_slot, st, &bv, grid);
-      sph_exclusive_scan(alive_by_slot, newslot, &cnt->n, bound, &cnt->scan_total, scan_tmp, st);
-      launch_batch_compact_plan(bv, newslot, cnt, st);
-      launch_renumber(cur, status, newslot, cnt, bound, st, &bv, grid);
+      launch_batch_compact_plan(v, bv, cnt, st);
+      launch_renumber(v, cur, Ma, sb, s2p_cell, false, cnt, st, &bv);
       pend();
     }
   }
@@ -602,15 +602,15 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
             b->alloc(b->sc.tile_hist, sph_sort_hist_elems(cap)) &&
             b->alloc(b->s2p_hash, cap) && b->alloc(b->s2p_cell, cap) &&
             b->alloc(b->cstart, b->total_cell) && b->alloc(b->cend, b->total_cell) &&
-            b->alloc(b->flag_by_slot, cap) && b->alloc(b->rank_by_slot, cap) &&
-            b->alloc(b->alive_by_slot, cap) && b->alloc(b->newslot, cap) &&
-            b->alloc(b->status, cap) && b->alloc(b->cnt, 1) && b->alloc(b->scn, n_scenes) &&
+            b->alloc(b->sb.split, sph_bit_words(cap)) && b->alloc(b->sb.dead, sph_bit_words(cap)) &&
+            b->alloc(b->sb.qual, sph_bit_words(cap)) && b->alloc(b->sb.toff, sph_bit_tiles(cap)) &&
+            b->alloc(b->newslot, cap) && b->alloc(b->cnt, 1) && b->alloc(b->scn, n_scenes) &&
             b->alloc(b->Ptab, n_scenes) && b->alloc(b->aos_dev, (size_t)b->max_cap * b->rec) &&
             b->alloc(b->aux.frec, 3 * cap) && b->alloc(b->aux.erec, cap) &&
             b->alloc(b->aux.nbl, (size_t)SPH_NBL_K * cap) && b->alloc(b->aux.nbl_cnt, cap) &&
             b->alloc(b->scan_tmp, sph_scan_tmp_elems(scan_n)) && b->alloc(b->sc.len_dev, 1);
   b->aux.nbl_stride = (uint)cap;
-  b->sc.scan_tmp = b->scan_tmp;
+  b->sc.scan_tmp = b->sb.scan_tmp = b->scan_tmp;
   if (ok && sph_use_bins(b->total_cell, cap)) {
     b->bins.hkey = b->keys;
     b->bins.rank = b->vals;

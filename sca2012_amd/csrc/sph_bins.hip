@@ -188,13 +188,21 @@ __global__ __launch_bounds__(BLK) void k_bin_ranges(uint *__restrict__ ccount, u
   put_ranges(cstart, cend, c, ncell, carry + ex, v);
 }
 
+// zero0, zero1 (optional): the bit arrays that the step's split and merge set, cleared for the
+// particles (zero0) and for them and their children (zero1), at most zmax words.
 __global__ __launch_bounds__(BLK) void k_bin_place(const uint *__restrict__ slot,
                                                    const uint *__restrict__ hkey,
                                                    const uint *__restrict__ rank,
                                                    const uint *__restrict__ cstart,
                                                    const Counters *cnt, uint m_host,
-                                                   uint *__restrict__ bslot) {
-  for_each_item<false>(min(cnt->m_in, m_host), [&](const uint k) {
+                                                   uint *__restrict__ bslot, uint *__restrict__ zero0,
+                                                   uint *__restrict__ zero1, uint per_split, uint zmax) {
+  const uint m = min(cnt->m_in, m_host), z = (m + 31u) / 32u, z1 = min(z * (1u + per_split), zmax);
+  for (uint x = blockIdx.x * BLK + threadIdx.x; x < z1; x += gridDim.x * BLK) {
+    if (zero0 && x < z) zero0[x] = 0u;
+    if (zero1) zero1[x] = 0u;
+  }
+  for_each_item<false>(m, [&](const uint k) {
     const uint w = slot[k];
     if (w != SPH_DEAD) bslot[cstart[hkey[k]] + rank[k]] = w;
   });
@@ -289,9 +297,10 @@ void launch_bin_table(const BinScratch &bs, uint total_cell, uint *cstart, uint 
 }
 
 void launch_bin_place(DevState src, const BinScratch &bs, const uint *cstart, const Counters *cnt, uint m,
-                      hipStream_t st, uint grid) {
+                      hipStream_t st, uint grid, uint *zero0, uint *zero1, uint per_split, uint zmax) {
   if (m == 0) return;
-  k_bin_place<<<bgrid(grid, m), dim3(BLK), 0, st>>>(src.slot, bs.hkey, bs.rank, cstart, cnt, m, bs.bslot);
+  k_bin_place<<<bgrid(grid, m), dim3(BLK), 0, st>>>(src.slot, bs.hkey, bs.rank, cstart, cnt, m, bs.bslot,
+                                                    zero0, zero1, per_split, zmax);
 }
 
 void launch_bin_reorder(DevState src, DevState dst, const BinScratch &bs, const uint *cstart,

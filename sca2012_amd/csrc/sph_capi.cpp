@@ -4,7 +4,7 @@
 // Per-step device work (one HIP stream, no host round trip until the end of the step):
 //   hash -> radix sort -> cell ranges + reorder into cell order -> density -> force ->
 //   integrate -> [density grid -> normals -> marching cubes] -> energy ->
-//   [decide -> scan -> split] -> [merge -> renumber survivors]
+//   [split] -> [merge -> renumber survivors]
 // Counts that change inside the step (after split and merge) stay on the device; kernels
 // read them and are launched over host-side upper bounds.
 #include <hip/hip_runtime.h>
@@ -299,8 +299,8 @@ struct SphCtx {
   int par = 0;  // parity of the step (counting path)
   uint *s2p_hash = nullptr, *s2p_cell = nullptr;
   uint *cstart = nullptr, *cend = nullptr;
-  uint *flag_by_slot = nullptr, *rank_by_slot = nullptr, *alive_by_slot = nullptr;
-  uint *newslot = nullptr, *status = nullptr, *q2d = nullptr;
+  SlotBits sb{};
+  uint *newslot = nullptr, *q2d = nullptr;
   uint *scan_tmp = nullptr;
   Counters *cnt = nullptr;
   Counters *cnt_host = nullptr;
@@ -316,6 +316,7 @@ struct SphCtx {
   uint n = 0, m = 0, n_pre = 0;
   uint n_sorted = 0, n_flagged = 0, n_status = 0;
   bool hashed = false, sorted = false, lists_valid = false, merged = false, compacted = false;
+  bool qual_ready = false;  // the step's energy kernel wrote sb.qual
   bool erec_ok = false;  // aux.erec holds the current positions and velocities
   // aux.nbl holds the force pairs of the current state, cell lists and parameters (the
   // density kernel writes them; anything else that runs invalidates them)
@@ -473,12 +474,15 @@ struct SphCtx {
     cur = alt;
     alt = t;
   }
-  // hash, sort, cell ranges and reorder of a step: by counting where the grid suits it
-  void q_bin_step() {
+  // hash, sort, cell ranges and reorder of a step: by counting where the grid suits it. The bits
+  // that the step's split and merge set start clear.
+  void q_bin_step(bool do_split, bool do_merge) {
     if (!bins.ccount || !sph_use_bins(P.total_cell, n)) {
       q_hash();
       q_sort();
       q_cells(true);
+      if (do_split) sph_fill_u32(sb.split, 0u, sph_bit_words(n), st);
+      if (do_merge) sph_fill_u32(sb.dead, 0u, sph_bit_words(grown(n)), st);
       return;
     }
     nbl_ok = false;
@@ -496,12 +500,19 @@ struct SphCtx {
     launch_bin_table(bins, P.total_cell, cstart, cend, cnt, par, st);
     pend();
     pbegin(SPH_P_SORT);
-    launch_bin_place(cur, bins, cstart, cnt, m, st);
+    launch_bin_place(cur, bins, cstart, cnt, m, st, 0, do_split ? sb.split : nullptr,
+                     do_merge ? sb.dead : nullptr, variant == SPH_V3D4 ? 3u : 1u,
+                     (uint)sph_bit_words(cap));
     pend();
     pbegin(SPH_P_REORDER);
     launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, m, st, false);
     pend();
     std::swap(cur, alt);
+  }
+  // entries that a split of k particles can leave
+  uint grown(uint k) const {
+    const uint64_t most = (uint64_t)k * (variant == SPH_V3D4 ? 4u : 2u);
+    return most < cap ? (uint)most : std::max(cap, k);
   }
   void q_density() {
     pbegin(SPH_P_DENSITY);
@@ -529,49 +540,57 @@ struct SphCtx {
     pend();
     erec_ok = true;
   }
-  // with_flags: the energy kernel also makes the split decisions (q_split(true) follows)
-  void q_energy(bool tuned = false, bool with_flags = false) {
+  // do_split, do_merge (a step): the energy kernel also makes the split decisions (q_split(true)
+  // follows), and its one-thread form the merge qualification
+  void q_energy(bool tuned = false, bool do_split = false, bool do_merge = false) {
     pbegin(SPH_P_ENERGY);
-    uint *flags = with_flags ? flag_by_slot : nullptr;
     if (!erec_ok) {  // not straight after integrate: records from the current state
       launch_make_erec(cur, n, aux.erec, st);
       erec_ok = true;
     }
     aux.choose_forms(variant, false, n);
+    qual_ready = do_merge && !aux.fine_energy;
     auto go = [&](int c) {
-      launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, flags, aux.erec, nullptr,
-                    aux.fine_energy);
+      launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, do_split ? sb.split : nullptr,
+                    qual_ready ? sb.qual : nullptr, aux.erec, nullptr, aux.fine_energy);
     };
     if (tuned) tune.run(1, st, go);
     else go(tune.energy);
     pend();
   }
-  void q_split(bool flags_ready = false) {
+  // in_step: the decisions and the slot map are there
+  void q_split(bool in_step = false) {
     nbl_ok = false;
     erec_ok = false;
     pbegin(SPH_P_SPLIT);
-    if (!flags_ready) launch_decide(variant, P, cur, n, flag_by_slot, st);
-    sph_exclusive_scan(flag_by_slot, rank_by_slot, nullptr, n, &cnt->scan_total, scan_tmp, st);
-    launch_split(variant, P, cur, n, flag_by_slot, rank_by_slot, cnt, status, st);
+    const uint *s2p = s2p_cell;
+    if (!in_step) {
+      sph_fill_u32(sb.split, 0u, sph_bit_words(n), st);
+      launch_decide(variant, P, cur, n, sb.split, st);
+      launch_slot2phys(cur, m, newslot, st);
+      s2p = newslot;
+    }
+    launch_split(variant, P, cur, n, sb, s2p, cnt, st, in_step && qual_ready);
     n_flagged = n;
     pend();
   }
-  void q_merge() {
+  void q_merge(bool in_step = false) {
     nbl_ok = false;
     erec_ok = false;
     pbegin(SPH_P_MERGE);
     if (variant == SPH_V2D) launch_merge_q2d(P, cur, s2p_cell, cnt, cstart, cend, q2d, st);
-    // flag_by_slot (the split's flags, consumed by now) is the qualification bits' scratch
-    launch_merge(variant, P, cur, cstart, cend, q2d, status, cnt, st, nullptr, skeys, n_sorted,
-                 nullptr, nullptr, flag_by_slot, cap);
+    if (!in_step) sph_fill_u32(sb.dead, 0u, sph_bit_words(m), st);
+    // a step in several lanes per particle leaves the qualification to each cell's walk
+    launch_merge(variant, P, cur, cstart, cend, q2d, sb.dead, cnt, st, nullptr, skeys, n_sorted,
+                 nullptr, nullptr, in_step && !qual_ready ? nullptr : sb.qual, in_step);
     pend();
   }
-  void q_compact() {
+  void q_compact(bool in_step = false) {
     nbl_ok = false;
     pbegin(SPH_P_COMPACT);
-    launch_alive_by_slot(cur, status, cnt, cap, alive_by_slot, st);
-    sph_exclusive_scan(alive_by_slot, newslot, &cnt->n, cap, &cnt->scan_total, scan_tmp, st);
-    launch_renumber(cur, status, newslot, cnt, cap, st);  // and n = survivors
+    if (!in_step) launch_slot2phys(cur, m, newslot, st);
+    launch_renumber(variant, cur, in_step ? grown(n) : m, sb, in_step ? s2p_cell : newslot, !in_step, cnt,
+                    st);  // and n = survivors
     pend();
   }
   void q_dgrid() {
@@ -667,9 +686,9 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
             c->alloc(c->sc.tile_hist, sph_sort_hist_elems(cap)) &&
             c->alloc(c->s2p_hash, cap) && c->alloc(c->s2p_cell, cap) &&
             c->alloc(c->cstart, c->P.total_cell) && c->alloc(c->cend, c->P.total_cell) &&
-            c->alloc(c->flag_by_slot, cap) && c->alloc(c->rank_by_slot, cap) &&
-            c->alloc(c->alive_by_slot, cap) && c->alloc(c->newslot, cap) &&
-            c->alloc(c->status, cap) && c->alloc(c->q2d, std::max<size_t>(c->P.total_cell, 1)) &&
+            c->alloc(c->sb.split, sph_bit_words(cap)) && c->alloc(c->sb.dead, sph_bit_words(cap)) &&
+            c->alloc(c->sb.qual, sph_bit_words(cap)) && c->alloc(c->sb.toff, sph_bit_tiles(cap)) &&
+            c->alloc(c->newslot, cap) && c->alloc(c->q2d, std::max<size_t>(c->P.total_cell, 1)) &&
             c->alloc(c->cnt, 1) && c->alloc(c->aos_dev, cap * sizeof(SphParticle3D)) &&
             c->alloc(c->aux.frec, 3 * (size_t)cap) && c->alloc(c->aux.erec, cap) &&
             c->alloc(c->aux.nbl, (size_t)SPH_NBL_K * cap) && c->alloc(c->aux.nbl_cnt, cap);
@@ -685,7 +704,7 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
   }
   size_t scan_elems = sph_scan_tmp_elems(std::max(scan_n, c->ncube));
   ok = ok && c->alloc(c->scan_tmp, scan_elems);
-  c->sc.scan_tmp = c->scan_tmp;
+  c->sc.scan_tmp = c->sb.scan_tmp = c->scan_tmp;
   if (ok && sph_use_bins(c->P.total_cell, cap)) {
     c->bins.hkey = c->keys;
     c->bins.rank = c->vals;
@@ -897,7 +916,8 @@ int sph_marching_cubes(SphCtx *ctx, uint32_t *n_tri) {
 int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
   CHECK_CTX(ctx);
   if (ctx->n == 0) return SPH_EEMPTY;
-  ctx->q_bin_step();
+  const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
+  ctx->q_bin_step(do_split, do_merge);
   ctx->q_density();
   ctx->q_force(true);
   ctx->q_integrate();
@@ -906,11 +926,11 @@ int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
     ctx->q_normals();
     ctx->q_mc();
   }
-  ctx->q_energy(true, (flags & SPH_STEP_SPLIT) != 0);
-  if (flags & SPH_STEP_SPLIT) ctx->q_split(true);
-  if (flags & SPH_STEP_MERGE) {
-    ctx->q_merge();
-    ctx->q_compact();
+  ctx->q_energy(true, do_split, do_merge);
+  if (do_split) ctx->q_split(true);
+  if (do_merge) {
+    ctx->q_merge(true);
+    ctx->q_compact(true);
   }
   // the cell-range phase made physical == live before split appended children
   int rc = ctx->sync();
@@ -962,16 +982,20 @@ int sph_get_u32(SphCtx *ctx, int which, uint32_t *out, size_t n) {
     case SPH_Q_INDEX: src = ctx->svals; break;
     case SPH_Q_START: src = ctx->cstart; break;
     case SPH_Q_END: src = ctx->cend; break;
-    case SPH_Q_SPLITFLAG: src = ctx->flag_by_slot; break;
-    case SPH_Q_STATUS: src = ctx->alive_by_slot; break;
+    case SPH_Q_SPLITFLAG: src = ctx->sb.split; break;
+    case SPH_Q_STATUS: src = ctx->sb.dead; break;
     case SPH_Q_COUNTERS: src = (const uint *)ctx->cnt; break;
     default: return SPH_EINVAL;
   }
-  if (hipMemcpyAsync(out, src, n * 4, hipMemcpyDeviceToHost, ctx->st) != hipSuccess) return SPH_EHIP;
+  const bool bits = which == SPH_Q_SPLITFLAG || which == SPH_Q_STATUS;
+  std::vector<uint32_t> w(bits ? (n + 31) / 32 : 0);
+  if (hipMemcpyAsync(bits ? w.data() : out, src, (bits ? w.size() : n) * 4, hipMemcpyDeviceToHost,
+                     ctx->st) != hipSuccess)
+    return SPH_EHIP;
   int rc = ctx->sync();
   if (rc) return rc;
-  if (which == SPH_Q_SPLITFLAG || which == SPH_Q_STATUS)
-    for (size_t k = 0; k < n; k++) out[k] = out[k] ? 0u : 1u;
+  for (size_t k = 0; bits && k < n; k++)
+    out[k] = ((w[k >> 5] >> (k & 31)) & 1u) ^ (which == SPH_Q_SPLITFLAG ? 1u : 0u);
   return SPH_OK;
 }
 

@@ -150,6 +150,24 @@ __device__ inline void nb_range(const DevParams &P, int o, const uint c[3],
 // kernel (sph_internal.h: kForceLists, kEnergyLists).
 __device__ inline uint pack_entry(int o, uint j) { return ((uint)o << 27) | j; }
 
+// Split decision of the particle with slot word w: its bit by slot (a batch: by dense slot, and
+// the scene's count of flagged parents, one atomic per wave where the wave's are of one scene).
+template <bool B>
+__device__ inline void flag_split(bool split, uint w, uint *__restrict__ split_bits, SceneCnt *scn) {
+  if (!split) return;
+  uint d = w;
+  if constexpr (B) {
+    const uint sc = w >> SPH_SCENE_SHIFT;
+    d = scn[sc].first + (w & SPH_LOCAL_MASK);
+    const uint sc0 = (uint)__builtin_amdgcn_readfirstlane((int)sc);
+    const unsigned long long here = __ballot(true), same = __ballot(sc == sc0);
+    if (here != same) atomicAdd(&scn[sc].s_req, 1u);
+    else if ((threadIdx.x & 63u) == (uint)__builtin_ctzll(here))
+      atomicAdd(&scn[sc].s_req, (uint)__popcll(here));
+  }
+  atomicOr(&split_bits[d >> 5], 1u << (d & 31u));
+}
+
 __device__ inline uint wave_incl_scan(uint x, int lane) {
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {

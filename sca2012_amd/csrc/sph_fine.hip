@@ -521,10 +521,10 @@ constexpr int EC = 12;   // words per component: nine values, padded to 16 bytes
 
 template <int V, bool B>
 __global__ __launch_bounds__(BLK) void k_energy_fine(
-    DevParams P0, const DevParams *__restrict__ Ptab, const SceneCnt *__restrict__ scn,
+    DevParams P0, const DevParams *__restrict__ Ptab, SceneCnt *scn,
     const uint *__restrict__ slot, const float4 *__restrict__ pos, const float4 *__restrict__ acc,
     float *__restrict__ energy, const uint *__restrict__ cstart, const uint *__restrict__ cend,
-    const uint *n_dev, uint n_host, uint *__restrict__ flag_by_slot,
+    const uint *n_dev, uint n_host, uint *__restrict__ split_bits,
     const float4 *__restrict__ erec) {
   constexpr bool D3 = VT<V>::dim == 3;
   __shared__ __align__(16) uint pre[BLK / 64][FP + 1][28];
@@ -659,13 +659,9 @@ __global__ __launch_bounds__(BLK) void k_energy_fine(
   if (V == SPH_V3D4) E = 0.5f * (Li ? P.mass[1] : P.mass[0]) * (e2);
   else E = 0.5f * (e2);
   energy[i] = E;
-  if (flag_by_slot) {  // decide_adaptive_kernel, as k_decide
-    const uint w = slot[i];
-    const float sf = acc[i].w;
-    const bool split = E * P.co_energy + sf * P.co_surface > P.split_criteria &&
-                       __float_as_uint(pi.w) == 1u;
-    flag_by_slot[B ? scn[w >> SPH_SCENE_SHIFT].first + (w & SPH_LOCAL_MASK) : w] = split ? 1u : 0u;
-  }
+  if (split_bits)  // decide_adaptive_kernel, as k_decide
+    flag_split<B>(E * P.co_energy + acc[i].w * P.co_surface > P.split_criteria && Li == 0, slot[i],
+                  split_bits, scn);
 }
 
 inline dim3 blocks_of(size_t n, int per) { return dim3((uint)((n + per - 1) / per)); }
@@ -702,8 +698,8 @@ void launch_force_fine(int variant, const DevParams &P, DevState s, Aux a, const
 
 void launch_energy_fine(int variant, const DevParams &P, DevState s, const uint *cstart,
                         const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                        uint *flag_by_slot, const float4 *erec, const uint *n_dev) {
+                        uint *split_bits, const float4 *erec, const uint *n_dev) {
   SPH_FINE(k_energy_fine, variant, bv != nullptr, blocks_of(n, FB), st, P, bv ? bv->Ptab : nullptr,
-           bv ? bv->scn : nullptr, s.slot, s.pos, s.acc, s.energy, cstart, cend, n_dev, n, flag_by_slot,
+           bv ? bv->scn : nullptr, s.slot, s.pos, s.acc, s.energy, cstart, cend, n_dev, n, split_bits,
            erec);
 }

@@ -130,7 +130,7 @@ struct Counters {
   uint groups;    // merge groups
   uint err;       // bit 0: particle outside the grid
   uint ntri;      // triangles emitted by marching cubes
-  uint scan_total;
+  uint scan_total;  // of launch_pack_live
   uint nmc;  // non-empty marching cubes
   uint m_in;     // entries at the start of the step (m as the step found it)
   uint err2[2];  // domain errors of the step being binned, by step parity (sph_bins.hip)
@@ -148,12 +148,12 @@ struct SceneCnt {
   uint n;          // live particles (updated by split and compaction)
   uint n_pre;      // live particles at the start of the step
   uint first;      // dense start of the scene's slots in the sort input (pre-split)
-  uint r0;         // split-flag scan at `first`
+  uint r0;         // split parents flagged of the scenes before this one
   uint s_req;      // split parents flagged
   uint s_done;     // split parents split (capacity policy)
   uint done_base;  // split parents of the scenes before this one
   uint first2;     // dense start of the scene's slots after split
-  uint a0;         // survivor scan at `first2`
+  uint a0;         // entries removed from the scenes before this one
   uint groups;     // merge groups
   uint err;        // bit 0: particle outside the scene's grid
   uint pad[5];
@@ -354,6 +354,16 @@ struct BinScratch {
   uint *bslot;   // slots by cell, in arrival order
   uint *tmp;     // tile sums, sph_bin_tiles(total_cell)
 };
+// Bits by slot (a batch: by dense slot) and by entry, for split and merge; sph_bit_words words each
+struct SlotBits {
+  uint *split;     // slot -> split decided
+  uint *dead;      // slot -> removed by a merge
+  uint *qual;      // entry in cell order -> qualifies for merging
+  uint *toff;      // sph_bit_tiles: scan of the tiles' counts (sph_slots.hip)
+  uint *scan_tmp;  // for that scan
+};
+size_t sph_bit_words(size_t n);
+size_t sph_bit_tiles(size_t n);
 // Counting or radix sort for n particles on total_cell cells. The scan reads and writes 20
 // bytes per cell (4M cells: 18 us, about what the sort's extra launches take). Hash, sort, table
 // and reorder against counting: 14k particles on 13,824 cells 33 -> 19 us, 498k on 262,144 cells
@@ -368,8 +378,11 @@ void launch_bin_count(int variant, const DevParams &P, DevState src, const BinSc
                       uint grid = 0);
 void launch_bin_table(const BinScratch &bs, uint total_cell, uint *cstart, uint *cend, Counters *cnt,
                       int par, hipStream_t st, bool single = true, bool keep_err = false);
+// zero0, zero1 (optional): bit arrays to clear, for the m entries and for (1 + per_split) m, at most
+// zmax words
 void launch_bin_place(DevState src, const BinScratch &bs, const uint *cstart, const Counters *cnt, uint m,
-                      hipStream_t st, uint grid = 0);
+                      hipStream_t st, uint grid = 0, uint *zero0 = nullptr, uint *zero1 = nullptr,
+                      uint per_split = 0, uint zmax = 0);
 // skeys, svals: the sorted keys and slots; s2p: slot -> place; set_m: also cnt->m = cnt->n;
 // init0, init1 (optional): SPH_DEAD for every particle
 void launch_bin_reorder(DevState src, DevState dst, const BinScratch &bs, const uint *cstart,
@@ -428,13 +441,14 @@ void launch_force(int variant, const DevParams &P, DevState s, Aux a, const uint
 void launch_integrate(int variant, const DevParams &P, DevState s, uint n, hipStream_t st,
                       const BatchView *bv = nullptr, float4 *erec = nullptr,
                       const uint *n_dev = nullptr, uint grid = 0);
-// flag_by_slot (optional): also the split decision of each particle (as launch_decide);
-// erec: the energy records of the current positions and velocities (written by the
+// split_bits (optional): also the split decision of each particle (as launch_decide), as bits
+// that were clear before; qbits (optional, not with `fine`): also the merge qualification of the
+// entries as it stands before the split; erec: the energy records of the current positions and velocities (written by the
 // integrate kernel, or by launch_make_erec), read for the neighbours' pair terms
 void launch_energy(int variant, const DevParams &P, DevState s, const uint *cstart,
                    const uint *cend, uint n, hipStream_t st, const BatchView *bv, int cfg,
-                   uint *flag_by_slot, const float4 *erec, const uint *n_dev = nullptr,
-                   bool fine = false);
+                   uint *split_bits, uint *qbits, const float4 *erec,
+                   const uint *n_dev = nullptr, bool fine = false);
 // the same phases in several lanes per particle (launch_density, launch_force and launch_energy
 // call these as Aux::choose_forms says)
 void launch_density_fine(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
@@ -445,44 +459,41 @@ void launch_force_fine(int variant, const DevParams &P, DevState s, Aux a, const
                        const uint *n_dev, bool use_nbl);
 void launch_energy_fine(int variant, const DevParams &P, DevState s, const uint *cstart,
                         const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                        uint *flag_by_slot, const float4 *erec, const uint *n_dev);
+                        uint *split_bits, const float4 *erec, const uint *n_dev);
 void launch_make_erec(DevState s, uint n, float4 *erec, hipStream_t st,
                       const uint *n_dev = nullptr);
-void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *flag_by_slot,
-                   hipStream_t st, const BatchView *bv = nullptr);
-// A single scene's split also applies the capacity policy to the counters (n, m, n_pre,
-// s_req, s_done); a batch's counters come from launch_batch_split_plan.
-void launch_split(int variant, const DevParams &P, DevState s, uint n, const uint *flag_by_slot,
-                  const uint *rank_by_slot, Counters *cnt, uint *status, hipStream_t st,
-                  const BatchView *bv = nullptr, const uint *n_dev = nullptr, uint grid = 0);
+void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *split_bits, hipStream_t st);
+// Split of the flagged ones of the cnt->n_pre (at most n) particles (sph_slots.hip). s2p: slot ->
+// entry. A single scene's split also applies the capacity policy to the counters (n, m, s_req,
+// s_done); a batch's counters come from launch_batch_split_plan. with_qual: the entries'
+// qualification bits are completed; child (optional): entry of a parent -> its first child.
+void launch_split(int variant, const DevParams &P, DevState s, uint n, const SlotBits &sb, const uint *s2p,
+                  Counters *cnt, hipStream_t st, bool with_qual, const BatchView *bv = nullptr,
+                  uint *child = nullptr);
 // 2D merge qualification word per cell (bit 0; the entry + 1 of the cell id's particle in
 // bits 1..31 when it is listed in that cell)
 void launch_merge_q2d(const DevParams &P, DevState s, const uint *slot2phys, const Counters *cnt,
                       const uint *cstart, const uint *cend, uint *q2d, hipStream_t st);
 // skeys/nkeys (optional): the step's sorted cell keys; on a grid with more cells than keys
 // the merge then runs one thread per key instead of one per cell (same result).
-// qbits (optional, qbits_len words of scratch, at least two per 64 keys): the entries'
-// qualification is evaluated first, one thread per entry (k_merge_qual), instead of inside
-// each cell's walk (same result)
+// dead: bits by slot (clear before) that receive the removed entries. qbits (optional): the
+// entries' qualification bits, ready (from the energy kernel and the split) or evaluated first,
+// one thread per entry, instead of inside each cell's walk (same result)
 void launch_merge(int variant, const DevParams &P, DevState s, const uint *cstart,
-                  const uint *cend, const uint *q2d, uint *status, Counters *cnt, hipStream_t st,
+                  const uint *cend, const uint *q2d, uint *dead, Counters *cnt, hipStream_t st,
                   const BatchView *bv = nullptr, const uint *skeys = nullptr, uint nkeys = 0,
                   const uint *nkeys_dev = nullptr, uint *group_out = nullptr,
-                  uint *qbits = nullptr, size_t qbits_len = 0);
-void launch_alive_by_slot(DevState s, const uint *status, const Counters *cnt, uint m_max,
-                          uint *alive_by_slot, hipStream_t st, const BatchView *bv = nullptr,
-                          uint grid = 0);
-// A single scene's renumbering also sets the live count to the survivors (cnt->scan_total).
-void launch_renumber(DevState s, const uint *status, const uint *newslot, Counters *cnt,
-                     uint m_max, hipStream_t st, const BatchView *bv = nullptr, uint grid = 0);
+                  uint *qbits = nullptr, bool qbits_ready = false);
+// Slots of the survivors among the cnt->m (at most m) entries; removed entries become SPH_DEAD.
+// A single scene's renumbering also sets the live count. all_slots: s2p maps every slot, else
+// those of the n_pre particles before the split.
+void launch_renumber(int variant, DevState s, uint m, const SlotBits &sb, const uint *s2p, bool all_slots,
+                     Counters *cnt, hipStream_t st, const BatchView *bv = nullptr);
 void launch_begin_step(Counters *cnt, hipStream_t st);
 // batch bookkeeping (one block each): dense slot starts, split plan, survivor counts
 void launch_batch_begin(const BatchView &bv, Counters *cnt, hipStream_t st);
-void launch_batch_split_plan(int variant, const BatchView &bv, const uint *rank_by_slot, uint m,
-                             bool do_split, Counters *cnt, hipStream_t st,
-                             const uint *m_dev = nullptr);
-void launch_batch_compact_plan(const BatchView &bv, const uint *newslot, Counters *cnt,
-                               hipStream_t st);
+void launch_batch_split_plan(int variant, const BatchView &bv, Counters *cnt, hipStream_t st);
+void launch_batch_compact_plan(int variant, const BatchView &bv, Counters *cnt, hipStream_t st);
 // entries of one scene: mark removed / slot -> physical index map
 void launch_scene_kill(DevState s, uint m, uint scene, hipStream_t st);
 void launch_scene_slot2phys(DevState s, uint m, uint scene, uint *slot2phys, hipStream_t st);

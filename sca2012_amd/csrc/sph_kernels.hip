@@ -612,11 +612,12 @@ __global__ __launch_bounds__(BLK) void k_integrate(DevParams P0, const DevParams
 // the cell changes. When the kernel length is exactly 1, x/h and x/sqrt(h) equal x, so
 // those divisions are skipped.
 // ---------------------------------------------------------------------------------------
-// flag_by_slot (optional): the step's split decision (k_decide) is made here too, from
-// the energy just computed, the surface value of the force phase and the level.
+// split_bits (optional): the step's split decision (k_decide) is made here too, from the
+// energy just computed, the surface value of the force phase and the level. qbits
+// (optional): and the merge qualification of the entries (k_merge_qual).
 template <int V, bool B, int LIST_E, bool U>
 __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *__restrict__ Ptab,
-                                                const SceneCnt *__restrict__ scn,
+                                                SceneCnt *scn,
                                                 const uint *__restrict__ slot,
                                                 const float4 *__restrict__ pos,
                                                 const float4 *__restrict__ vel,
@@ -625,7 +626,8 @@ __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *_
                                                 const uint *__restrict__ cstart,
                                                 const uint *__restrict__ cend,
                                                 const uint *n_dev, uint n_host,
-                                                uint *__restrict__ flag_by_slot,
+                                                uint *__restrict__ split_bits,
+                                                uint *__restrict__ qbits,
                                                 const float4 *__restrict__ erec) {
   constexpr bool D3 = VT<V>::dim == 3;
   __shared__ uint list[LIST_E * BLK];  // each thread uses its own column only
@@ -754,12 +756,18 @@ __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *_
   if (V == SPH_V3D4) E = 0.5f * (Li ? P.mass[1] : P.mass[0]) * (e2);
   else E = 0.5f * (e2);
   energy[i] = E;
-  if (flag_by_slot) {  // decide_adaptive_kernel, as k_decide
-    const uint w = slot[i];
-    const float sf = acc[i].w;
-    const bool split = E * P.co_energy + sf * P.co_surface > P.split_criteria &&
-                       __float_as_uint(pi.w) == 1u;
-    flag_by_slot[B ? scn[w >> SPH_SCENE_SHIFT].first + (w & SPH_LOCAL_MASK) : w] = split ? 1u : 0u;
+  const float sf = split_bits || qbits ? acc[i].w : 0.0f;
+  const bool low = E * P.co_energy + sf * P.co_surface < P.merge_criteria;
+  if (split_bits)  // decide_adaptive_kernel, as k_decide
+    flag_split<B>(E * P.co_energy + sf * P.co_surface > P.split_criteria && lvl_index(pi.w) == 0,
+                  slot[i], split_bits, scn);
+  if (qbits) {  // merge qualification as it stands before the split (k_split completes it)
+    const uint lev = __float_as_uint(pi.w);
+    const unsigned long long b = __ballot(D3 ? lev != 1u && low : lev == 2u);
+    if ((t & 63u) == 0u) {  // lane 0 has an item whenever a lane of the wave has one
+      qbits[i >> 5] = (uint)b;
+      qbits[(i >> 5) + 1u] = (uint)(b >> 32);
+    }
   }
 }
 
@@ -768,10 +776,11 @@ __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *_
 // 2D :1067-1090): flag 1 = split (the reference stores 0 for split and sorts ascending).
 // Flags go to slot positions so the scan ranks parents in slot order.
 // ---------------------------------------------------------------------------------------
+// Flags are bits by slot (a batch: by dense slot), so ranks follow slot order.
 template <bool B>
 __global__ __launch_bounds__(BLK) void k_decide(DevParams P0, const DevParams *__restrict__ Ptab,
-                                                const SceneCnt *__restrict__ scn, DevState S,
-                                                uint n, uint *__restrict__ flag_by_slot) {
+                                                SceneCnt *scn, DevState S, uint n,
+                                                uint *__restrict__ split_bits) {
   const uint k = blockIdx.x * BLK + threadIdx.x;
   if (k >= n) return;
   const uint w = S.slot[k];
@@ -779,108 +788,7 @@ __global__ __launch_bounds__(BLK) void k_decide(DevParams P0, const DevParams *_
   const float E = S.energy[k];
   const float sf = S.acc[k].w;
   const uint lev = __float_as_uint(S.pos[k].w);
-  const bool split = E * P.co_energy + sf * P.co_surface > P.split_criteria && lev == 1u;
-  flag_by_slot[B ? scn[w >> SPH_SCENE_SHIFT].first + (w & SPH_LOCAL_MASK) : w] = split ? 1u : 0u;
-}
-
-// A12 adaptive_particle_kernel (3D-2 :1576-1615; 3D-4 :1583-1656) / split_particle_kernel
-// (2D :1092-1131). Parent of rank r (slot order) writes its children at N + r(n-1) + c.
-// Capacity policy on the counters after a single scene's split: only the first
-// floor((cap - n) / (NS - 1)) flagged parents split.
-template <int V> __device__ inline void finish_split_counts(const DevParams &P, Counters *cnt) {
-  constexpr int NS = VT<V>::nsplit;
-  const uint n = cnt->n;
-  const uint total = cnt->scan_total;
-  const uint room = (P.cap - n) / (uint)(NS - 1);
-  const uint done = total < room ? total : room;
-  cnt->n_pre = n;
-  cnt->s_req = total;
-  cnt->s_done = done;
-  cnt->n = n + done * (uint)(NS - 1);
-  cnt->m = cnt->n;
-}
-
-// A single scene's split: thread 0 also updates the counters (no thread of this kernel
-// reads n, m, n_pre, s_req or s_done).
-template <int V, bool B>
-__global__ __launch_bounds__(BLK) void k_split(DevParams P0, const DevParams *__restrict__ Ptab,
-                                               const SceneCnt *__restrict__ scn, DevState S,
-                                               const uint *n_dev, uint n_host,
-                                               const uint *__restrict__ flag_by_slot,
-                                               const uint *__restrict__ rank_by_slot,
-                                               Counters *cnt, uint *__restrict__ status) {
-  constexpr int NS = VT<V>::nsplit;
-  if (!B && blockIdx.x == 0 && threadIdx.x == 0) finish_split_counts<V>(P0, cnt);
-  const uint n = dev_count(n_dev, n_host);  // live entries before the split
-  for_each_item<false>(n, [&](const uint k) {
-  const uint w = S.slot[k];
-  const DevParams &P = scene_params<B>(P0, Ptab, w);
-  // base: physical index of the first child; sbase: its slot word
-  uint base, sbase;
-  if (!B) {
-    if (!flag_by_slot[w]) return;
-    const uint rank = rank_by_slot[w];
-    const uint total = cnt->scan_total;
-    const uint room = (P.cap - n) / (uint)(NS - 1);
-    const uint done = total < room ? total : room;
-    if (rank >= done) return;
-    base = n + rank * (uint)(NS - 1);
-    sbase = base;
-  } else {
-    // children of a batch go after all live entries, scene by scene in parent rank order;
-    // their slots continue the scene's own numbering
-    const uint sc = w >> SPH_SCENE_SHIFT;
-    const SceneCnt &C = scn[sc];
-    const uint d = C.first + (w & SPH_LOCAL_MASK);
-    if (!flag_by_slot[d]) return;
-    const uint rank = rank_by_slot[d] - C.r0;
-    if (rank >= C.s_done) return;
-    base = n + (C.done_base + rank) * (uint)(NS - 1);
-    sbase = (sc << SPH_SCENE_SHIFT) | (C.n_pre + rank * (uint)(NS - 1));
-  }
-  const float hs = P.kernel[1] / 2;
-  float4 p = S.pos[k];
-  const float4 v = S.vel[k], e = S.ev[k], a = S.acc[k];
-  const float2 dpk = S.dp[k];
-  const float en = S.energy[k];
-  const float lev2 = __uint_as_float(2u);
-  // children copy every field of the parent (3D leaves dens/press/surface/tension
-  // unwritten in the reference; copies make the downloaded state defined)
-  if (NS == 2) {
-    S.pos[base] = make_float4(p.x - hs, p.y, p.z, lev2);
-    S.vel[base] = v;
-    S.ev[base] = e;
-    S.acc[base] = a;
-    S.dp[base] = dpk;
-    S.energy[base] = en;
-    S.slot[base] = sbase;
-    status[base] = 0u;
-    S.pos[k] = make_float4(p.x + hs, p.y, p.z, lev2);
-  } else {
-    const float e4 = en / 4;
-    const float4 cp[3] = {make_float4(p.x - hs, p.y, p.z, lev2), make_float4(p.x, p.y, p.z - hs, lev2),
-                          make_float4(p.x, p.y, p.z + hs, lev2)};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      const uint q = base + c;
-      S.pos[q] = cp[c];
-      S.vel[q] = v;
-      S.ev[q] = e;
-      S.acc[q] = a;
-      S.dp[q] = dpk;
-      S.energy[q] = e4;
-      S.slot[q] = sbase + c;
-      status[q] = 0u;
-    }
-    S.pos[k] = make_float4(p.x + hs, p.y, p.z, lev2);
-    S.energy[k] = e4;
-  }
-  status[k] = 0u;
-  });
-}
-
-template <int V> __global__ void k_finish_split(DevParams P, Counters *cnt) {
-  finish_split_counts<V>(P, cnt);
+  flag_split<B>(E * P.co_energy + sf * P.co_surface > P.split_criteria && lev == 1u, w, split_bits, scn);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -900,7 +808,7 @@ template <int V, bool B>
 __device__ inline uint merge_cell(const DevParams &P0, const DevParams *__restrict__ Ptab,
                                   SceneCnt *scn, uint cl, DevState &S,
                                   const uint *__restrict__ cstart, const uint *__restrict__ cend,
-                                  const uint *__restrict__ q2d, uint *__restrict__ status,
+                                  const uint *__restrict__ q2d, uint *__restrict__ dead,
                                   uint *__restrict__ group_out, const uint *__restrict__ qbits) {
   constexpr int NM = VT<V>::nsplit;
   constexpr bool D3 = VT<V>::dim == 3;
@@ -930,8 +838,8 @@ __device__ inline uint merge_cell(const DevParams &P0, const DevParams *__restri
   uint q = 0;
   unsigned long long qb = 0ull;
   if (qbits) {
-    // the entries' bits from k_merge_qual (which also cleared their status): the count over
-    // [s, e) and the first 64 bits relative to s
+    // the entries' bits from the energy kernel and the split, or from k_merge_qual: the count
+    // over [s, e) and the first 64 bits relative to s
     for (uint wi = s >> 5; wi <= (e - 1u) >> 5; wi++) {
       const uint b0 = wi << 5;
       const uint lo = s > b0 ? s - b0 : 0u, hi = e - b0 < 32u ? e - b0 : 32u;
@@ -957,7 +865,6 @@ __device__ inline uint merge_cell(const DevParams &P0, const DevParams *__restri
     for (int t = 0; t < 8; t++) {
       const uint j = j0 + t;
       if (j < e) {
-        status[j] = 0u;
         if (qq[t]) {
           q++;
           if (j - s < 64u) qb |= 1ull << (j - s);
@@ -1031,9 +938,12 @@ __device__ inline uint merge_cell(const DevParams &P0, const DevParams *__restri
       S.energy[p1] = e1;
       if (p1 == kown) cell_q = e1 * P.co_energy + A1.w * P.co_surface < P.merge_criteria;
     }
-    status[p1] = 0u;
 #pragma unroll
-    for (int t = 1; t < NM; t++) status[pm[t]] = 1u;
+    for (int t = 1; t < NM; t++) {  // removed, as a bit by slot (a batch: by dense slot)
+      const uint w = S.slot[pm[t]];
+      const uint d = B ? scn[w >> SPH_SCENE_SHIFT].first2 + (w & SPH_LOCAL_MASK) : w;
+      atomicOr(&dead[d >> 5], 1u << (d & 31u));
+    }
     if (NM == 2 && group_out) group_out[p1] = pm[1];
   }
   if (B) atomicAdd(&scn[w0 >> SPH_SCENE_SHIFT].groups, ng);
@@ -1044,12 +954,12 @@ __device__ inline uint merge_cell(const DevParams &P0, const DevParams *__restri
 // merge_cell's walk would evaluate it before any merge of the step (merges write only
 // entries of their own cell): bit j of qbits -- 3D: level 2 and
 // energy * co_energy + surface * co_surface < merge_criteria; 2D: level 2 (the cell's own
-// qualification is applied in the walk) -- and status[j] = 0.
+// qualification is applied in the walk). A step's energy kernel and split write the same bits;
+// this pass serves a merge that is called by itself.
 template <int V, bool B>
 __global__ __launch_bounds__(BLK) void k_merge_qual(DevParams P0, const DevParams *__restrict__ Ptab,
                                                     DevState S, const uint *n_dev, uint n_host,
-                                                    uint *__restrict__ qbits,
-                                                    uint *__restrict__ status) {
+                                                    uint *__restrict__ qbits) {
   const uint j = blockIdx.x * BLK + threadIdx.x;
   const uint n = dev_count(n_dev, n_host);
   bool q = false;
@@ -1061,7 +971,6 @@ __global__ __launch_bounds__(BLK) void k_merge_qual(DevParams P0, const DevParam
           (S.energy[j] * P.co_energy + S.acc[j].w * P.co_surface < P.merge_criteria);
     else
       q = lev == 2u;
-    status[j] = 0u;
   }
   const unsigned long long b = __ballot(q);
   const uint j0 = j & ~63u;  // the wave's first entry: its 64 bits are words j0/32, +1
@@ -1080,7 +989,7 @@ __global__ __launch_bounds__(BLK) void k_merge(DevParams P0, const DevParams *__
                                                const uint *__restrict__ cstart,
                                                const uint *__restrict__ cend,
                                                const uint *__restrict__ q2d,
-                                               uint *__restrict__ status, Counters *cnt,
+                                               uint *__restrict__ dead, Counters *cnt,
                                                const uint *__restrict__ skeys,
                                                const uint *nkeys_dev, uint nkeys_host,
                                                uint *__restrict__ group_out,
@@ -1091,10 +1000,10 @@ __global__ __launch_bounds__(BLK) void k_merge(DevParams P0, const DevParams *__
     if (t < dev_count(nkeys_dev, nkeys_host)) {
       const uint h = skeys[t];
       if ((t == 0 || skeys[t - 1] != h) && h < ncell)
-        ng = merge_cell<V, B>(P0, Ptab, scn, h, S, cstart, cend, q2d, status, group_out, qbits);
+        ng = merge_cell<V, B>(P0, Ptab, scn, h, S, cstart, cend, q2d, dead, group_out, qbits);
     }
   } else if (t < ncell) {
-    ng = merge_cell<V, B>(P0, Ptab, scn, t, S, cstart, cend, q2d, status, group_out, qbits);
+    ng = merge_cell<V, B>(P0, Ptab, scn, t, S, cstart, cend, q2d, dead, group_out, qbits);
   }
   ng = wave_sum(ng);  // every lane of the wave reaches this point
   if ((threadIdx.x & 63u) == 0 && ng) atomicAdd(&cnt->groups, ng);
@@ -1124,42 +1033,6 @@ __global__ __launch_bounds__(BLK) void k_merge_q2d(DevParams P, DevState S,
   q2d[cl] = w;
 }
 
-// A14 rearrange (SPH-3D-2/sph_system.cu:1818-1840) as a renumbering: survivors get the
-// rank of their slot among survivors; removed entries are dropped by the next sort.
-template <bool B>
-__global__ __launch_bounds__(BLK) void k_alive_by_slot(DevState S, const uint *__restrict__ status,
-                                                       const SceneCnt *__restrict__ scn,
-                                                       const Counters *cnt,
-                                                       uint *__restrict__ alive_by_slot) {
-  for_each_item<false>(cnt->n, [&](const uint k) {
-    const uint w = S.slot[k];
-    const uint d = B ? scn[w >> SPH_SCENE_SHIFT].first2 + (w & SPH_LOCAL_MASK) : w;
-    alive_by_slot[d] = status[k] == 0u ? 1u : 0u;
-  });
-}
-
-// Bound = cnt->m, the physical count (a single scene compacts right after merge, where
-// m == n; a batch's compaction plan has already set cnt->n). A single scene's thread 0
-// also sets the live count to the survivors; no thread here reads cnt->n.
-template <bool B>
-__global__ __launch_bounds__(BLK) void k_renumber(DevState S, const uint *__restrict__ status,
-                                                  const uint *__restrict__ newslot,
-                                                  const SceneCnt *__restrict__ scn,
-                                                  Counters *cnt) {
-  if (!B && blockIdx.x == 0 && threadIdx.x == 0) cnt->n = cnt->scan_total;
-  for_each_item<false>(cnt->m, [&](const uint k) {
-    const uint w = S.slot[k];
-    if (!B) {
-      S.slot[k] = status[k] == 0u ? newslot[w] : SPH_DEAD;
-    } else {
-      const uint sc = w >> SPH_SCENE_SHIFT;
-      const SceneCnt &C = scn[sc];
-      const uint d = C.first2 + (w & SPH_LOCAL_MASK);
-      S.slot[k] = status[k] == 0u ? (sc << SPH_SCENE_SHIFT) | (newslot[d] - C.a0) : SPH_DEAD;
-    }
-  });
-}
-
 __global__ void k_begin_step(Counters *cnt) {
   cnt->n_pre = cnt->n;
   cnt->s_req = 0u;
@@ -1169,11 +1042,6 @@ __global__ void k_begin_step(Counters *cnt) {
 }
 
 __global__ void k_set_phys_count(Counters *cnt) { cnt->m = cnt->n; }
-
-__global__ void k_finish_compact(Counters *cnt) {
-  cnt->m = cnt->n;
-  cnt->n = cnt->scan_total;
-}
 
 // ---------------------------------------------------------------------------------------
 // A15 integrate_dens_kernel + integrate_cell_dens (SPH-3D-2/sph_system.cu:1842-2183):
@@ -1637,39 +1505,29 @@ __global__ __launch_bounds__(SCN_BLK) void k_batch_begin(SceneCnt *scn, uint ns,
   }
 }
 
-// After the split-flag scan: per scene, parents flagged, parents split under the scene's
-// capacity (the first floor((cap - n)/(n_split - 1)) in slot order), where its children
-// go, and its dense slot start after split. Without split only the starts are set.
+// After the split decisions (s_req: parents flagged per scene): parents split under the scene's
+// capacity (the first floor((cap - n)/(n_split - 1)) in slot order), where its children go, and
+// its dense slot start after split.
 template <int NS>
 __global__ __launch_bounds__(SCN_BLK) void k_batch_split_plan(const DevParams *__restrict__ Ptab,
-                                                              SceneCnt *scn, uint ns,
-                                                              const uint *__restrict__ rank,
-                                                              const uint *m_dev, uint m_host,
-                                                              int do_split, Counters *cnt) {
+                                                              SceneCnt *scn, uint ns, Counters *cnt) {
   __shared__ uint sh[SCN_BLK];
   const uint t = threadIdx.x;
-  const uint m = dev_count(m_dev, m_host);
-  uint n = 0u, req = 0u, done = 0u, r0 = 0u;
+  uint n = 0u, req = 0u, done = 0u;
   if (t < ns) {
     n = scn[t].n_pre;
-    if (do_split) {
-      const uint total = cnt->scan_total;
-      const uint f = scn[t].first, e = f + n;
-      r0 = f < m ? rank[f] : total;
-      req = (e < m ? rank[e] : total) - r0;
-      const uint room = (Ptab[t].cap - n) / (uint)(NS - 1);
-      done = req < room ? req : room;
-    }
+    req = scn[t].s_req;
+    const uint room = (Ptab[t].cap - n) / (uint)(NS - 1);
+    done = req < room ? req : room;
   }
   uint tot_done, tot_n2, tot_req;
   const uint done_base = block_exscan(done, sh, tot_done);
   const uint n2 = n + done * (uint)(NS - 1);
   const uint first2 = block_exscan(n2, sh, tot_n2);
-  (void)block_exscan(req, sh, tot_req);
+  const uint r0 = block_exscan(req, sh, tot_req);
   if (t < ns) {
     SceneCnt &C = scn[t];
     C.r0 = r0;
-    C.s_req = req;
     C.s_done = done;
     C.done_base = done_base;
     C.n = n2;
@@ -1683,24 +1541,21 @@ __global__ __launch_bounds__(SCN_BLK) void k_batch_split_plan(const DevParams *_
   }
 }
 
-// After the survivor scan: each scene's survivors and the scan value its renumbering
-// subtracts. cnt->m (entries, removed ones included) stays for the renumber bound.
-__global__ __launch_bounds__(SCN_BLK) void k_batch_compact_plan(SceneCnt *scn, uint ns,
-                                                                const uint *__restrict__ newslot,
-                                                                Counters *cnt) {
+// After the merge: each scene's survivors and the removed entries before it, which its
+// renumbering leaves out of the count. cnt->m (entries, removed ones included) stays for the
+// renumber bound.
+template <int NS>
+__global__ __launch_bounds__(SCN_BLK) void k_batch_compact_plan(SceneCnt *scn, uint ns, Counters *cnt) {
+  __shared__ uint sh[SCN_BLK];
   const uint t = threadIdx.x;
-  const uint D = cnt->m;
-  const uint total = cnt->scan_total;
+  const uint gone = t < ns ? scn[t].groups * (uint)(NS - 1) : 0u;
+  uint tot;
+  const uint a0 = block_exscan(gone, sh, tot);
   if (t < ns) {
-    SceneCnt &C = scn[t];
-    const uint f = C.first2, e = f + C.n;
-    const uint a0 = f < D ? newslot[f] : total;
-    const uint a1 = e < D ? newslot[e] : total;
-    C.a0 = a0;
-    C.n = a1 - a0;
+    scn[t].a0 = a0;
+    scn[t].n -= gone;
   }
-  __syncthreads();
-  if (t == 0) cnt->n = total;
+  if (t == 0) cnt->n -= tot;
 }
 
 __global__ __launch_bounds__(BLK) void k_scene_kill(uint *__restrict__ slot, uint m, uint scene) {
@@ -1851,11 +1706,11 @@ void launch_integrate(int variant, const DevParams &P, DevState s, uint n, hipSt
 template <int L, bool U>
 static void launch_energy_lu(int variant, const DevParams &P, DevState s, const uint *cstart,
                              const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                             uint *flag_by_slot, const float4 *erec, const uint *n_dev) {
+                             uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev) {
 #define SPH_EN(VV, BB)                                                                       \
   k_energy<VV, BB, L, U><<<grid_for(n), dim3(BLK), 0, st>>>(                                 \
       P, ptab_of(bv), scn_of(bv), s.slot, s.pos, s.vel, s.acc, s.energy, cstart, cend, n_dev, \
-      n, flag_by_slot, erec)
+      n, split_bits, qbits, erec)
   if (bv) {
     if (variant == SPH_V3D2) SPH_EN(SPH_V3D2, true);
     else if (variant == SPH_V3D4) SPH_EN(SPH_V3D4, true);
@@ -1870,11 +1725,11 @@ static void launch_energy_lu(int variant, const DevParams &P, DevState s, const 
 template <int L>
 static void launch_energy_l(int variant, const DevParams &P, DevState s, const uint *cstart,
                             const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                            uint *flag_by_slot, const float4 *erec, const uint *n_dev) {
+                            uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev) {
   if (P.energy_unit)
-    launch_energy_lu<L, true>(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    launch_energy_lu<L, true>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
   else
-    launch_energy_lu<L, false>(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    launch_energy_lu<L, false>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
 }
 
 // erec (pos.x, pos.y, vel.x, vel.y) from the state, for an energy pass that does not follow
@@ -1896,38 +1751,23 @@ void launch_make_erec(DevState s, uint n, float4 *erec, hipStream_t st, const ui
 
 void launch_energy(int variant, const DevParams &P, DevState s, const uint *cstart,
                    const uint *cend, uint n, hipStream_t st, const BatchView *bv, int cfg,
-                   uint *flag_by_slot, const float4 *erec, const uint *n_dev, bool fine) {
+                   uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev, bool fine) {
   if (n == 0) return;
   if (fine)
-    return launch_energy_fine(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    return launch_energy_fine(variant, P, s, cstart, cend, n, st, bv, split_bits, erec, n_dev);
   static_assert(kEnergyLists[0] == 16 && kEnergyLists[1] == 24 && kEnergyLists[2] == 32, "energy lists");
   if (cfg == 1)
-    launch_energy_l<24>(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    launch_energy_l<24>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
   else if (cfg == 2)
-    launch_energy_l<32>(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    launch_energy_l<32>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
   else
-    launch_energy_l<16>(variant, P, s, cstart, cend, n, st, bv, flag_by_slot, erec, n_dev);
+    launch_energy_l<16>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
 }
 
-void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *flag_by_slot,
-                   hipStream_t st, const BatchView *bv) {
+void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *split_bits, hipStream_t st) {
   (void)variant;
   if (n == 0) return;
-  if (bv)
-    k_decide<true><<<grid_for(n), dim3(BLK), 0, st>>>(P, bv->Ptab, bv->scn, s, n, flag_by_slot);
-  else
-    k_decide<false><<<grid_for(n), dim3(BLK), 0, st>>>(P, nullptr, nullptr, s, n, flag_by_slot);
-}
-
-void launch_split(int variant, const DevParams &P, DevState s, uint n, const uint *flag_by_slot,
-                  const uint *rank_by_slot, Counters *cnt, uint *status, hipStream_t st,
-                  const BatchView *bv, const uint *n_dev, uint grid) {
-  if (n == 0) {  // nothing to split; a single scene still applies the counter update
-    if (!bv) SPH_DISPATCH(variant, k_finish_split, dim3(1), dim3(1), 0, st, P, cnt);
-    return;
-  }
-  SPH_DISPATCH_VB(variant, bv != nullptr, k_split, grid_or(grid, n), dim3(BLK), 0, st, P,
-                  ptab_of(bv), scn_of(bv), s, n_dev, n, flag_by_slot, rank_by_slot, cnt, status);
+  k_decide<false><<<grid_for(n), dim3(BLK), 0, st>>>(P, nullptr, nullptr, s, n, split_bits);
 }
 
 void launch_merge_q2d(const DevParams &P, DevState s, const uint *slot2phys, const Counters *cnt,
@@ -1937,45 +1777,19 @@ void launch_merge_q2d(const DevParams &P, DevState s, const uint *slot2phys, con
 }
 
 void launch_merge(int variant, const DevParams &P, DevState s, const uint *cstart,
-                  const uint *cend, const uint *q2d, uint *status, Counters *cnt, hipStream_t st,
+                  const uint *cend, const uint *q2d, uint *dead, Counters *cnt, hipStream_t st,
                   const BatchView *bv, const uint *skeys, uint nkeys, const uint *nkeys_dev,
-                  uint *group_out, uint *qbits, size_t qbits_len) {
+                  uint *group_out, uint *qbits, bool qbits_ready) {
   const uint ncell = bv ? bv->total_cell : P.total_cell;
   // a sparse grid (the 512^3-cell collision: 4M keys, 134M cells) runs by key; on a
   // denser one the per-cell threads keep more lanes of a wave busy
   const bool by_entry = skeys && (size_t)nkeys * 4 < ncell;
-  // the qualification pass needs the entry count (the sorted keys) and two words per 64
-  // entries of scratch
-  if (!(qbits && nkeys && ((size_t)nkeys + 63) / 64 * 2 <= qbits_len)) qbits = nullptr;
-  if (qbits)
+  if (qbits && !qbits_ready)
     SPH_DISPATCH_VB(variant, bv != nullptr, k_merge_qual, grid_for(nkeys), dim3(BLK), 0, st, P,
-                    ptab_of(bv), s, nkeys_dev, nkeys, qbits, status);
+                    ptab_of(bv), s, nkeys_dev, nkeys, qbits);
   SPH_DISPATCH_VB(variant, bv != nullptr, k_merge, grid_for(by_entry ? nkeys : ncell),
                   dim3(BLK), 0, st, P, ptab_of(bv), scn_of(bv), ncell, s, cstart, cend, q2d,
-                  status, cnt, by_entry ? skeys : nullptr, nkeys_dev, nkeys, group_out, qbits);
-}
-
-void launch_alive_by_slot(DevState s, const uint *status, const Counters *cnt, uint m_max,
-                          uint *alive_by_slot, hipStream_t st, const BatchView *bv, uint grid) {
-  if (m_max == 0) return;
-  if (bv)
-    k_alive_by_slot<true><<<grid_or(grid, m_max), dim3(BLK), 0, st>>>(s, status, bv->scn, cnt,
-                                                                      alive_by_slot);
-  else
-    k_alive_by_slot<false><<<grid_or(grid, m_max), dim3(BLK), 0, st>>>(s, status, nullptr, cnt,
-                                                                       alive_by_slot);
-}
-
-void launch_renumber(DevState s, const uint *status, const uint *newslot, Counters *cnt,
-                     uint m_max, hipStream_t st, const BatchView *bv, uint grid) {
-  if (m_max == 0) {
-    if (!bv) hipLaunchKernelGGL(k_finish_compact, dim3(1), dim3(1), 0, st, cnt);
-    return;
-  }
-  if (bv)
-    k_renumber<true><<<grid_or(grid, m_max), dim3(BLK), 0, st>>>(s, status, newslot, bv->scn, cnt);
-  else
-    k_renumber<false><<<grid_or(grid, m_max), dim3(BLK), 0, st>>>(s, status, newslot, nullptr, cnt);
+                  dead, cnt, by_entry ? skeys : nullptr, nkeys_dev, nkeys, group_out, qbits);
 }
 
 void launch_begin_step(Counters *cnt, hipStream_t st) {
@@ -1986,19 +1800,14 @@ void launch_batch_begin(const BatchView &bv, Counters *cnt, hipStream_t st) {
   k_batch_begin<<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, cnt);
 }
 
-void launch_batch_split_plan(int variant, const BatchView &bv, const uint *rank_by_slot, uint m,
-                             bool do_split, Counters *cnt, hipStream_t st, const uint *m_dev) {
-  if (variant == SPH_V3D4)
-    k_batch_split_plan<4><<<1, SCN_BLK, 0, st>>>(bv.Ptab, bv.scn, bv.n_scenes, rank_by_slot, m_dev,
-                                                 m, do_split ? 1 : 0, cnt);
-  else
-    k_batch_split_plan<2><<<1, SCN_BLK, 0, st>>>(bv.Ptab, bv.scn, bv.n_scenes, rank_by_slot, m_dev,
-                                                 m, do_split ? 1 : 0, cnt);
+void launch_batch_split_plan(int variant, const BatchView &bv, Counters *cnt, hipStream_t st) {
+  if (variant == SPH_V3D4) k_batch_split_plan<4><<<1, SCN_BLK, 0, st>>>(bv.Ptab, bv.scn, bv.n_scenes, cnt);
+  else k_batch_split_plan<2><<<1, SCN_BLK, 0, st>>>(bv.Ptab, bv.scn, bv.n_scenes, cnt);
 }
 
-void launch_batch_compact_plan(const BatchView &bv, const uint *newslot, Counters *cnt,
-                               hipStream_t st) {
-  k_batch_compact_plan<<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, newslot, cnt);
+void launch_batch_compact_plan(int variant, const BatchView &bv, Counters *cnt, hipStream_t st) {
+  if (variant == SPH_V3D4) k_batch_compact_plan<4><<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, cnt);
+  else k_batch_compact_plan<2><<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, cnt);
 }
 
 void launch_scene_kill(DevState s, uint m, uint scene, hipStream_t st) {
