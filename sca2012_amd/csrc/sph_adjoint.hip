@@ -1140,7 +1140,7 @@ int sph_adj_upload(SphAdj *a, const void *aos, uint32_t n) {
   if (hipMemcpyAsync(a->aos_dev, aos, (size_t)n * sizeof(SphParticle3D), hipMemcpyHostToDevice,
                      a->st) != hipSuccess)
     return SPH_EHIP;
-  launch_upload_scatter(SPH_V3D2, a->aos_dev, n, a->state0, a->st);
+  launch_upload(SPH_V3D2, a->aos_dev, n, a->state0, 0, a->st, nullptr, n, n);
   a->have_state = true;
   a->forward_done = false;
   return a->sync();
@@ -1270,8 +1270,7 @@ int sph_adj_download(SphAdj *a, void *aos, uint32_t n) {
   CHECK_ADJ(a);
   if (!aos || !a->forward_done || n != a->n_live) return SPH_EINVAL;
   // the forward's final state: cur, m_final entries (merged-away ones marked), by slot
-  launch_slot2phys(a->cur, a->m_final, a->s2p_cell, a->st);
-  launch_download_gather(SPH_V3D2, a->cur, a->s2p_cell, n, a->aos_dev, a->st);
+  launch_download(SPH_V3D2, a->cur, Span{0u, a->m_final, 0u, 0u}, n, a->aos_dev, a->st);
   if (hipMemcpyAsync(aos, a->aos_dev, (size_t)n * sizeof(SphParticle3D), hipMemcpyDeviceToHost, a->st) != hipSuccess)
     return SPH_EHIP;
   return a->sync();

@@ -217,6 +217,7 @@ struct SphBatch {
   uint M = 0;      // live particles of all scenes
   uint m = 0;      // entries, removed ones included
   std::vector<uint> n_host;  // live particles per scene
+  std::vector<Span> at;      // entries of cur that hold the scene's particles (and maybe others)
   bool pushes = false;       // some scene has a one-step push pending
   hipError_t last_err = hipSuccess;
   // profiling (hipEvents around each phase on the batch's stream)
@@ -305,8 +306,8 @@ struct SphBatch {
     pending.clear();
   }
 
-  // host mirrors -> device counters (after uploads)
-  int push_counts() {
+  // the host's copy of the counters after an upload
+  void host_counts() {
     Counters c;
     std::memset(&c, 0, sizeof(c));
     c.n = M;
@@ -318,9 +319,25 @@ struct SphBatch {
       scn_host[s].n = n_host[s];
       scn_host[s].n_pre = n_host[s];
     }
+  }
+  // ... and on the device
+  int push_counts() {
+    host_counts();
     if (hipMemcpyAsync(cnt, cnt_host, sizeof(Counters), hipMemcpyHostToDevice, st) != hipSuccess ||
         hipMemcpyAsync(scn, scn_host, sizeof(SceneCnt) * ns, hipMemcpyHostToDevice, st) != hipSuccess)
       return SPH_EHIP;
+    return SPH_OK;
+  }
+
+  // wait for the stream's work; the counters stay as the host knows them
+  int drain() {
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) {
+      last_err = e;
+      return SPH_EHIP;
+    }
+    collect();
     return SPH_OK;
   }
 
@@ -341,6 +358,18 @@ struct SphBatch {
     for (uint s = 0; s < ns; s++) n_host[s] = scn_host[s].n;
     return SPH_OK;
   }
+  // where a step left the scenes: their particles before the split in cell order, scene after
+  // scene, then the children, scene after scene
+  void spans_after_step() {
+    const uint per = variant == SPH_V3D4 ? 3u : 1u;
+    for (uint s = 0; s < ns; s++) {
+      const SceneCnt &c = scn_host[s];
+      at[s].a = c.first;
+      at[s].na = c.n_pre;
+      at[s].b = cnt_host->n_pre + c.done_base * per;
+      at[s].nb = c.s_done * per;
+    }
+  }
 
   int upload_params() {
     return hipMemcpyAsync(Ptab, P.data(), sizeof(DevParams) * ns, hipMemcpyHostToDevice, st) ==
@@ -355,6 +384,7 @@ struct SphBatch {
     launch_pack_live(cur, alt, m, keys, vals, scan_tmp, &cnt->scan_total, st);
     swap_state();
     m = M;
+    for (Span &x : at) x = Span{0u, m, 0u, 0u};
     return SPH_OK;
   }
   void swap_state() {
@@ -523,6 +553,7 @@ struct SphBatch {
     }
     const int rc = sync();
     ltune.collect();
+    if (rc == SPH_OK) spans_after_step();
     return rc;
   }
 
@@ -562,6 +593,7 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
   b->raw.assign((const unsigned char *)sysparams,
                 (const unsigned char *)sysparams + b->raw_size * n_scenes);
   b->n_host.assign(n_scenes, 0u);
+  b->at.assign(n_scenes, Span{});
   size_t cells = 0, total = 0;
   for (uint s = 0; s < n_scenes; s++) {
     const uint c = capacity[s];
@@ -677,26 +709,25 @@ int sph_batch_upload(SphBatch *b, uint32_t scene, const void *aos, uint32_t n) {
   CHECK_BATCH(b);
   if (scene >= b->ns || (n > 0 && !aos)) return SPH_EINVAL;
   if (n > b->cap[scene]) return SPH_ECAP;
-  if (b->n_host[scene] > 0) launch_scene_kill(b->cur, b->m, scene, b->st);
+  const BatchView bv = b->view();
+  const uint bits = scene << SPH_SCENE_SHIFT;
+  Span old = b->n_host[scene] > 0 ? b->at[scene] : Span{};
   b->M -= b->n_host[scene];
   b->n_host[scene] = 0;
   if ((size_t)b->m + n > b->phys_cap) {  // drop removed entries to make room
-    if (b->push_counts() != SPH_OK) return SPH_EHIP;
+    launch_upload(b->variant, b->aos_dev, 0, b->cur, 0, b->st, b->cnt, b->M, b->m, bits, old, &bv);
+    old = Span{};
     b->pack();
   }
-  if (n > 0) {
-    if (hipMemcpyAsync(b->aos_dev, aos, b->rec * n, hipMemcpyHostToDevice, b->st) != hipSuccess)
-      return SPH_EHIP;
-    DevState at = b->cur;
-    at.pos += b->m; at.vel += b->m; at.ev += b->m; at.acc += b->m;
-    at.dp += b->m; at.energy += b->m; at.slot += b->m;
-    launch_upload_scatter(b->variant, b->aos_dev, n, at, b->st, scene << SPH_SCENE_SHIFT);
-  }
+  if (n > 0 && hipMemcpyAsync(b->aos_dev, aos, b->rec * n, hipMemcpyHostToDevice, b->st) != hipSuccess)
+    return SPH_EHIP;
+  launch_upload(b->variant, b->aos_dev, n, b->cur, b->m, b->st, b->cnt, b->M + n, b->m + n, bits, old, &bv);
+  b->at[scene] = Span{b->m, n, 0u, 0u};
   b->n_host[scene] = n;
   b->M += n;
   b->m += n;
-  if (b->push_counts() != SPH_OK) return SPH_EHIP;
-  return b->sync();
+  b->host_counts();
+  return b->drain();
 }
 
 int sph_batch_download(SphBatch *b, uint32_t scene, void *aos, uint32_t n) {
@@ -704,11 +735,10 @@ int sph_batch_download(SphBatch *b, uint32_t scene, void *aos, uint32_t n) {
   if (scene >= b->ns || n > b->n_host[scene]) return SPH_EINVAL;
   if (n == 0) return SPH_OK;
   if (!aos) return SPH_EINVAL;
-  launch_scene_slot2phys(b->cur, b->m, scene, b->newslot, b->st);
-  launch_download_gather(b->variant, b->cur, b->newslot, n, b->aos_dev, b->st);
+  launch_download(b->variant, b->cur, b->at[scene], n, b->aos_dev, b->st, scene << SPH_SCENE_SHIFT);
   if (hipMemcpyAsync(aos, b->aos_dev, b->rec * n, hipMemcpyDeviceToHost, b->st) != hipSuccess)
     return SPH_EHIP;
-  return b->sync();
+  return b->drain();
 }
 
 int sph_batch_num_particles(SphBatch *b, uint32_t *n_per_scene) {
@@ -749,6 +779,7 @@ int sph_batch_step(SphBatch *b, uint32_t flags, uint32_t steps, uint32_t *n_tota
     rc = b->sync();
     b->clear_pushes();
     if (rc) return rc;
+    b->spans_after_step();
     b->tune.end_step();
     if (b->cnt_host->err) rc = SPH_EDOMAIN;
   }

@@ -269,6 +269,14 @@ int key_bits(uint total_cell) {
 
 }  // namespace
 
+namespace {
+// Polls of a report before the host waits for the stream instead (about 0.3 ms)
+constexpr uint kReportPolls = 10000;
+// Steps with the same launches before they are captured, and captured steps that are kept
+constexpr uint kGraphAfter = 3;
+constexpr size_t kGraphsMax = 16;
+}  // namespace
+
 namespace sphhost {
 bool valid_variant(int v) { return ::valid_variant(v); }
 DevParams make_dev_params(int variant, const void *raw, uint cap) {
@@ -303,7 +311,10 @@ struct SphCtx {
   uint *newslot = nullptr, *q2d = nullptr;
   uint *scan_tmp = nullptr;
   Counters *cnt = nullptr;
-  Counters *cnt_host = nullptr;
+  uint *rep_seq = nullptr;       // reports made, on the device
+  Report *rep = nullptr;         // the last report (pinned host memory) and its device address
+  Report *rep_dev = nullptr;
+  uint rep_want = 0;             // reports launched
   float *dgrid = nullptr, *normal3 = nullptr, *tris = nullptr;
   uint *cube_count = nullptr, *cube_off = nullptr;  // per z-segment: triangles, their offsets
   uint *seg_cube = nullptr, *seg_coff = nullptr;    // per z-segment: non-empty cubes, offsets
@@ -341,6 +352,26 @@ struct SphCtx {
 
   ListTuner tune;  // pair-list lengths of the force and energy kernels
 
+  // Captured steps (graph_step): everything a step's launches depend on but the device's state
+  struct StepKey {
+    uint bound, flags, forms, lists, buffers;
+    bool operator==(const StepKey &o) const {
+      return bound == o.bound && flags == o.flags && forms == o.forms && lists == o.lists &&
+             buffers == o.buffers;
+    }
+  };
+  struct StepGraph {
+    StepKey key;
+    uint uses;
+    uint64_t last;
+    hipGraphExec_t exec;  // null until the step has run kGraphAfter times
+  };
+  std::vector<StepGraph> graphs;
+  uint64_t graph_clock = 0;
+  bool graphs_work = true;    // false once a capture has failed
+  bool flipped = false;       // cur is the second state buffer
+  const uint *nd = nullptr;   // during a capture: the live count on the device, n and m bound it
+
   ~SphCtx() {
     if (st) (void)hipStreamSynchronize(st);
     tune.destroy();
@@ -350,7 +381,9 @@ struct SphCtx {
     }
     for (auto e : ev_pool) (void)hipEventDestroy(e);
     for (void *p : allocs) (void)hipFree(p);
-    if (cnt_host) (void)hipHostFree(cnt_host);
+    for (auto &g : graphs)
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    if (rep) (void)hipHostFree(rep);
     if (st) (void)hipStreamDestroy(st);
   }
 
@@ -404,29 +437,47 @@ struct SphCtx {
     pending.clear();
   }
 
-  // Synchronise, read the counters, collect timings. Returns an SPH status.
-  int sync() {
+  int fail(hipError_t e) {
+    last_err = e;
+    return SPH_EHIP;
+  }
+  // Wait for the stream's work; the counters stay as the host knows them.
+  int drain() {
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(cnt_host, cnt, sizeof(Counters), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-      last_err = e;
-      return SPH_EHIP;
-    }
+    if (e != hipSuccess) return fail(e);
     collect();
-    n = cnt_host->n;
-    m = cnt_host->m;
     return SPH_OK;
   }
-
-  void set_counts_on_device(uint nn, uint mm) {
-    Counters c;
-    std::memset(&c, 0, sizeof(c));
-    c.n = nn;
-    c.m = mm;
-    c.n_pre = nn;
-    *cnt_host = c;
-    (void)hipMemcpyAsync(cnt, cnt_host, sizeof(Counters), hipMemcpyHostToDevice, st);
+  // Read the counters once the stream's work is done, collect timings. Returns an SPH status.
+  // reported: the work ended with a report kernel. The host polls the report's number for a
+  // while, about what a small scene's step takes, and then waits for the stream; a stream that
+  // fails, or ends without the report, ends the wait there.
+  int sync(bool reported = false) {
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(e);
+    if (!reported) launch_report(cnt, rep_seq, rep_dev, st);
+    rep_want++;
+    const bool events = !pending.empty() || tune.pending;  // read below or by the caller
+    auto there = [&] { return __atomic_load_n(&rep->seq, __ATOMIC_ACQUIRE) == rep_want; };
+    bool done = false;
+    for (uint k = 0; !events && !done && k < kReportPolls; k++) {
+      done = there();
+      __builtin_ia32_pause();
+    }
+    if (!done) {
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) return fail(e);
+      if (!there()) {  // a launch that failed
+        rep_want = rep->seq;
+        return fail(hipErrorUnknown);
+      }
+    }
+    collect();
+    n = rep->c.n;
+    m = rep->c.m;
+    return SPH_OK;
   }
 
   // ---- enqueue-only phase bodies ----
@@ -470,14 +521,14 @@ struct SphCtx {
     launch_reorder(cur, alt, svals, s2p_hash, n, s2p_cell, st, cnt, !in_step);  // and m = n
     pend();
     erec_ok = false;
-    DevState t = cur;
-    cur = alt;
-    alt = t;
+    std::swap(cur, alt);
+    flipped = !flipped;
   }
   // hash, sort, cell ranges and reorder of a step: by counting where the grid suits it. The bits
   // that the step's split and merge set start clear.
+  bool by_counting() const { return bins.ccount && sph_use_bins(P.total_cell, n); }
   void q_bin_step(bool do_split, bool do_merge) {
-    if (!bins.ccount || !sph_use_bins(P.total_cell, n)) {
+    if (!nd && !by_counting()) {
       q_hash();
       q_sort();
       q_cells(true);
@@ -508,6 +559,7 @@ struct SphCtx {
     launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, m, st, false);
     pend();
     std::swap(cur, alt);
+    flipped = !flipped;
   }
   // entries that a split of k particles can leave
   uint grown(uint k) const {
@@ -516,8 +568,8 @@ struct SphCtx {
   }
   void q_density() {
     pbegin(SPH_P_DENSITY);
-    aux.choose_forms(variant, false, n);
-    launch_density(variant, P, cur, aux, cstart, cend, n, st);
+    if (!nd) aux.choose_forms(variant, false, n);
+    launch_density(variant, P, cur, aux, cstart, cend, n, st, nullptr, nd);
     pend();
     nbl_ok = true;
   }
@@ -525,9 +577,9 @@ struct SphCtx {
   void q_force(bool tuned = false) {
     pbegin(SPH_P_FORCE);
     const bool use = nbl_ok;
-    aux.choose_forms(variant, false, n);
+    if (!nd) aux.choose_forms(variant, false, n);
     auto go = [&](int c) {
-      launch_force(variant, P, cur, aux, cstart, cend, n, st, nullptr, c, nullptr, use);
+      launch_force(variant, P, cur, aux, cstart, cend, n, st, nullptr, c, nd, use);
     };
     if (tuned) tune.run(0, st, go);
     else go(tune.force);
@@ -536,7 +588,7 @@ struct SphCtx {
   void q_integrate() {
     nbl_ok = false;
     pbegin(SPH_P_INTEGRATE);
-    launch_integrate(variant, P, cur, n, st, nullptr, aux.erec);
+    launch_integrate(variant, P, cur, n, st, nullptr, aux.erec, nd);
     pend();
     erec_ok = true;
   }
@@ -548,11 +600,11 @@ struct SphCtx {
       launch_make_erec(cur, n, aux.erec, st);
       erec_ok = true;
     }
-    aux.choose_forms(variant, false, n);
+    if (!nd) aux.choose_forms(variant, false, n);
     qual_ready = do_merge && !aux.fine_energy;
     auto go = [&](int c) {
       launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, do_split ? sb.split : nullptr,
-                    qual_ready ? sb.qual : nullptr, aux.erec, nullptr, aux.fine_energy);
+                    qual_ready ? sb.qual : nullptr, aux.erec, nd, aux.fine_energy);
     };
     if (tuned) tune.run(1, st, go);
     else go(tune.energy);
@@ -582,7 +634,7 @@ struct SphCtx {
     if (!in_step) sph_fill_u32(sb.dead, 0u, sph_bit_words(m), st);
     // a step in several lanes per particle leaves the qualification to each cell's walk
     launch_merge(variant, P, cur, cstart, cend, q2d, sb.dead, cnt, st, nullptr, skeys, n_sorted,
-                 nullptr, nullptr, in_step && !qual_ready ? nullptr : sb.qual, in_step);
+                 nd, nullptr, in_step && !qual_ready ? nullptr : sb.qual, in_step);
     pend();
   }
   void q_compact(bool in_step = false) {
@@ -611,6 +663,117 @@ struct SphCtx {
     launch_mc_list(P, dgrid, seg_cube, cube_off, seg_coff, max_tri, clist, st);
     launch_mc_emit(P, dgrid, normal3, clist, cnt, max_tri, tris, st);
     pend();
+  }
+
+  void q_step(uint flags) {
+    const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
+    q_bin_step(do_split, do_merge);
+    q_density();
+    q_force(true);
+    q_integrate();
+    if ((flags & SPH_STEP_MC) && P.dim == 3 && dgrid) {
+      q_dgrid();
+      q_normals();
+      q_mc();
+    }
+    q_energy(true, do_split, do_merge);
+    if (do_split) q_split(true);
+    if (do_merge) {
+      q_merge(true);
+      q_compact(true);
+    }
+  }
+
+  void drop_graphs() {
+    if (graphs.empty()) return;
+    (void)hipStreamSynchronize(st);
+    for (auto &g : graphs)
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    graphs.clear();
+  }
+  // The step as one captured graph, its report included, when it has run kGraphAfter times with
+  // the same launches (a capture takes longer than a step; a scene that is stepped a few times
+  // never pays for one). The launches are sized by a power of two above the particle and entry
+  // counts and read the counts on the device. Steps of sparse grids (whose host state decides how
+  // the cell tables are cleared), timed steps and steps with one-step forces are launched one by
+  // one. Returns false if the step is still to be launched.
+  bool graph_step(uint flags) {
+    if (!graphs_work || prof_mask || tune.tuning() || !by_counting() || P.push_left || P.push_right || P.mouse)
+      return false;
+    uint bound = 1024;
+    while (bound < std::max(n, m) && bound < cap) bound *= 2;
+    bound = std::min(bound, cap);
+    aux.choose_forms(variant, false, n);
+    const StepKey key{bound, flags & 7u, aux.forms(), (uint)tune.force | (uint)tune.energy << 8,
+                      (flipped ? 1u : 0u) | (par ? 2u : 0u)};
+    auto g = std::find_if(graphs.begin(), graphs.end(), [&](const StepGraph &x) { return x.key == key; });
+    if (g == graphs.end()) {
+      if (graphs.size() >= kGraphsMax) {  // the one unused for longest goes
+        g = std::min_element(graphs.begin(), graphs.end(),
+                             [](const StepGraph &a, const StepGraph &b) { return a.last < b.last; });
+        if (g->exec) {
+          (void)hipStreamSynchronize(st);
+          (void)hipGraphExecDestroy(g->exec);
+        }
+        graphs.erase(g);
+      }
+      graphs.push_back({key, 0u, 0u, nullptr});
+      g = graphs.end() - 1;
+    }
+    g->last = ++graph_clock;
+    if (!g->exec) {
+      if (++g->uses <= kGraphAfter) return false;
+      // the capture records the step without running it: what it leaves in the host's state is undone
+      struct Host {
+        DevState cur, alt;
+        bool flipped, nbl_ok, erec_ok, qual_ready, cells_clean;
+        int par;
+        uint n, m, n_sorted, n_flagged, cells_nkeys;
+        uint *skeys, *svals;
+        const uint *cells_keys;
+      } h{cur, alt, flipped, nbl_ok, erec_ok, qual_ready, cells_clean, par, n, m, n_sorted, n_flagged,
+          cells_nkeys, skeys, svals, cells_keys};
+      hipGraph_t rec = nullptr;
+      hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+      if (e == hipSuccess) {
+        n = m = bound;
+        nd = &cnt->n_pre;
+        q_step(flags);
+        launch_report(cnt, rep_seq, rep_dev, st);
+        nd = nullptr;
+        e = hipStreamEndCapture(st, &rec);
+      }
+      cur = h.cur, alt = h.alt, flipped = h.flipped, nbl_ok = h.nbl_ok, erec_ok = h.erec_ok;
+      qual_ready = h.qual_ready, cells_clean = h.cells_clean, par = h.par, n = h.n, m = h.m;
+      n_sorted = h.n_sorted, n_flagged = h.n_flagged, cells_nkeys = h.cells_nkeys;
+      skeys = h.skeys, svals = h.svals, cells_keys = h.cells_keys;
+      if (e == hipSuccess) e = hipGraphInstantiateWithFlags(&g->exec, rec, 0);
+      if (rec) (void)hipGraphDestroy(rec);
+      if (e != hipSuccess) {
+        g->exec = nullptr;
+        graphs_work = false;
+        (void)hipGetLastError();
+        return false;
+      }
+    }
+    if (hipGraphLaunch(g->exec, st) != hipSuccess) {
+      graphs_work = false;
+      (void)hipGetLastError();
+      return false;
+    }
+    // the host's state after q_step
+    std::swap(cur, alt);
+    flipped = !flipped;
+    par ^= 1;
+    skeys = sc.keys_alt;
+    svals = sc.vals_alt;
+    n_sorted = n;
+    cells_keys = nullptr;
+    cells_clean = false;
+    nbl_ok = false;
+    erec_ok = !(flags & (SPH_STEP_SPLIT | SPH_STEP_MERGE));
+    if (flags & SPH_STEP_SPLIT) n_flagged = n;
+    return true;
   }
 
   void clear_force_flags() {
@@ -689,7 +852,7 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
             c->alloc(c->sb.split, sph_bit_words(cap)) && c->alloc(c->sb.dead, sph_bit_words(cap)) &&
             c->alloc(c->sb.qual, sph_bit_words(cap)) && c->alloc(c->sb.toff, sph_bit_tiles(cap)) &&
             c->alloc(c->newslot, cap) && c->alloc(c->q2d, std::max<size_t>(c->P.total_cell, 1)) &&
-            c->alloc(c->cnt, 1) && c->alloc(c->aos_dev, cap * sizeof(SphParticle3D)) &&
+            c->alloc(c->cnt, 1) && c->alloc(c->rep_seq, 1) && c->alloc(c->aos_dev, cap * sizeof(SphParticle3D)) &&
             c->alloc(c->aux.frec, 3 * (size_t)cap) && c->alloc(c->aux.erec, cap) &&
             c->alloc(c->aux.nbl, (size_t)SPH_NBL_K * cap) && c->alloc(c->aux.nbl_cnt, cap);
   c->aux.nbl_stride = cap;
@@ -714,7 +877,8 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
     if (ok) sph_fill_u32(c->bins.ccount, 0u, c->P.total_cell, c->st);
   }
   c->sc.max_tiles = sph_sort_tiles(cap);
-  if (ok && hipHostMalloc((void **)&c->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
+  if (ok && (hipHostMalloc((void **)&c->rep, sizeof(Report), hipHostMallocDefault) != hipSuccess ||
+             hipHostGetDevicePointer((void **)&c->rep_dev, c->rep, 0) != hipSuccess))
     ok = false;
   if (ok && !c->tune.create()) ok = false;
   c->tune.start(kTuneRounds, kTuneAfter, kTuneEvery);
@@ -722,7 +886,9 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
     delete c;
     return SPH_ECAP;
   }
-  c->set_counts_on_device(0, 0);
+  std::memset(c->rep, 0, sizeof(Report));
+  sph_fill_u32(c->rep_seq, 0u, 1, c->st);
+  launch_upload(variant, c->aos_dev, 0, c->cur, 0, c->st, c->cnt, 0, 0);
   if (c->sync() != SPH_OK) {
     delete c;
     return SPH_EHIP;
@@ -743,6 +909,7 @@ int sph_set_params(SphCtx *ctx, const void *sysparam) {
   DevParams P = make_dev_params(ctx->variant, sysparam, ctx->cap);
   if (P.total_cell != ctx->P.total_cell || P.tot_dens != ctx->P.tot_dens) return SPH_EINVAL;
   std::memcpy(ctx->raw, sysparam, ctx->raw_size);
+  if (std::memcmp(&P, &ctx->P, sizeof(P)) != 0) ctx->drop_graphs();  // they hold the parameters
   ctx->P = P;
   ctx->nbl_ok = false;  // the pair lists were made with the old kernel radii
   return SPH_OK;
@@ -760,12 +927,9 @@ int sph_upload_particles(SphCtx *ctx, const void *aos, uint32_t n) {
   if (n > ctx->cap) return SPH_ECAP;
   if (n > 0 && !aos) return SPH_EINVAL;
   const size_t rec = ctx->variant == SPH_V2D ? sizeof(SphParticle2D) : sizeof(SphParticle3D);
-  if (n > 0) {
-    if (hipMemcpyAsync(ctx->aos_dev, aos, rec * n, hipMemcpyHostToDevice, ctx->st) != hipSuccess)
-      return SPH_EHIP;
-    launch_upload_scatter(ctx->variant, ctx->aos_dev, n, ctx->cur, ctx->st);
-  }
-  ctx->set_counts_on_device(n, n);
+  if (n > 0 && hipMemcpyAsync(ctx->aos_dev, aos, rec * n, hipMemcpyHostToDevice, ctx->st) != hipSuccess)
+    return SPH_EHIP;
+  launch_upload(ctx->variant, ctx->aos_dev, n, ctx->cur, 0, ctx->st, ctx->cnt, n, n);
   ctx->hashed = ctx->sorted = ctx->lists_valid = ctx->merged = false;
   ctx->erec_ok = false;
   ctx->nbl_ok = false;
@@ -778,12 +942,10 @@ int sph_download_particles(SphCtx *ctx, void *aos, uint32_t n) {
   if (n == 0) return SPH_OK;
   if (!aos) return SPH_EINVAL;
   const size_t rec = ctx->variant == SPH_V2D ? sizeof(SphParticle2D) : sizeof(SphParticle3D);
-  // slot -> physical map of the current numbering (scratch: newslot)
-  launch_slot2phys(ctx->cur, ctx->m, ctx->newslot, ctx->st);
-  launch_download_gather(ctx->variant, ctx->cur, ctx->newslot, n, ctx->aos_dev, ctx->st);
+  launch_download(ctx->variant, ctx->cur, Span{0u, ctx->m, 0u, 0u}, n, ctx->aos_dev, ctx->st);
   if (hipMemcpyAsync(aos, ctx->aos_dev, rec * n, hipMemcpyDeviceToHost, ctx->st) != hipSuccess)
     return SPH_EHIP;
-  return ctx->sync();
+  return ctx->drain();
 }
 
 int sph_num_particles(SphCtx *ctx, uint32_t *n) {
@@ -801,7 +963,7 @@ int sph_calc_hash(SphCtx *ctx) {
   if (rc) return rc;
   ctx->hashed = true;
   ctx->sorted = ctx->lists_valid = ctx->merged = false;
-  return ctx->cnt_host->err ? SPH_EDOMAIN : SPH_OK;
+  return ctx->rep->c.err ? SPH_EDOMAIN : SPH_OK;
 }
 
 int sph_sort(SphCtx *ctx) {
@@ -857,8 +1019,8 @@ int sph_split(SphCtx *ctx, uint32_t *n_requested, uint32_t *n_done) {
   ctx->q_split();
   int rc = ctx->sync();
   if (rc) return rc;
-  if (n_requested) *n_requested = ctx->cnt_host->s_req;
-  if (n_done) *n_done = ctx->cnt_host->s_done;
+  if (n_requested) *n_requested = ctx->rep->c.s_req;
+  if (n_done) *n_done = ctx->rep->c.s_done;
   return SPH_OK;
 }
 
@@ -870,7 +1032,7 @@ int sph_merge(SphCtx *ctx, uint32_t *groups) {
   int rc = ctx->sync();
   if (rc) return rc;
   ctx->merged = true;
-  if (groups) *groups = ctx->cnt_host->groups;
+  if (groups) *groups = ctx->rep->c.groups;
   return SPH_OK;
 }
 
@@ -909,31 +1071,17 @@ int sph_marching_cubes(SphCtx *ctx, uint32_t *n_tri) {
   ctx->q_mc();
   int rc = ctx->sync();
   if (rc) return rc;
-  if (n_tri) *n_tri = ctx->cnt_host->ntri;
-  return ctx->cnt_host->ntri > ctx->max_tri ? SPH_ETRI : SPH_OK;
+  if (n_tri) *n_tri = ctx->rep->c.ntri;
+  return ctx->rep->c.ntri > ctx->max_tri ? SPH_ETRI : SPH_OK;
 }
 
 int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
   CHECK_CTX(ctx);
   if (ctx->n == 0) return SPH_EEMPTY;
-  const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
-  ctx->q_bin_step(do_split, do_merge);
-  ctx->q_density();
-  ctx->q_force(true);
-  ctx->q_integrate();
-  if ((flags & SPH_STEP_MC) && ctx->P.dim == 3 && ctx->dgrid) {
-    ctx->q_dgrid();
-    ctx->q_normals();
-    ctx->q_mc();
-  }
-  ctx->q_energy(true, do_split, do_merge);
-  if (do_split) ctx->q_split(true);
-  if (do_merge) {
-    ctx->q_merge(true);
-    ctx->q_compact(true);
-  }
+  const bool reported = ctx->graph_step(flags);
+  if (!reported) ctx->q_step(flags);
   // the cell-range phase made physical == live before split appended children
-  int rc = ctx->sync();
+  int rc = ctx->sync(reported);
   if (rc == SPH_OK) ctx->tune.end_step();
   ctx->clear_force_flags();
   ctx->hashed = ctx->sorted = ctx->merged = false;
@@ -941,7 +1089,7 @@ int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
   if (rc) return rc;
   if (flags & SPH_STEP_MERGE) ctx->n_status = ctx->m;
   if (n_out) *n_out = ctx->n;
-  return ctx->cnt_host->err ? SPH_EDOMAIN : SPH_OK;
+  return ctx->rep->c.err ? SPH_EDOMAIN : SPH_OK;
 }
 
 static size_t count_of(SphCtx *ctx, int which) {
@@ -956,7 +1104,7 @@ static size_t count_of(SphCtx *ctx, int which) {
     case SPH_Q_DGRID: return ctx->dgrid ? ctx->P.tot_dens : 0;
     case SPH_Q_NORMAL: return ctx->dgrid ? (size_t)ctx->P.tot_dens * 3 : 0;
     case SPH_Q_TRI: {
-      uint nt = ctx->cnt_host->ntri < ctx->max_tri ? ctx->cnt_host->ntri : ctx->max_tri;
+      uint nt = ctx->rep->c.ntri < ctx->max_tri ? ctx->rep->c.ntri : ctx->max_tri;
       return ctx->tris ? (size_t)nt * 18 : 0;
     }
   }
@@ -992,7 +1140,7 @@ int sph_get_u32(SphCtx *ctx, int which, uint32_t *out, size_t n) {
   if (hipMemcpyAsync(bits ? w.data() : out, src, (bits ? w.size() : n) * 4, hipMemcpyDeviceToHost,
                      ctx->st) != hipSuccess)
     return SPH_EHIP;
-  int rc = ctx->sync();
+  int rc = ctx->drain();
   if (rc) return rc;
   for (size_t k = 0; bits && k < n; k++)
     out[k] = ((w[k >> 5] >> (k & 31)) & 1u) ^ (which == SPH_Q_SPLITFLAG ? 1u : 0u);
@@ -1011,7 +1159,7 @@ int sph_get_f32(SphCtx *ctx, int which, float *out, size_t n) {
     default: return SPH_EINVAL;
   }
   if (hipMemcpyAsync(out, src, n * 4, hipMemcpyDeviceToHost, ctx->st) != hipSuccess) return SPH_EHIP;
-  return ctx->sync();
+  return ctx->drain();
 }
 
 int sph_autotune(SphCtx *ctx, uint32_t rounds, uint32_t after_steps, uint32_t every_steps) {

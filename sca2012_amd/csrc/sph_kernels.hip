@@ -1043,6 +1043,20 @@ __global__ void k_begin_step(Counters *cnt) {
 
 __global__ void k_set_phys_count(Counters *cnt) { cnt->m = cnt->n; }
 
+// The counters into pinned host memory, then the number of this report (one wave).
+__global__ __launch_bounds__(64) void k_report(const Counters *__restrict__ cnt, uint *__restrict__ seq,
+                                               Report *__restrict__ host) {
+  const uint t = threadIdx.x;
+  if (t < sizeof(Counters) / 4)
+    reinterpret_cast<uint *>(&host->c)[t] = reinterpret_cast<const uint *>(cnt)[t];
+  __threadfence_system();
+  if (t == 0u) {
+    const uint s = *seq + 1u;
+    *seq = s;
+    __hip_atomic_store(&host->seq, s, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // A15 integrate_dens_kernel + integrate_cell_dens (SPH-3D-2/sph_system.cu:1842-2183):
 // voxel v (x fastest) gathers poly6 (particle radius) splats from the 27 cells around
@@ -1394,37 +1408,63 @@ __global__ __launch_bounds__(BLK) void k_mc_emit(DevParams P, const float *__res
 // ---------------------------------------------------------------------------------------
 // AoS <-> SoA (copy_array boundary)
 // ---------------------------------------------------------------------------------------
+// AoS records -> entries [base, base + n) of S, entry base + i with slot word slot_or | i. cnt
+// (optional): the counters of `live` particles in `entries` entries. A batch (scn): the scene's
+// entries in `old` (before base) are removed and the scenes' counters start over.
 template <int V>
-__global__ __launch_bounds__(BLK) void k_upload(const void *__restrict__ aos, uint n, DevState S,
-                                                uint slot_or) {
+__global__ __launch_bounds__(BLK) void k_upload(const void *__restrict__ aos, uint n, DevState S, uint base,
+                                                uint slot_or, Span old, Counters *cnt, uint live,
+                                                uint entries, SceneCnt *__restrict__ scn, uint ns) {
   const uint i = blockIdx.x * BLK + threadIdx.x;
+  if (cnt && i == 0u) {
+    Counters c = {};
+    c.n = c.n_pre = live;
+    c.m = entries;
+    *cnt = c;
+  }
+  if (i < ns) {
+    SceneCnt c = {};
+    c.n = c.n_pre = i == slot_or >> SPH_SCENE_SHIFT ? n : scn[i].n;
+    scn[i] = c;
+  }
+  auto remove = [&](uint k) {
+    if ((S.slot[k] ^ slot_or) >> SPH_SCENE_SHIFT == 0u) S.slot[k] = SPH_DEAD;
+  };
+  if (i < old.na) remove(old.a + i);
+  if (i < old.nb) remove(old.b + i);
   if (i >= n) return;
+  const uint k = base + i;
   if (V == SPH_V2D) {
     const SphParticle2D q = ((const SphParticle2D *)aos)[i];
-    S.pos[i] = make_float4(q.pos.x, q.pos.y, 0.0f, __uint_as_float(q.level));
-    S.vel[i] = make_float4(q.vel.x, q.vel.y, 0.0f, 0.0f);
-    S.ev[i] = make_float4(q.ev.x, q.ev.y, 0.0f, 0.0f);
-    S.acc[i] = make_float4(q.acc.x, q.acc.y, 0.0f, q.surface_normal);
-    S.dp[i] = make_float2(q.dens, q.pres);
-    S.energy[i] = q.energy;
+    S.pos[k] = make_float4(q.pos.x, q.pos.y, 0.0f, __uint_as_float(q.level));
+    S.vel[k] = make_float4(q.vel.x, q.vel.y, 0.0f, 0.0f);
+    S.ev[k] = make_float4(q.ev.x, q.ev.y, 0.0f, 0.0f);
+    S.acc[k] = make_float4(q.acc.x, q.acc.y, 0.0f, q.surface_normal);
+    S.dp[k] = make_float2(q.dens, q.pres);
+    S.energy[k] = q.energy;
   } else {
     const SphParticle3D q = ((const SphParticle3D *)aos)[i];
-    S.pos[i] = make_float4(q.pos.x, q.pos.y, q.pos.z, __uint_as_float(q.level));
-    S.vel[i] = make_float4(q.vel.x, q.vel.y, q.vel.z, 0.0f);
-    S.ev[i] = make_float4(q.ev.x, q.ev.y, q.ev.z, q.tension);
-    S.acc[i] = make_float4(q.acc.x, q.acc.y, q.acc.z, q.surface);
-    S.dp[i] = make_float2(q.dens, q.press);
-    S.energy[i] = q.energy;
+    S.pos[k] = make_float4(q.pos.x, q.pos.y, q.pos.z, __uint_as_float(q.level));
+    S.vel[k] = make_float4(q.vel.x, q.vel.y, q.vel.z, 0.0f);
+    S.ev[k] = make_float4(q.ev.x, q.ev.y, q.ev.z, q.tension);
+    S.acc[k] = make_float4(q.acc.x, q.acc.y, q.acc.z, q.surface);
+    S.dp[k] = make_float2(q.dens, q.press);
+    S.energy[k] = q.energy;
   }
-  S.slot[i] = slot_or | i;
+  S.slot[k] = slot_or | i;
 }
 
+// The first n records, by slot, of the scene whose slot words start with the bits `scene`; `at`
+// holds its entries, and may hold removed ones and other scenes'. Each thread reads its entry's
+// fields in order and writes one record, so no slot -> entry map is made first.
 template <int V>
-__global__ __launch_bounds__(BLK) void k_download(DevState S, const uint *__restrict__ slot2phys,
-                                                  uint n, void *__restrict__ aos) {
-  const uint s = blockIdx.x * BLK + threadIdx.x;
-  if (s >= n) return;
-  const uint k = slot2phys[s];
+__global__ __launch_bounds__(BLK) void k_download(DevState S, Span at, uint scene, uint n,
+                                                  void *__restrict__ aos) {
+  const uint i = blockIdx.x * BLK + threadIdx.x;
+  if (i >= at.na + at.nb) return;
+  const uint k = i < at.na ? at.a + i : at.b + (i - at.na);
+  const uint w = S.slot[k], s = w - scene;
+  if (w == SPH_DEAD || s >= n) return;
   const float4 p = S.pos[k], v = S.vel[k], e = S.ev[k], a = S.acc[k];
   const float2 d = S.dp[k];
   if (V == SPH_V2D) {
@@ -1556,21 +1596,6 @@ __global__ __launch_bounds__(SCN_BLK) void k_batch_compact_plan(SceneCnt *scn, u
     scn[t].n -= gone;
   }
   if (t == 0) cnt->n -= tot;
-}
-
-__global__ __launch_bounds__(BLK) void k_scene_kill(uint *__restrict__ slot, uint m, uint scene) {
-  const uint k = blockIdx.x * BLK + threadIdx.x;
-  if (k >= m) return;
-  const uint w = slot[k];
-  if (w != SPH_DEAD && (w >> SPH_SCENE_SHIFT) == scene) slot[k] = SPH_DEAD;
-}
-
-__global__ __launch_bounds__(BLK) void k_scene_slot2phys(const uint *__restrict__ slot, uint m,
-                                                         uint scene, uint *__restrict__ s2p) {
-  const uint k = blockIdx.x * BLK + threadIdx.x;
-  if (k >= m) return;
-  const uint w = slot[k];
-  if (w != SPH_DEAD && (w >> SPH_SCENE_SHIFT) == scene) s2p[w & SPH_LOCAL_MASK] = k;
 }
 
 __global__ __launch_bounds__(BLK) void k_live_flags(const uint *__restrict__ slot, uint m,
@@ -1792,6 +1817,11 @@ void launch_merge(int variant, const DevParams &P, DevState s, const uint *cstar
                   dead, cnt, by_entry ? skeys : nullptr, nkeys_dev, nkeys, group_out, qbits);
 }
 
+void launch_report(const Counters *cnt, uint *seq, Report *host, hipStream_t st) {
+  static_assert(sizeof(Counters) / 4 <= 64, "one wave copies the counters");
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, cnt, seq, host);
+}
+
 void launch_begin_step(Counters *cnt, hipStream_t st) {
   hipLaunchKernelGGL(k_begin_step, dim3(1), dim3(1), 0, st, cnt);
 }
@@ -1808,16 +1838,6 @@ void launch_batch_split_plan(int variant, const BatchView &bv, Counters *cnt, hi
 void launch_batch_compact_plan(int variant, const BatchView &bv, Counters *cnt, hipStream_t st) {
   if (variant == SPH_V3D4) k_batch_compact_plan<4><<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, cnt);
   else k_batch_compact_plan<2><<<1, SCN_BLK, 0, st>>>(bv.scn, bv.n_scenes, cnt);
-}
-
-void launch_scene_kill(DevState s, uint m, uint scene, hipStream_t st) {
-  if (m == 0) return;
-  k_scene_kill<<<grid_for(m), dim3(BLK), 0, st>>>(s.slot, m, scene);
-}
-
-void launch_scene_slot2phys(DevState s, uint m, uint scene, uint *slot2phys, hipStream_t st) {
-  if (m == 0) return;
-  k_scene_slot2phys<<<grid_for(m), dim3(BLK), 0, st>>>(s.slot, m, scene, slot2phys);
 }
 
 void launch_pack_live(DevState src, DevState dst, uint m, uint *flags, uint *pos, uint *tmp,
@@ -1917,16 +1937,16 @@ void launch_mc_emit(const DevParams &P, const float *dgrid, const float *normal3
                      max_tri, tris);
 }
 
-void launch_upload_scatter(int variant, const void *aos_dev, uint n, DevState s, hipStream_t st,
-                           uint slot_or) {
-  if (n == 0) return;
-  SPH_DISPATCH(variant, k_upload, grid_for(n), dim3(BLK), 0, st, aos_dev, n, s, slot_or);
+void launch_upload(int variant, const void *aos_dev, uint n, DevState s, uint base, hipStream_t st,
+                   Counters *cnt, uint live, uint entries, uint slot_or, Span old, const BatchView *bv) {
+  SPH_DISPATCH(variant, k_upload, grid_for(std::max(std::max(n, 1u), std::max(old.na, old.nb))), dim3(BLK), 0,
+               st, aos_dev, n, s, base, slot_or, old, cnt, live, entries, scn_of(bv), bv ? bv->n_scenes : 0u);
 }
 
-void launch_download_gather(int variant, DevState s, const uint *slot2phys, uint n, void *aos_dev,
-                            hipStream_t st) {
-  if (n == 0) return;
-  SPH_DISPATCH(variant, k_download, grid_for(n), dim3(BLK), 0, st, s, slot2phys, n, aos_dev);
+void launch_download(int variant, DevState s, Span at, uint n, void *aos_dev, hipStream_t st, uint scene) {
+  const uint m = at.na + at.nb;
+  if (n == 0 || m == 0) return;
+  SPH_DISPATCH(variant, k_download, grid_for(m), dim3(BLK), 0, st, s, at, scene, n, aos_dev);
 }
 
 void launch_slot2phys(DevState s, uint m, uint *slot2phys, hipStream_t st) {
