@@ -957,7 +957,7 @@ struct SphAdj {
     launch_bin_place(S, bins, cs, cnt, cap, st, 0, child ? sb.split : nullptr, partner ? sb.dead : nullptr, 1u,
                      (uint)sph_bit_words(cap));
     launch_bin_reorder(S, T, bins, cs, ce, sc.keys_alt, sc.vals_alt, s2p_cell, cnt, cap, st, true, set_m,
-                       nullptr, 0, child, partner);
+                       nullptr, 0, child, partner, QPosOut{aux.qpos, P.q, nullptr});
   }
   // one forward step of state S (counters in cnt): cell order into the tape entry, next
   // state back into S; no host round trip
@@ -972,7 +972,8 @@ struct SphAdj {
       sph_radix_sort(keys, vals, cap, kbits, sc, &skeys, &svals, st, nd);
       sph_fill_cells(t.cs, t.ce, cells, st);
       launch_cell_bounds(skeys, cap, cells, t.cs, t.ce, st, nd);
-      launch_reorder(S, t.T, svals, s2p_hash, cap, s2p_cell, st, cnt, true, nd);  // and m = n
+      launch_reorder(S, t.T, svals, s2p_hash, cap, s2p_cell, st, cnt, true, nd, 0,
+                     QPosOut{aux.qpos, P.q, nullptr});  // and m = n
       sph_fill_u32(t.child, SPH_DEAD, cap, st);
       sph_fill_u32(t.partner, SPH_DEAD, cap, st);
       sph_fill_u32(sb.split, 0u, sph_bit_words(cap), st);
@@ -983,9 +984,9 @@ struct SphAdj {
     k_adj_integrate_fwd<<<agrid(cap), ABLK, 0, st>>>(P, theta, nf, t.T, S, nd, cap);
     const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
     if (do_split || do_merge) {  // the energy decides split and merge (SPH-3D-2/sph_system.cpp:356)
-      launch_make_erec(S, cap, aux.erec, st, nd);
-      launch_energy(SPH_V3D2, P, S, t.cs, t.ce, cap, st, nullptr, kEnergyListDefault,
-                    do_split ? sb.split : nullptr, nullptr, aux.erec, nd, aux.fine_energy);
+      launch_make_erec(P, S, cap, aux, st, nd);
+      launch_energy(SPH_V3D2, P, S, aux, t.cs, t.ce, cap, st, nullptr, do_split ? sb.split : nullptr,
+                    nullptr, nd);
     }
     if (do_split) launch_split(SPH_V3D2, P, S, cap, sb, s2p_cell, cnt, st, false, nullptr, t.child);
     if (do_merge) {
@@ -1088,7 +1089,7 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
             a->alloc(a->cs_scr, a->cells) && a->alloc(a->ce_scr, a->cells) &&
             a->alloc(a->sb.split, sph_bit_words(cap)) && a->alloc(a->sb.dead, sph_bit_words(cap)) &&
             a->alloc(a->sb.toff, sph_bit_tiles(cap)) &&
-            a->alloc(a->cnt, 1) && a->alloc(a->aux.frec, 3 * cap) && a->alloc(a->aux.erec, cap) &&
+            a->alloc(a->cnt, 1) && a->alloc(a->aux.frec, 3 * cap) && a->alloc(a->aux.erec, cap) && a->alloc(a->aux.ez, cap) && a->alloc(a->aux.qpos, cap) &&
             a->alloc(a->aux.nbl, (size_t)SPH_NBL_K * cap) && a->alloc(a->aux.nbl_cnt, cap) &&
             a->alloc(a->theta, nth) && a->alloc(a->dtheta, nth) && a->alloc(a->th_part, iblocks * nth) &&
             a->alloc(a->th_csum, ((iblocks + THETA_CHUNK - 1) / THETA_CHUNK) * nth) &&

@@ -435,7 +435,7 @@ struct SphBatch {
       pbegin(SPH_P_REORDER);
       // and m = n; acc, dp and energy are recomputed by the step's kernels below
       launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, mb, st, false, true,
-                         &bv, grid);
+                         &bv, grid, nullptr, nullptr, QPosOut{aux.qpos, {}, Ptab});
       pend();
     } else {
       pbegin(SPH_P_HASH);
@@ -449,7 +449,8 @@ struct SphBatch {
       launch_cell_bounds(skeys, Mb, total_cell, cstart, cend, st, n_live, grid);
       pend();
       pbegin(SPH_P_REORDER);
-      launch_reorder(cur, alt, svals, s2p_hash, Mb, s2p_cell, st, cnt, false, n_live, grid);
+      launch_reorder(cur, alt, svals, s2p_hash, Mb, s2p_cell, st, cnt, false, n_live, grid,
+                     QPosOut{aux.qpos, {}, Ptab});
       if (do_split) sph_fill_u32(sb.split, 0u, sph_bit_words(Mb), st);
       if (do_merge) sph_fill_u32(sb.dead, 0u, sph_bit_words(Ma), st);
       pend();
@@ -466,16 +467,15 @@ struct SphBatch {
     else tune.run(0, st, force);
     pend();
     pbegin(SPH_P_INTEGRATE);
-    launch_integrate(v, P0, cur, Mb, st, &bv, aux.erec, n_live, grid);
+    launch_integrate(v, P0, cur, Mb, st, &bv, aux, n_live, grid);
     pend();
     pbegin(SPH_P_ENERGY);
     uint *split_bits = do_split ? sb.split : nullptr;  // the energy kernel decides splits
     uint *qual = do_merge && !aux.fine_energy ? sb.qual : nullptr;
     DevParams Pe = P0;  // the energy kernel's unit-length path only if every scene takes it
     Pe.energy_unit = energy_unit_all() ? 1 : 0;
-    auto energy = [&](int c) {
-      launch_energy(v, Pe, cur, cstart, cend, Mb, st, &bv, c, split_bits, qual, aux.erec, n_live,
-                    aux.fine_energy);
+    auto energy = [&](int) {
+      launch_energy(v, Pe, cur, aux, cstart, cend, Mb, st, &bv, split_bits, qual, n_live);
     };
     if (dev) energy(le);
     else tune.run(1, st, energy);
@@ -638,7 +638,7 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
             b->alloc(b->sb.qual, sph_bit_words(cap)) && b->alloc(b->sb.toff, sph_bit_tiles(cap)) &&
             b->alloc(b->newslot, cap) && b->alloc(b->cnt, 1) && b->alloc(b->scn, n_scenes) &&
             b->alloc(b->Ptab, n_scenes) && b->alloc(b->aos_dev, (size_t)b->max_cap * b->rec) &&
-            b->alloc(b->aux.frec, 3 * cap) && b->alloc(b->aux.erec, cap) &&
+            b->alloc(b->aux.frec, 3 * cap) && b->alloc(b->aux.erec, cap) && b->alloc(b->aux.ez, cap) && b->alloc(b->aux.qpos, cap) &&
             b->alloc(b->aux.nbl, (size_t)SPH_NBL_K * cap) && b->alloc(b->aux.nbl_cnt, cap) &&
             b->alloc(b->scan_tmp, sph_scan_tmp_elems(scan_n)) && b->alloc(b->sc.len_dev, 1);
   b->aux.nbl_stride = (uint)cap;

@@ -221,7 +221,7 @@ __global__ __launch_bounds__(BLK) void k_bin_reorder(DevState src, DevState dst,
                                                      uint m_host, uint *__restrict__ skeys,
                                                      uint *__restrict__ svals, uint *__restrict__ s2p,
                                                      bool all, bool set_m, uint *__restrict__ init0,
-                                                     uint *__restrict__ init1) {
+                                                     uint *__restrict__ init1, QPosOut qo) {
   if (set_m && blockIdx.x == 0 && threadIdx.x == 0) cnt->m = cnt->n;  // physical == live
   // XCD-contiguous blocks keep a single scene's destinations in one L2 (498k: 24.4 -> 22 us); a
   // batch's were slower that way (81 -> 96 us)
@@ -239,6 +239,7 @@ __global__ __launch_bounds__(BLK) void k_bin_reorder(DevState src, DevState dst,
            (uint)((d < w) & (j + 3u < t));
     }
     dst.pos[q] = p;
+    put_qpos<B>(qo, q, w, p);
     dst.vel[q] = v;
     dst.ev[q] = e;
     if (all) {
@@ -306,14 +307,14 @@ void launch_bin_place(DevState src, const BinScratch &bs, const uint *cstart, co
 void launch_bin_reorder(DevState src, DevState dst, const BinScratch &bs, const uint *cstart,
                         const uint *cend, uint *skeys, uint *svals, uint *s2p, Counters *cnt, uint m,
                         hipStream_t st, bool all_fields, bool set_m, const BatchView *bv, uint grid,
-                        uint *init0, uint *init1) {
+                        uint *init0, uint *init1, QPosOut qo) {
   if (m == 0) return;
   if (bv)
     k_bin_reorder<true><<<bgrid(grid, m), dim3(BLK), 0, st>>>(
         src, dst, bv->scn, bs.hkey, cstart, cend, bs.bslot, cnt, m, skeys, svals, s2p, all_fields, set_m,
-        init0, init1);
+        init0, init1, qo);
   else
     k_bin_reorder<false><<<bgrid(grid, m), dim3(BLK), 0, st>>>(
         src, dst, nullptr, bs.hkey, cstart, cend, bs.bslot, cnt, m, skeys, svals, s2p, all_fields, set_m,
-        init0, init1);
+        init0, init1, qo);
 }

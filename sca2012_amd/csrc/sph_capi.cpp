@@ -239,6 +239,18 @@ DevParams make_dev_params(int variant, const void *raw, uint cap) {
     for (float d : {P.kernel[l], P.sqrt_kernel[l]})
       if (!(d >= 0x1p-20f && d <= 0x1p20f)) P.kernel_div_fast = 0;
   }
+  // steps for the quantised distance test (sph_near_q), from the longer kernel
+  const double hq = std::sqrt((double)std::max(P.k2[0], P.k2[1]));
+  P.q = QParams{0.0f, {-1, -1}, 0u, 0u};  // every position the same: no pair is ruled out
+  if (hq > 1e-30 && hq < 1e30 && P.k2[0] >= 0.0f && P.k2[1] >= 0.0f) {
+    P.q.scale = (float)std::exp2(std::floor(std::log2(4096.0 / hq)));
+    for (int l = 0; l < 2; l++) {
+      const double r = std::sqrt((double)P.k2[l]) * P.q.scale * (1.0 + 1e-5) + 2.0;
+      P.q.neg[l] = -(int)std::ceil(r * r);
+    }
+    P.q.mark_level = P.k2[1] <= P.k2[0] ? 1u : 0u;
+    P.q.mark = (uint)std::sqrt((double)std::abs(P.q.neg[0] - P.q.neg[1])) & ~1u;
+  }
   P.energy_unit = 1;
   for (int l = 0; l < (P.dim == 3 ? 1 : 2); l++)
     if (!(P.kernel[l] == 1.0f && P.sqrt_kernel[l] == 1.0f)) P.energy_unit = 0;
@@ -508,6 +520,7 @@ struct SphCtx {
   }
   // in_step: the step's density, force and energy kernels follow, so the reorder leaves out
   // the fields they overwrite
+  QPosOut qout() const { return QPosOut{aux.qpos, P.q, nullptr}; }
   void q_cells(bool in_step = false) {
     nbl_ok = false;
     pbegin(SPH_P_CELLS);
@@ -518,7 +531,8 @@ struct SphCtx {
     cells_clean = false;
     pend();
     pbegin(SPH_P_REORDER);
-    launch_reorder(cur, alt, svals, s2p_hash, n, s2p_cell, st, cnt, !in_step);  // and m = n
+    launch_reorder(cur, alt, svals, s2p_hash, n, s2p_cell, st, cnt, !in_step, nullptr, 0,
+                   qout());  // and m = n
     pend();
     erec_ok = false;
     std::swap(cur, alt);
@@ -556,7 +570,8 @@ struct SphCtx {
                      (uint)sph_bit_words(cap));
     pend();
     pbegin(SPH_P_REORDER);
-    launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, m, st, false);
+    launch_bin_reorder(cur, alt, bins, cstart, cend, skeys, svals, s2p_cell, cnt, m, st, false, true, nullptr,
+                       0, nullptr, nullptr, qout());
     pend();
     std::swap(cur, alt);
     flipped = !flipped;
@@ -566,9 +581,10 @@ struct SphCtx {
     const uint64_t most = (uint64_t)k * (variant == SPH_V3D4 ? 4u : 2u);
     return most < cap ? (uint)most : std::max(cap, k);
   }
-  void q_density() {
+  void q_density(bool in_step = false) {
     pbegin(SPH_P_DENSITY);
     if (!nd) aux.choose_forms(variant, false, n);
+    if (!in_step && !aux.fine_density) launch_make_erec(P, cur, n, aux, st);  // for qpos
     launch_density(variant, P, cur, aux, cstart, cend, n, st, nullptr, nd);
     pend();
     nbl_ok = true;
@@ -588,7 +604,7 @@ struct SphCtx {
   void q_integrate() {
     nbl_ok = false;
     pbegin(SPH_P_INTEGRATE);
-    launch_integrate(variant, P, cur, n, st, nullptr, aux.erec, nd);
+    launch_integrate(variant, P, cur, n, st, nullptr, aux, nd);
     pend();
     erec_ok = true;
   }
@@ -597,14 +613,14 @@ struct SphCtx {
   void q_energy(bool tuned = false, bool do_split = false, bool do_merge = false) {
     pbegin(SPH_P_ENERGY);
     if (!erec_ok) {  // not straight after integrate: records from the current state
-      launch_make_erec(cur, n, aux.erec, st);
+      launch_make_erec(P, cur, n, aux, st);
       erec_ok = true;
     }
     if (!nd) aux.choose_forms(variant, false, n);
     qual_ready = do_merge && !aux.fine_energy;
-    auto go = [&](int c) {
-      launch_energy(variant, P, cur, cstart, cend, n, st, nullptr, c, do_split ? sb.split : nullptr,
-                    qual_ready ? sb.qual : nullptr, aux.erec, nd, aux.fine_energy);
+    auto go = [&](int) {
+      launch_energy(variant, P, cur, aux, cstart, cend, n, st, nullptr, do_split ? sb.split : nullptr,
+                    qual_ready ? sb.qual : nullptr, nd);
     };
     if (tuned) tune.run(1, st, go);
     else go(tune.energy);
@@ -668,7 +684,7 @@ struct SphCtx {
   void q_step(uint flags) {
     const bool do_split = (flags & SPH_STEP_SPLIT) != 0, do_merge = (flags & SPH_STEP_MERGE) != 0;
     q_bin_step(do_split, do_merge);
-    q_density();
+    q_density(true);
     q_force(true);
     q_integrate();
     if ((flags & SPH_STEP_MC) && P.dim == 3 && dgrid) {
@@ -853,7 +869,7 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
             c->alloc(c->sb.qual, sph_bit_words(cap)) && c->alloc(c->sb.toff, sph_bit_tiles(cap)) &&
             c->alloc(c->newslot, cap) && c->alloc(c->q2d, std::max<size_t>(c->P.total_cell, 1)) &&
             c->alloc(c->cnt, 1) && c->alloc(c->rep_seq, 1) && c->alloc(c->aos_dev, cap * sizeof(SphParticle3D)) &&
-            c->alloc(c->aux.frec, 3 * (size_t)cap) && c->alloc(c->aux.erec, cap) &&
+            c->alloc(c->aux.frec, 3 * (size_t)cap) && c->alloc(c->aux.erec, cap) && c->alloc(c->aux.ez, cap) && c->alloc(c->aux.qpos, cap) &&
             c->alloc(c->aux.nbl, (size_t)SPH_NBL_K * cap) && c->alloc(c->aux.nbl_cnt, cap);
   c->aux.nbl_stride = cap;
   if (ok && c->P.dim == 3 && c->P.tot_dens > 0) {

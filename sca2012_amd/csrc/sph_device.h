@@ -66,6 +66,12 @@ __device__ inline const DevParams &scene_params(const DevParams &P0,
   else return P0;
 }
 
+// entry q of the quantised positions (w: its slot word)
+template <bool B> __device__ inline void put_qpos(const QPosOut &qo, uint q, uint w, const float4 &p) {
+  if (!qo.q) return;
+  qo.q[q] = sph_qpos(p.x, p.y, p.z, __float_as_uint(p.w), B ? qo.Ptab[w >> SPH_SCENE_SHIFT].q : qo.Q);
+}
+
 // calc_grid_pos (SPH-3D-2/sph_system.cu:18-27): (uint)floor(p / cell_size); false when the
 // coordinate is outside [0, ncell) or NaN.
 template <int V>
@@ -146,8 +152,7 @@ __device__ inline void nb_range(const DevParams &P, int o, const uint c[3],
 // Interacting-pair lists: entry = (offset index << 27) | particle index, kept in LDS
 // column-major ([k][thread]) so a wave's accesses hit distinct banks.
 // The list length only moves the drain points, never the order in which a particle's
-// pairs are summed, so every length gives the same bits; the autotuner picks one per
-// kernel (sph_internal.h: kForceLists, kEnergyLists).
+// pairs are summed, so every length gives the same bits (sph_internal.h: kForceLists).
 __device__ inline uint pack_entry(int o, uint j) { return ((uint)o << 27) | j; }
 
 // Split decision of the particle with slot word w: its bit by slot (a batch: by dense slot, and

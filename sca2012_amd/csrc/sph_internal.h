@@ -26,6 +26,15 @@ typedef unsigned int uint;
 #define SPH_DEAD 0xffffffffu
 #define SPH_EMPTY 0xffffffffu
 
+// Quantised positions (sph_near_q): steps per unit length; per level, minus the squared distance in
+// steps below which a pair may interact; the level of the smaller kernel radius, and the mark that
+// its particles carry (even; its square is at most the difference of the two squared distances).
+struct QParams {
+  float scale;
+  int neg[2];
+  uint mark, mark_level;
+};
+
 // Parameters as a by-value kernel argument (no __constant__ global, so contexts are
 // independent). Index [0] = large particles (level 1), [1] = small (level 2).
 struct DevParams {
@@ -62,6 +71,7 @@ struct DevParams {
   // 1 when every particle's energy kernel length h and sqrt(h) are exactly 1 (3D: the large
   // level's, which both levels use; 2D: both levels'), so x/h and x/sqrt(h) equal x
   int energy_unit;
+  QParams q;  // quantised positions (struct Aux: qpos)
 };
 
 // Per-step per-particle factors written by the density kernel for the force kernel.
@@ -71,8 +81,8 @@ struct DevParams {
 //   vpd.x vpd.y ev.x ev.y | gr_0 lc_0 ev.z - | gr_1 lc_1 ev.z -    (2D: vpd.x vpd.y ev.x ev.y)
 // with vpd = (m/dens, press/dens^2), gr_L = ((-grad_L) m)/dens and lc_L = (lapc_L m)/dens
 // for L = large (0), small (1): a receiver of level L reads the first part and part 1 + L.
-// erec: what the energy kernel reads of a neighbour, (pos.x, pos.y, vel.x, vel.y) after
-// integration, written by the integrate kernel (the z components never reach the energy).
+// erec, ez: what the energy kernel reads of a neighbour, (pos.x, pos.y, vel.x, vel.y) and pos.z
+// after integration, written by the integrate kernel (the velocity's z never reaches the energy).
 // nbl (optional): the force kernel's interacting pairs, written by the density kernel,
 // which walks the same candidates in the same order: entries packed as
 // (offset index << 27) | j in visiting order, four to a 16-byte group, group g of
@@ -80,10 +90,16 @@ struct DevParams {
 // group are one contiguous run); nbl_cnt[i] entries. A count above SPH_NBL_K means the
 // list overflowed (the entries past SPH_NBL_K are not stored) and the force kernel walks
 // the cells itself for that particle's wave.
+// qpos: the positions in steps of 1/q.scale, modulo 2^16, x | y << 16 and z | mark << 16
+// (sph_near_q; the mark of a particle of the smaller kernel, else 0): what the
+// one-thread density and energy kernels read of a candidate before its position. Written wherever
+// the current positions are: by the reorder, by the integrate kernel and by launch_make_erec.
 #define SPH_NBL_K 128u
 struct Aux {
   float4 *frec;
   float4 *erec;
+  float *ez = nullptr;
+  uint2 *qpos = nullptr;
   uint *nbl = nullptr;
   uint *nbl_cnt = nullptr;
   uint nbl_stride = 0;
@@ -94,16 +110,18 @@ struct Aux {
   // For n live particles of a scene or of a batch's scenes together. Several lanes per
   // particle shorten the chain of dependent loads and cost more instructions, so density and
   // energy are chosen by whether n threads fill the GPU. Measured (one thread -> several
-  // lanes, us): density 3D-2 25k particles 70 -> 28, 118k 73 -> 63, 206k 80 -> 99; 3D-4 64k
-  // 100 -> 80, 214k 133 -> 222; 2D 17k 19 -> 12, 66k 19 -> 24. Energy 3D-2 25k 88 -> 26, 206k
-  // 100 -> 87, 330k 112 -> 123; 3D-4 64k 174 -> 91, 214k 215 -> 248; 2D 66k 25 -> 17, 264k
-  // 28 -> 42. Force evaluates the same pairs either way, with one pair's registers instead of
+  // lanes, us): density, a falling dam 3D-2 27k 40 -> 32, 43k 44 -> 44, 65k 51 -> 59, 93k 61 -> 78;
+  // a collision 3D-4 27k 44 -> 32, 76k 52 -> 73; the line lies above 65k because sparse scenes
+  // keep several lanes longer (a calm 3D-2 block of 33k to 65k: 14). 2D 20k 14 -> 12, 37k
+  // 15 -> 15. Energy 3D-2 65k 63 -> 53, 93k 78 -> 69, 128k 101 -> 91, 330k 112 -> 123; 3D-4 76k
+  // 108 -> 73, 124k 124 -> 103; 2D 67k 19 -> 16. Force evaluates the same pairs either way, with
+  // one pair's registers instead of
   // four: 3D-2 25k 36 -> 15, 498k 107 -> 91; 3D-4 506k 219 -> 134, 1.7M 501 -> 392, 4.2M
   // shrinking to 2M 732 -> 717; 2D 66k 15 -> 13, 264k 24 -> 30; in a batch, whose lanes each
   // load their scene's parameters, 126k 49 -> 39, 400k 41 -> 52.
   void choose_forms(int variant, bool batch, uint n) {
     const bool d3 = variant != SPH_V2D;
-    fine_density = n <= (d3 ? 100000u : 32000u);
+    fine_density = n <= (d3 ? 66000u : 32000u);
     fine_energy = n <= (d3 ? 180000u : 128000u);
     fine_force = n <= (d3 ? (batch ? 150000u : 6000000u) : 100000u);
   }
@@ -111,6 +129,14 @@ struct Aux {
   uint forms() const {
     return (fine_density ? 1u : 0u) | (fine_force ? 2u : 0u) | (fine_energy ? 4u : 0u);
   }
+};
+
+// where a kernel that writes positions also puts the quantised ones (struct Aux: qpos), if q is
+// given; a batch's steps come from its parameter table
+struct QPosOut {
+  uint2 *q = nullptr;
+  QParams Q = {};
+  const DevParams *Ptab = nullptr;
 };
 
 struct DevState {
@@ -188,21 +214,6 @@ struct BatchView {
 // then mostly in its own XCD's L2. A pure permutation of the work: results do not change.
 // ---------------------------------------------------------------------------------------
 #define SPH_NXCD 8u
-// Wave priority from a neighbour walk's progress (o of NNB cells): 3 in the first quarter
-// down to 0 in the last. The instruction arbiter prefers higher priority, then older waves;
-// waves that are ahead step down, so the waves of a SIMD progress together instead of the
-// youngest running alone at the end. Only the order of issue changes, never a result.
-template <int NNB> __device__ inline void sph_walk_prio(int o) {
-  const int p = 3 - (o * 4) / NNB;
-  if (o > 0 && p == 3 - ((o - 1) * 4) / NNB) return;
-  switch (p) {
-    case 3: __builtin_amdgcn_s_setprio(3); break;
-    case 2: __builtin_amdgcn_s_setprio(2); break;
-    case 1: __builtin_amdgcn_s_setprio(1); break;
-    default: __builtin_amdgcn_s_setprio(0); break;
-  }
-}
-
 __device__ inline uint xcd_block(uint b, uint nb) {
   const uint x = b % SPH_NXCD, k = b / SPH_NXCD;
   const uint q = nb / SPH_NXCD, r = nb % SPH_NXCD;
@@ -309,6 +320,59 @@ __device__ inline void sph_group4(__amdgpu_buffer_rsrc_t r, uint j, float4 q[4])
   }
 }
 
+__device__ inline __amdgpu_buffer_rsrc_t sph_rsrc8(const uint2 *a, uint n) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint2 *>(a), (short)0, (int)(n * 8u), 0x00020000);
+}
+
+// Quantised positions. A candidate's squared distance is first formed in whole steps of 1/q.scale
+// (a power of two; the larger kernel radius is 2048 to 4096 steps): two packed 16-bit subtractions
+// and two dot products instead of eight fp32 operations, from 8 bytes instead of 16. A rounded
+// coordinate is within half a step, so a difference is within one, and a pair whose fp32 distance
+// is below h has a squared step distance below (h q.scale (1 + 1e-5) + 2)^2 = -q.neg (sqrt(3) < 2;
+// 1e-5 covers the rounding of the fp32 distance). Coordinates are kept modulo 2^16 and sums modulo
+// 2^32, so a candidate far away may pass as well: every one that passes is tested in fp32, and none
+// that interacts is lost. Coordinates beyond 2^31 steps saturate.
+// The fourth 16-bit place makes the distance of a pair of the smaller kernel's level count for
+// more, where the pair's reach is the larger of the two radii: with a particle of that level at 0
+// there, a candidate of the same level (at the mark) gains mark^2, the difference of the two
+// thresholds; a particle at mark / 2 sees candidates of both levels alike.
+typedef short sph_short2 __attribute__((ext_vector_type(2)));
+__host__ __device__ inline uint sph_qcoord(float x, float scale) {
+  // NaN and everything below -2^31 become -2^31, what is above the last float below 2^31 that float
+  const float s = __builtin_fminf(__builtin_fmaxf(__builtin_rintf(x * scale), -0x1p31f), 0x1.fffffep30f);
+  return (uint)(int)s & 0xffffu;
+}
+// of a position with its level in w
+__host__ __device__ inline uint2 sph_qpos(float x, float y, float z, uint level, const QParams &Q) {
+  uint2 q;
+  q.x = sph_qcoord(x, Q.scale) | sph_qcoord(y, Q.scale) << 16;
+  q.y = sph_qcoord(z, Q.scale) | ((level == 1u ? 0u : 1u) == Q.mark_level ? Q.mark << 16 : 0u);
+  return q;
+}
+// what a particle of level index L compares its candidates with: reach of a pair max(h_i, h_j)
+// (either) or h of level index L alone
+struct QSelf {
+  uint2 q;
+  int neg;
+};
+__host__ __device__ inline QSelf sph_qself(uint2 q, int L, bool either, const QParams &Q) {
+  const bool marked = either && (uint)L == Q.mark_level;
+  const uint half = marked ? 0u : Q.mark / 2u;
+  QSelf r;
+  r.q = q;
+  r.q.y = (q.y & 0xffffu) | half << 16;
+  const int far = Q.neg[0] < Q.neg[1] ? Q.neg[0] : Q.neg[1];
+  // half^2 less, which every candidate gains
+  r.neg = (either ? far : Q.neg[L]) + (int)(half * half) * -1;
+  return r;
+}
+// negative when the pair may interact
+__device__ inline int sph_near_q(const QSelf &a, uint bx, uint by) {
+  const sph_short2 d = __builtin_bit_cast(sph_short2, a.q.x) - __builtin_bit_cast(sph_short2, bx);
+  const sph_short2 e = __builtin_bit_cast(sph_short2, a.q.y) - __builtin_bit_cast(sph_short2, by);
+  return __builtin_amdgcn_sdot2(d, d, __builtin_amdgcn_sdot2(e, e, a.neg, false), false);
+}
+
 // Correctly rounded sqrtf for finite x >= 2^-96: the hardware estimate, then whichever
 // neighbour one ulp away the two fma residuals select (the correction the compiler's IEEE
 // sqrtf applies; its extra input scaling and zero/infinity fix-ups concern only x below
@@ -403,7 +467,7 @@ void launch_bin_reorder(DevState src, DevState dst, const BinScratch &bs, const 
                         const uint *cend, uint *skeys, uint *svals, uint *s2p, Counters *cnt, uint m,
                         hipStream_t st, bool all_fields, bool set_m = true,
                         const BatchView *bv = nullptr, uint grid = 0, uint *init0 = nullptr,
-                        uint *init1 = nullptr);
+                        uint *init1 = nullptr, QPosOut qo = {});
 void sph_fill_u32(uint *p, uint value, size_t n, hipStream_t st);
 // cstart[0..n) = SPH_EMPTY and cend[0..n) = 0 in one launch
 void sph_fill_cells(uint *cstart, uint *cend, size_t n, hipStream_t st);
@@ -427,7 +491,8 @@ void launch_cell_bounds(const uint *skeys, uint n, uint ncell, uint *cstart, uin
 // all_fields == false: acc, dp and energy are not carried (a step recomputes them)
 void launch_reorder(DevState src, DevState dst, const uint *svals, const uint *slot2phys, uint n,
                     uint *slot2phys_new, hipStream_t st, Counters *set_m = nullptr,
-                    bool all_fields = true, const uint *n_dev = nullptr, uint grid = 0);
+                    bool all_fields = true, const uint *n_dev = nullptr, uint grid = 0,
+                    QPosOut qo = {});
 // The neighbour kernels (density, force, energy) and merge run one thread per particle (or
 // cell, or sorted key) on a grid sized by n, which bounds the device count n_dev if given.
 // density with a.nbl: also the force kernel's pair lists; force with use_nbl: reads them
@@ -435,7 +500,8 @@ void launch_reorder(DevState src, DevState dst, const uint *svals, const uint *s
 void launch_density(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
                     const uint *cend, uint n, hipStream_t st, const BatchView *bv = nullptr,
                     const uint *n_dev = nullptr);
-// Pair-list lengths the force and energy kernels are built with; `cfg` indexes them.
+// Pair-list lengths that a program can set; `cfg` indexes the force kernel's. The energy kernel
+// keeps cells, not pairs, in its lanes' rings and is the same for every energy length.
 constexpr int kForceLists[3] = {24, 32, 48};
 constexpr int kEnergyLists[3] = {16, 24, 32};
 constexpr int kForceListDefault = 1, kEnergyListDefault = 0;
@@ -451,18 +517,17 @@ void launch_force(int variant, const DevParams &P, DevState s, Aux a, const uint
                   const uint *cend, uint n, hipStream_t st, const BatchView *bv = nullptr,
                   int cfg = kForceListDefault, const uint *n_dev = nullptr,
                   bool use_nbl = false);
-// erec (optional): also each particle's energy record (struct Aux)
+// and each particle's energy record and quantised position (a.erec, a.ez, a.qpos)
 void launch_integrate(int variant, const DevParams &P, DevState s, uint n, hipStream_t st,
-                      const BatchView *bv = nullptr, float4 *erec = nullptr,
-                      const uint *n_dev = nullptr, uint grid = 0);
+                      const BatchView *bv, Aux a, const uint *n_dev = nullptr, uint grid = 0);
 // split_bits (optional): also the split decision of each particle (as launch_decide), as bits
 // that were clear before; qbits (optional, not with `fine`): also the merge qualification of the
-// entries as it stands before the split; erec: the energy records of the current positions and velocities (written by the
-// integrate kernel, or by launch_make_erec), read for the neighbours' pair terms
-void launch_energy(int variant, const DevParams &P, DevState s, const uint *cstart,
-                   const uint *cend, uint n, hipStream_t st, const BatchView *bv, int cfg,
-                   uint *split_bits, uint *qbits, const float4 *erec,
-                   const uint *n_dev = nullptr, bool fine = false);
+// entries as it stands before the split; a.erec, a.qpos: the energy records and quantised
+// positions of the current positions and velocities (written by the integrate kernel, or by
+// launch_make_erec)
+void launch_energy(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
+                   const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                   uint *split_bits, uint *qbits, const uint *n_dev = nullptr);
 // the same phases in several lanes per particle (launch_density, launch_force and launch_energy
 // call these as Aux::choose_forms says)
 void launch_density_fine(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
@@ -474,7 +539,7 @@ void launch_force_fine(int variant, const DevParams &P, DevState s, Aux a, const
 void launch_energy_fine(int variant, const DevParams &P, DevState s, const uint *cstart,
                         const uint *cend, uint n, hipStream_t st, const BatchView *bv,
                         uint *split_bits, const float4 *erec, const uint *n_dev);
-void launch_make_erec(DevState s, uint n, float4 *erec, hipStream_t st,
+void launch_make_erec(const DevParams &P, DevState s, uint n, Aux a, hipStream_t st,
                       const uint *n_dev = nullptr);
 void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *split_bits, hipStream_t st);
 // Split of the flagged ones of the cnt->n_pre (at most n) particles (sph_slots.hip). s2p: slot ->

@@ -72,12 +72,15 @@ __global__ __launch_bounds__(BLK) void k_reorder(DevState src, DevState dst,
                                                  const uint *__restrict__ slot2phys,
                                                  const uint *n_dev, uint n_host,
                                                  uint *__restrict__ slot2phys_new,
-                                                 Counters *set_m, bool all) {
+                                                 Counters *set_m, bool all, QPosOut qo) {
   if (set_m && blockIdx.x == 0 && threadIdx.x == 0) set_m->m = set_m->n;
   for_each_item<false>(dev_count(n_dev, n_host), [&](const uint k) {
   const uint s = svals[k];
   const uint q = slot2phys[s];
-  dst.pos[k] = src.pos[q];
+  const float4 p = src.pos[q];
+  dst.pos[k] = p;
+  if (qo.Ptab) put_qpos<true>(qo, k, src.slot[q], p);
+  else put_qpos<false>(qo, k, 0u, p);
   dst.vel[k] = src.vel[q];
   dst.ev[k] = src.ev[q];
   if (all) {
@@ -91,13 +94,140 @@ __global__ __launch_bounds__(BLK) void k_reorder(DevState src, DevState dst,
 }
 
 // ---------------------------------------------------------------------------------------
+// The candidate walk of the density and energy kernels. A particle's 27 cells (2D: nine) hold some
+// 120 to 200 candidates, of which 20 to 40 interact, so most of the work is ruling the others out:
+//   1. Three cells at a time in offset order, every candidate's quantised distance (sph_near_q, six
+//      instructions), eight in flight; the signs are shifted into one 32-bit word per cell. A cell
+//      with a pair goes to the lane's ring in LDS: the word, and its run's end with the offset index.
+//   2. A lane takes the next set bit of its current cell, or the next cell from the ring, and
+//      evaluates that pair in fp32: near(entry), next_cell() before a cell's first. This runs while
+//      some lane's ring has no room for three cells, and at the end.
+// The ring lets lanes with few pairs in one cell go on to the next while others catch up: in a
+// falling dam break (20 pairs) a wave takes 29 rounds of step 2, 41 when rings are emptied after
+// each layer of nine cells and 84 when after each cell; rings of 16 cells take 26 and twice the LDS.
+// From the first cells on of which some lane has a run above 32, step 1 is left out.
+// Bound: VALU issue in the crowded waves, whose chain ends the launch when every wave is resident
+// (dam break), and the L1 misses of the scattered pairs (energy: 2400 lines of 64 bytes per wave).
+// Against a fp32 test of every candidate, us per launch: density 3D-2 500k 133 -> 111, 3D-4 2 to 4M
+// 1105 -> 743, a batch of 3.2M 362 -> 271, of 240k 70 -> 48; energy 176 -> 172, 1700 -> 1114, 492 ->
+// 357, 102 -> 81. One pair per round instead of two: energy 192, 1186, 409 and 83. Emptying the
+// rings after each layer: density 101, 797, 278 and 50, energy 194, 1271, 407 and 88.
+// ---------------------------------------------------------------------------------------
+constexpr int QC = 3;    // cells looked up together
+constexpr uint QR = 8;   // cells of a lane's ring
+
+template <int V, bool TWO, class LOAD, class NEAR, class CELL>
+__device__ inline void walk_near(const DevParams &P, const uint c[3], bool valid, const QSelf &qi,
+                                 const __amdgpu_buffer_rsrc_t qrs, const uint *__restrict__ cstart,
+                                 const uint *__restrict__ cend, uint2 (*sh)[BLK], LOAD &&load,
+                                 NEAR &&near, CELL &&next_cell) {
+  constexpr int NT = VT<V>::nnb / QC;
+  constexpr int QG = TWO ? 8 : 4;  // candidates in flight
+  const uint t = threadIdx.x;
+  const uint nx = P.ncell[0], ny = P.ncell[1], nz = P.ncell[2], nxy = nx * ny;
+  const uint hc = P.cell_base + c[2] * nxy + c[1] * nx + c[0];
+  const bool x0 = c[0] != 0u, x1 = c[0] != nx - 1u, y0 = c[1] != 0u, y1 = c[1] != ny - 1u;
+  const bool z0 = c[2] != 0u, z1 = c[2] != nz - 1u;
+  uint head = 0, tail = 0;  // cells taken from and put into the ring
+  uint m = 0, base = 0;     // the current cell: bits left, entry of bit 0
+  auto take = [&](uint &ent) -> bool {
+    const bool fresh = !m;
+    if (fresh) {
+      const uint2 w = sh[head++ % QR][t];
+      m = w.x;
+      base = w.y;
+    }
+    ent = base + (uint)__builtin_ctz(m);
+    m &= m - 1u;
+    return fresh;
+  };
+  auto step = [&]() {  // up to two pairs, both loaded before the first is evaluated
+    uint e0, e1;
+    const bool f0 = take(e0);
+    const bool two = TWO && (m | (tail ^ head)) != 0u;
+    bool f1 = false;
+    e1 = e0;
+    if (two) f1 = take(e1);
+    const auto d0 = load(e0), d1 = load(e1);
+    if (f0) next_cell();
+    near(e0, d0);
+    if (two) {
+      if (f1) next_cell();
+      near(e1, d1);
+    }
+  };
+  int done = NT;
+#pragma unroll
+  for (int it = 0; it < NT; it++) {
+    // The instruction arbiter prefers higher priority, then older waves: waves that are ahead yield,
+    // so a SIMD's waves progress together instead of the youngest running alone at the end. (The
+    // crowded waves first instead: dam break density 111 -> 115 us.)
+    if (it == 0) __builtin_amdgcn_s_setprio(2);
+    else if (it == NT / 3) __builtin_amdgcn_s_setprio(1);
+    else if (it == 2 * NT / 3) __builtin_amdgcn_s_setprio(0);
+    uint s[QC], e[QC];
+    uint longest = 0;
+#pragma unroll
+    for (int k = 0; k < QC; k++) {
+      const int o = it * QC + k, dx = kDX[o % 9], dy = kDY[o % 9], dz = kDZ[o / 9];
+      s[k] = e[k] = 0u;
+      if (valid && (dx < 0 ? x0 : (dx > 0 ? x1 : true)) && (dy < 0 ? y0 : (dy > 0 ? y1 : true)) &&
+          (dz < 0 ? z0 : (dz > 0 ? z1 : true))) {
+        const uint h = hc + (uint)(dz * (int)nxy + dy * (int)nx + dx);
+        s[k] = cstart[h];
+        e[k] = cend[h];
+      }
+    }
+    if (it > 1)  // (the lookups are in flight)
+      while (__any(tail - head > QR - QC))
+        if (m | (tail ^ head)) step();
+#pragma unroll
+    for (int k = 0; k < QC; k++) {
+      if (s[k] == SPH_EMPTY) s[k] = e[k];
+      longest = max(longest, e[k] - s[k]);
+    }
+    if (__any(longest > 32u)) {
+      done = it;
+      break;
+    }
+#pragma unroll
+    for (int k = 0; k < QC; k++) {
+      uint w = 0;
+      for (uint j = s[k]; j < e[k]; j += QG) {
+#pragma unroll
+        for (int x = 0; x < QG; x += 2) {
+          const auto q = __builtin_amdgcn_raw_buffer_load_b128(qrs, j * 8u + 8u * x, 0, 0);
+          w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[0], q[1]), 31);
+          w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[2], q[3]), 31);
+        }
+      }
+      // the last group's places past the run go; candidate x of c is then bit 32 - c + x
+      w = __builtin_bitreverse32(w >> ((s[k] - e[k]) & (QG - 1)));
+      if (w) sh[tail++ % QR][t] = make_uint2(w, pack_entry(it * QC + k, 0u) + e[k] - 32u);
+    }
+  }
+  while (m | (tail ^ head)) step();
+#pragma unroll 1
+  for (int o = done * QC; o < VT<V>::nnb; o++) {
+    uint s0 = 0, e0 = 0;
+    if (valid) nb_range<V>(P, o, c, cstart, cend, s0, e0);
+    next_cell();
+    for (uint j = s0; j < e0; j++) {
+      const uint ent = pack_entry(o, j);
+      near(ent, load(ent));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // A5 compute_density_kernel + compute_cell_density (SPH-3D-2/sph_system.cu:338-677;
 // 3D-4 :345-684; 2D :268-460). Per-cell partial sums, accumulated in offset order.
 // ---------------------------------------------------------------------------------------
 template <int V, bool B>
-__global__ __launch_bounds__(BLK) void k_density(DevParams P0, const DevParams *__restrict__ Ptab,
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(8))) void k_density(DevParams P0, const DevParams *__restrict__ Ptab,
                                                  const uint *__restrict__ slot,
                                                  const float4 *__restrict__ pos,
+                                                 const uint2 *__restrict__ qpos,
                                                  const float4 *__restrict__ ev,
                                                  float2 *__restrict__ dp,
                                                  float4 *__restrict__ frec,
@@ -107,9 +237,9 @@ __global__ __launch_bounds__(BLK) void k_density(DevParams P0, const DevParams *
                                                  uint *__restrict__ nbl,
                                                  uint *__restrict__ nbl_cnt, uint nbl_stride) {
   constexpr bool D3 = VT<V>::dim == 3;
+  __shared__ uint2 sh[QR][BLK];  // each thread uses its own column only
   uint i;
   if (!one_item(dev_count(n_dev, n_host), i)) return;
-  const __amdgpu_buffer_rsrc_t prs = sph_rsrc(pos, n_host);  // candidates' positions
   const DevParams &P = scene_params<B>(P0, Ptab, B ? slot[i] : 0u);
   const float4 pi = pos[i];
   const int L = lvl_index(pi.w);
@@ -123,103 +253,53 @@ __global__ __launch_bounds__(BLK) void k_density(DevParams P0, const DevParams *
   const float mp0 = P.mass[0] * poly6, mp1 = P.mass[1] * poly6;
   const float self_t = mi * poly6 * k6;
   uint c[3];
-  float total = 0.0f;
   const bool valid = cell_of<V>(P, pi.x, pi.y, pi.z, c);
-  // squared distance to a candidate (from pj - pi: the same float as from pi - pj)
-  auto dist2 = [&](const float4 &pj) {
-    const float dx = pj.x - pi.x, dy = pj.y - pi.y;
-    if (VT<V>::dim == 3) {
-      const float dz = pj.z - pi.z;
-      return dx * dx + dy * dy + dz * dz;
-    }
-    return dx * dx + dy * dy;
-  };
-  // j != i: the term if eps <= r2 < k2; j == i: the self term (j == i has r2 = 0 < eps, or
-  // NaN, so testing r2 first picks the same case); otherwise nothing. Evaluated without a
-  // branch: adding +0 to the cell sum, which starts at +0 and only gains positive terms,
-  // changes no bits.
-  auto term = [&](float &cs, uint j, float r2, bool lj) {
+  // The force kernel's pairs (r2 < max(h_i^2, h_j^2), r2 >= 1e-4; 2D also j == i, its self term)
+  // are collected in visiting order: each shifted into a group of four registers (oldest first),
+  // stored as one 16-byte group when complete; the last, partial group is moved to the front and
+  // stored at the end. 3D sets eps = 1e-4 (the force test's bound), so the tests share their
+  // comparisons.
+  uint4 *const g4 = reinterpret_cast<uint4 *>(nbl) + i;
+  const size_t gs = nbl_stride;
+  const float feps = D3 ? eps : 0.0001f;
+  // r2 < max(h_i^2, h_j^2) for a neighbour of either level: r2 < k2 || r2 < k2j
+  const float fk0 = k2 > P.k2[0] ? k2 : P.k2[0], fk1 = k2 > P.k2[1] ? k2 : P.k2[1];
+  uint4 grp = make_uint4(0u, 0u, 0u, 0u);
+  uint nc = 0;
+  float total = 0.0f, cs = 0.0f;  // finished cells, the current cell
+  const QSelf qi = sph_qself(qpos[i], L, true, P.q);
+  walk_near<V, true>(P, c, valid, qi, sph_rsrc8(qpos, n_host), cstart, cend, sh, [&](uint ent) { return pos[ent & 0x7ffffffu]; },
+               [&](uint ent, const float4 &pj) {
+    const uint j = ent & 0x7ffffffu;
+    // squared distance (from pj - pi: the same float as from pi - pj)
+    const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = D3 ? pj.z - pi.z : 0.0f;
+    const float r2 = D3 ? dx * dx + dy * dy + dz * dz : dx * dx + dy * dy;
+    const bool lj = lvl_index(pj.w);
+    // j != i: the term if eps <= r2 < k2; j == i: the self term (j == i has r2 = 0 < eps, or
+    // NaN, so testing r2 first picks the same case); otherwise nothing. Evaluated without a
+    // branch: adding +0 to the cell sum, which starts at +0 and only gains positive terms,
+    // changes no bits; neither does leaving out a cell without terms.
     const float d = k2 - r2;
     const float tv = (lj ? mp1 : mp0) * ((d * d) * d);
     cs = cs + ((!(r2 < eps) && r2 < k2) ? tv : (j == i ? self_t : 0.0f));
-  };
-  if (!nbl) {
-    if (valid) {
-#pragma unroll
-      for (int o = 0; o < VT<V>::nnb; o++) {
-        uint h;
-        if (!neighbor_cell<V>(P, o, c, h)) continue;
-        float cs = 0.0f;
-        const uint s = cstart[h];
-        if (s != SPH_EMPTY) {
-          const uint e = cend[h];
-          // four loads in flight, then the terms in list order
-          for (uint j = s; j < e; j += 4) {
-            float4 q[4];
-            sph_group4(prs, j, q);
-            term(cs, j, dist2(q[0]), lvl_index(q[0].w));
-            if (j + 1 < e) term(cs, j + 1, dist2(q[1]), lvl_index(q[1].w));
-            if (j + 2 < e) term(cs, j + 2, dist2(q[2]), lvl_index(q[2].w));
-            if (j + 3 < e) term(cs, j + 3, dist2(q[3]), lvl_index(q[3].w));
-          }
-        }
-        total = total + cs;
-      }
+    if ((!D3 && j == i) || (!(r2 < feps) && r2 < (lj ? fk1 : fk0))) {
+      grp = make_uint4(grp.y, grp.z, grp.w, ent);
+      if ((nc & 3u) == 3u && nc < SPH_NBL_K) g4[(nc >> 2) * gs] = grp;
+      nc++;
     }
-  } else {
-    // The same walk, also collecting the force kernel's pairs (r2 < max(h_i^2, h_j^2),
-    // r2 >= 1e-4; 2D also j == i, its self term) in visiting order: each shifted into a
-    // group of four registers (oldest first), stored as one 16-byte group when complete;
-    // the last, partial group is moved to the front and stored at the end. 3D sets
-    // eps = 1e-4 (the force test's bound), so the tests share their comparisons.
-    uint4 *const g4 = reinterpret_cast<uint4 *>(nbl) + i;
-    const size_t gs = nbl_stride;
-    const float feps = D3 ? eps : 0.0001f;
-    // r2 < max(h_i^2, h_j^2) for a neighbour of either level: r2 < k2 || r2 < k2j
-    const float fk0 = k2 > P.k2[0] ? k2 : P.k2[0], fk1 = k2 > P.k2[1] ? k2 : P.k2[1];
-    uint4 grp = make_uint4(0u, 0u, 0u, 0u);
-    uint nc = 0;
-    if (valid) {
-#pragma unroll
-      for (int o = 0; o < VT<V>::nnb; o++) {
-        sph_walk_prio<VT<V>::nnb>(o);
-        uint h;
-        if (!neighbor_cell<V>(P, o, c, h)) continue;
-        float cs = 0.0f;
-        const uint s = cstart[h];
-        if (s != SPH_EMPTY) {
-          const uint e = cend[h];
-          auto cand = [&](uint j, const float4 &pj) {
-            const float r2 = dist2(pj);
-            const bool lj = lvl_index(pj.w);
-            term(cs, j, r2, lj);
-            if ((!D3 && j == i) || (!(r2 < feps) && r2 < (lj ? fk1 : fk0))) {
-              grp = make_uint4(grp.y, grp.z, grp.w, pack_entry(o, j));
-              if ((nc & 3u) == 3u && nc < SPH_NBL_K) g4[(nc >> 2) * gs] = grp;
-              nc++;
-            }
-          };
-          for (uint j = s; j < e; j += 4) {
-            float4 q[4];
-            sph_group4(prs, j, q);
-            cand(j, q[0]);
-            if (j + 1 < e) cand(j + 1, q[1]);
-            if (j + 2 < e) cand(j + 2, q[2]);
-            if (j + 3 < e) cand(j + 3, q[3]);
-          }
-        }
-        total = total + cs;
-      }
-    }
-    const uint r = nc & 3u;  // entries of the partial group, in its last r places
-    if (r && nc < SPH_NBL_K) {
-      const uint4 v = r == 1u ? make_uint4(grp.w, 0u, 0u, 0u)
-                    : r == 2u ? make_uint4(grp.z, grp.w, 0u, 0u)
-                              : make_uint4(grp.y, grp.z, grp.w, 0u);
-      g4[(nc >> 2) * gs] = v;
-    }
-    nbl_cnt[i] = nc;
+  }, [&] {
+    total = total + cs;
+    cs = 0.0f;
+  });
+  total = total + cs;
+  const uint r = nc & 3u;  // entries of the partial group, in its last r places
+  if (r && nc < SPH_NBL_K) {
+    const uint4 v = r == 1u ? make_uint4(grp.w, 0u, 0u, 0u)
+                  : r == 2u ? make_uint4(grp.z, grp.w, 0u, 0u)
+                            : make_uint4(grp.y, grp.z, grp.w, 0u);
+    g4[(nc >> 2) * gs] = v;
   }
+  nbl_cnt[i] = nc;
   const float q = total / P.rest_density;
   const float press = ((q * q) * q - 1.0f) * P.gas_constant;
   dp[i] = make_float2(total, press);
@@ -504,7 +584,9 @@ void k_force(DevParams P0, const DevParams *__restrict__ Ptab,
 template <int V, bool B>
 __global__ __launch_bounds__(BLK) void k_integrate(DevParams P0, const DevParams *__restrict__ Ptab,
                                                    DevState S, const uint *n_dev, uint n_host,
-                                                   float4 *__restrict__ erec) {
+                                                   float4 *__restrict__ erec,
+                                                   float *__restrict__ ez,
+                                                   uint2 *__restrict__ qpos) {
   for_each_item<false>(dev_count(n_dev, n_host), [&](const uint i) {
   const DevParams &P = scene_params<B>(P0, Ptab, B ? S.slot[i] : 0u);
   float4 p = S.pos[i];
@@ -601,6 +683,8 @@ __global__ __launch_bounds__(BLK) void k_integrate(DevParams P0, const DevParams
   S.pos[i] = make_float4(pp[0], pp[1], pp[2], p.w);
   S.vel[i] = make_float4(vv[0], vv[1], vv[2], v.w);
   if (erec) erec[i] = make_float4(pp[0], pp[1], vv[0], vv[1]);
+  if (ez) ez[i] = pp[2];
+  if (qpos) qpos[i] = sph_qpos(pp[0], pp[1], pp[2], __float_as_uint(p.w), P.q);
   S.ev[i] = make_float4(ee[0], ee[1], ee[2], e.w);
   });
 }
@@ -608,19 +692,18 @@ __global__ __launch_bounds__(BLK) void k_integrate(DevParams P0, const DevParams
 // ---------------------------------------------------------------------------------------
 // A9 compute_energy_kernel + compute_cell_energy + wavelet (SPH-3D-2/sph_system.cu:11-16,
 // :1169-1546; 3D-4 :1176-1553; 2D :827-1065). Start-of-step cell lists, current positions.
-// Same two-phase structure as the force kernel; per-cell wavelet sums are flushed when
-// the cell changes. When the kernel length is exactly 1, x/h and x/sqrt(h) equal x, so
+// Per-cell wavelet sums are flushed when the cell changes (walk_near). When the kernel length is exactly 1, x/h and x/sqrt(h) equal x, so
 // those divisions are skipped.
 // ---------------------------------------------------------------------------------------
 // split_bits (optional): the step's split decision (k_decide) is made here too, from the
 // energy just computed, the surface value of the force phase and the level. qbits
 // (optional): and the merge qualification of the entries (k_merge_qual).
-template <int V, bool B, int LIST_E, bool U>
-__global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *__restrict__ Ptab,
+template <int V, bool B, bool U>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(8))) void k_energy(DevParams P0, const DevParams *__restrict__ Ptab,
                                                 SceneCnt *scn,
                                                 const uint *__restrict__ slot,
                                                 const float4 *__restrict__ pos,
-                                                const float4 *__restrict__ vel,
+                                                const uint2 *__restrict__ qpos,
                                                 const float4 *__restrict__ acc,
                                                 float *__restrict__ energy,
                                                 const uint *__restrict__ cstart,
@@ -628,13 +711,13 @@ __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *_
                                                 const uint *n_dev, uint n_host,
                                                 uint *__restrict__ split_bits,
                                                 uint *__restrict__ qbits,
-                                                const float4 *__restrict__ erec) {
+                                                const float4 *__restrict__ erec,
+                                                const float *__restrict__ ez) {
   constexpr bool D3 = VT<V>::dim == 3;
-  __shared__ uint list[LIST_E * BLK];  // each thread uses its own column only
+  __shared__ uint2 sh[QR][BLK];  // each thread uses its own column only
   const uint t = threadIdx.x;
   uint i;
   if (!one_item(dev_count(n_dev, n_host), i)) return;
-  const __amdgpu_buffer_rsrc_t prs = sph_rsrc(pos, n_host);  // candidates' positions
   const DevParams &P = scene_params<B>(P0, Ptab, B ? slot[i] : 0u);
   const float4 pi = pos[i];
   const int Li = lvl_index(pi.w);
@@ -648,106 +731,47 @@ __global__ __launch_bounds__(BLK) void k_energy(DevParams P0, const DevParams *_
   const bool unit = U || (ker == 1.0f && sk == 1.0f);
   float ttx = 0.0f, tty = 0.0f, tvx = 0.0f, tvy = 0.0f;
   float ctx = 0.0f, cty = 0.0f;
-  int cur_o = -1;
   uint c[3];
   const bool valid = cell_of<V>(P, pi.x, pi.y, pi.z, c);
-  uint cnt = 0;
+  const QSelf qi = sph_qself(qpos[i], Lk, false, P.q);
   struct Nb {
-    int eo;
-    float4 pj, vj;
+    float4 e;  // pos.xy, vel.xy
+    float z;
   };
-  auto fetch_ent = [&](uint ent) {
-    Nb f;
-    f.eo = (int)(ent >> 27);
+  // a batch's general form would spill with two pairs loaded
+  walk_near<V, !B || U>(P, c, valid, qi, sph_rsrc8(qpos, n_host), cstart, cend, sh, [&](uint ent) {
     const uint j = ent & 0x7ffffffu;
-    const float4 r = erec[j];  // one 16-byte record: pos.xy, vel.xy
-    f.pj = make_float4(r.x, r.y, 0.0f, 0.0f);
-    f.vj = make_float4(r.z, r.w, 0.0f, 0.0f);
-    return f;
-  };
-  auto body = [&](const Nb &f) {
-    if (f.eo != cur_o) {
-      ttx = ttx + ctx;
-      tty = tty + cty;
-      ctx = cty = 0.0f;
-      cur_o = f.eo;
-    }
-    const float ax = pi.x - f.pj.x, ay = pi.y - f.pj.y;
+    return Nb{erec[j], D3 ? ez[j] : 0.0f};
+  }, [&](uint ent, const Nb &nb) {
+    const uint j = ent & 0x7ffffffu;
+    const float4 ej = nb.e;
+    const float zj = nb.z;
+    const float ax = pi.x - ej.x, ay = pi.y - ej.y, az = D3 ? pi.z - zj : 0.0f;
+    const float r2 = D3 ? ax * ax + ay * ay + az * az : ax * ax + ay * ay;
+    // 3D skips r2 < 1e-4 (so j == i); 2D clamps r2 to EXT2 and never uses it again.
+    if (!(r2 < ker2) || (D3 ? r2 < 0.0001f : j == i)) return;
     // the z component of the transform never reaches the energy (3D-2 :1521)
     if (unit) {
       // |ax|, |ay| <= h = 1 here, so the exp argument is within [-0.125, 0]
       const float tx = sph_wavelet_unit(ax), ty = sph_wavelet_unit(ay);
       ctx = ctx + tx;
       cty = cty + ty;
-      tvx = tvx + (f.vj.x * tx);
-      tvy = tvy + (f.vj.y * ty);
+      tvx = tvx + (ej.z * tx);
+      tvy = tvy + (ej.w * ty);
     } else {
       // ax / ker, ay / ker, (vx * tx) / sk, (vy * ty) / sk, each correctly rounded
       auto dv = [&](float a, float b, float y) { return div_fast ? sph_div_rn(a, b, y) : a / b; };
       const float tx = sph_wavelet_unit(dv(ax, ker, rker)), ty = sph_wavelet_unit(dv(ay, ker, rker));
       ctx = ctx + tx;
       cty = cty + ty;
-      tvx = tvx + dv(f.vj.x * tx, sk, rsk);
-      tvy = tvy + dv(f.vj.y * ty, sk, rsk);
+      tvx = tvx + dv(ej.z * tx, sk, rsk);
+      tvy = tvy + dv(ej.w * ty, sk, rsk);
     }
-  };
-  // The LDS list as a ring per lane (entries head .. head + cnt - 1, mod LIST_E). The
-  // candidate groups advance together over the wave (the same cell, group k of every
-  // lane's run); whenever some lane has fewer than four free places, every lane with
-  // entries evaluates its oldest two (one, if it has one) -- so a lane's pairs are
-  // evaluated in visiting order, mostly while other lanes' lists fill up, and a body row
-  // is spent only when some lane needs the room.
-  uint head = 0;
-  auto ring = [&](uint x) {
-    const uint p = head + x;
-    if constexpr ((LIST_E & (LIST_E - 1)) == 0) return p & (uint)(LIST_E - 1);
-    else return p >= (uint)LIST_E ? p - (uint)LIST_E : p;
-  };
-  auto pop2 = [&]() {
-    const bool h0 = cnt > 0u, h1 = cnt > 1u;
-    Nb f0, f1;
-    if (h0) f0 = fetch_ent(list[ring(0) * BLK + t]);
-    if (h1) f1 = fetch_ent(list[ring(1) * BLK + t]);
-    if (h0) body(f0);
-    if (h1) body(f1);
-    const uint k = h1 ? 2u : (h0 ? 1u : 0u);
-    head = ring(k);
-    cnt -= k;
-  };
-  for (int o = 0; o < VT<V>::nnb; o++) {
-    sph_walk_prio<VT<V>::nnb>(o);
-    uint s0 = 0, e0 = 0;
-    if (valid) nb_range<V>(P, o, c, cstart, cend, s0, e0);
-    auto cand = [&](uint j, const float4 &pj) {
-      if (!D3 && j == i) return;  // 3D: r2 = 0 fails the r2 >= 1e-4 test below
-      const float rx = pi.x - pj.x, ry = pi.y - pj.y;
-      const float rz = D3 ? pi.z - pj.z : 0.0f;
-      const float r2 = D3 ? rx * rx + ry * ry + rz * rz : rx * rx + ry * ry;
-      // 3D skips r2 < 1e-4; 2D clamps r2 to EXT2 and never uses it again.
-      if (r2 < ker2 && !(D3 && r2 < 0.0001f)) {
-        list[ring(cnt) * BLK + t] = pack_entry(o, j);
-        cnt++;
-      }
-    };
-    for (;; s0 += 4) {
-      // the group's loads are issued first, so they are in flight during the rows below
-      float4 q[4];
-      if (s0 < e0) sph_group4(prs, s0, q);
-      // every lane had room for four before the last group, so two rows restore it
-      if (__any(cnt + 4u > (uint)LIST_E)) {
-        pop2();
-        if (__any(cnt + 4u > (uint)LIST_E)) pop2();
-      }
-      if (!__any(s0 < e0)) break;
-      if (s0 < e0) {
-        cand(s0, q[0]);
-        if (s0 + 1 < e0) cand(s0 + 1, q[1]);
-        if (s0 + 2 < e0) cand(s0 + 2, q[2]);
-        if (s0 + 3 < e0) cand(s0 + 3, q[3]);
-      }
-    }
-  }
-  while (__any(cnt > 0u)) pop2();
+  }, [&] {
+    ttx = ttx + ctx;
+    tty = tty + cty;
+    ctx = cty = 0.0f;
+  });
   ttx = ttx + ctx;
   tty = tty + cty;
   const float ux = tvx / ttx, uy = tvy / tty;
@@ -1681,13 +1705,13 @@ void launch_cell_bounds(const uint *skeys, uint n, uint ncell, uint *cstart, uin
 
 void launch_reorder(DevState src, DevState dst, const uint *svals, const uint *slot2phys, uint n,
                     uint *slot2phys_new, hipStream_t st, Counters *set_m, bool all_fields,
-                    const uint *n_dev, uint grid) {
+                    const uint *n_dev, uint grid, QPosOut qo) {
   if (n == 0) {
     if (set_m) hipLaunchKernelGGL(k_set_phys_count, dim3(1), dim3(1), 0, st, set_m);
     return;
   }
   hipLaunchKernelGGL(k_reorder, grid_or(grid, n), dim3(BLK), 0, st, src, dst, svals, slot2phys,
-                     n_dev, n, slot2phys_new, set_m, all_fields);
+                     n_dev, n, slot2phys_new, set_m, all_fields, qo);
 }
 
 void launch_density(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
@@ -1696,7 +1720,7 @@ void launch_density(int variant, const DevParams &P, DevState s, Aux a, const ui
   if (n == 0) return;
   if (a.fine_density) return launch_density_fine(variant, P, s, a, cstart, cend, n, st, bv, n_dev);
   SPH_DISPATCH_VB(variant, bv != nullptr, k_density, grid_for(n), dim3(BLK), 0, st, P,
-                  ptab_of(bv), s.slot, s.pos, s.ev, s.dp, a.frec, cstart, cend, n_dev, n, a.nbl,
+                  ptab_of(bv), s.slot, s.pos, a.qpos, s.ev, s.dp, a.frec, cstart, cend, n_dev, n, a.nbl,
                   a.nbl_cnt, a.nbl_stride);
 }
 
@@ -1722,20 +1746,20 @@ void launch_force(int variant, const DevParams &P, DevState s, Aux a, const uint
 }
 
 void launch_integrate(int variant, const DevParams &P, DevState s, uint n, hipStream_t st,
-                      const BatchView *bv, float4 *erec, const uint *n_dev, uint grid) {
+                      const BatchView *bv, Aux a, const uint *n_dev, uint grid) {
   if (n == 0) return;
   SPH_DISPATCH_VB(variant, bv != nullptr, k_integrate, grid_or(grid, n), dim3(BLK), 0, st, P,
-                  ptab_of(bv), s, n_dev, n, erec);
+                  ptab_of(bv), s, n_dev, n, a.erec, a.ez, a.qpos);
 }
 
-template <int L, bool U>
-static void launch_energy_lu(int variant, const DevParams &P, DevState s, const uint *cstart,
-                             const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                             uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev) {
+template <bool U>
+static void launch_energy_u(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
+                            const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                            uint *split_bits, uint *qbits, const uint *n_dev) {
 #define SPH_EN(VV, BB)                                                                       \
-  k_energy<VV, BB, L, U><<<grid_for(n), dim3(BLK), 0, st>>>(                                 \
-      P, ptab_of(bv), scn_of(bv), s.slot, s.pos, s.vel, s.acc, s.energy, cstart, cend, n_dev, \
-      n, split_bits, qbits, erec)
+  k_energy<VV, BB, U><<<grid_for(n), dim3(BLK), 0, st>>>(                                    \
+      P, ptab_of(bv), scn_of(bv), s.slot, s.pos, a.qpos, s.acc, s.energy, cstart, cend, n_dev, \
+      n, split_bits, qbits, a.erec, a.ez)
   if (bv) {
     if (variant == SPH_V3D2) SPH_EN(SPH_V3D2, true);
     else if (variant == SPH_V3D4) SPH_EN(SPH_V3D4, true);
@@ -1747,46 +1771,38 @@ static void launch_energy_lu(int variant, const DevParams &P, DevState s, const 
 #undef SPH_EN
 }
 
-template <int L>
-static void launch_energy_l(int variant, const DevParams &P, DevState s, const uint *cstart,
-                            const uint *cend, uint n, hipStream_t st, const BatchView *bv,
-                            uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev) {
-  if (P.energy_unit)
-    launch_energy_lu<L, true>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
-  else
-    launch_energy_lu<L, false>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
-}
-
-// erec (pos.x, pos.y, vel.x, vel.y) from the state, for an energy pass that does not follow
-// the integrate kernel (which writes the same records)
-__global__ __launch_bounds__(BLK) void k_make_erec(const float4 *__restrict__ pos,
+// erec (pos.x, pos.y, vel.x, vel.y) and qpos from a single scene's state, for a density or energy
+// pass that does not follow the kernels that write the same (reorder and integrate)
+__global__ __launch_bounds__(BLK) void k_make_erec(QParams Q, const float4 *__restrict__ pos,
                                                    const float4 *__restrict__ vel,
                                                    const uint *n_dev, uint n_host,
-                                                   float4 *__restrict__ erec) {
+                                                   float4 *__restrict__ erec,
+                                                   float *__restrict__ ez,
+                                                   uint2 *__restrict__ qpos) {
   for_each_item<false>(dev_count(n_dev, n_host), [&](const uint i) {
     const float4 p = pos[i], v = vel[i];
     erec[i] = make_float4(p.x, p.y, v.x, v.y);
+    ez[i] = p.z;
+    qpos[i] = sph_qpos(p.x, p.y, p.z, __float_as_uint(p.w), Q);
   });
 }
 
-void launch_make_erec(DevState s, uint n, float4 *erec, hipStream_t st, const uint *n_dev) {
+void launch_make_erec(const DevParams &P, DevState s, uint n, Aux a, hipStream_t st, const uint *n_dev) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_make_erec, grid_for(n), dim3(BLK), 0, st, s.pos, s.vel, n_dev, n, erec);
+  hipLaunchKernelGGL(k_make_erec, grid_for(n), dim3(BLK), 0, st, P.q, s.pos, s.vel, n_dev, n, a.erec,
+                     a.ez, a.qpos);
 }
 
-void launch_energy(int variant, const DevParams &P, DevState s, const uint *cstart,
-                   const uint *cend, uint n, hipStream_t st, const BatchView *bv, int cfg,
-                   uint *split_bits, uint *qbits, const float4 *erec, const uint *n_dev, bool fine) {
+void launch_energy(int variant, const DevParams &P, DevState s, Aux a, const uint *cstart,
+                   const uint *cend, uint n, hipStream_t st, const BatchView *bv,
+                   uint *split_bits, uint *qbits, const uint *n_dev) {
   if (n == 0) return;
-  if (fine)
-    return launch_energy_fine(variant, P, s, cstart, cend, n, st, bv, split_bits, erec, n_dev);
-  static_assert(kEnergyLists[0] == 16 && kEnergyLists[1] == 24 && kEnergyLists[2] == 32, "energy lists");
-  if (cfg == 1)
-    launch_energy_l<24>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
-  else if (cfg == 2)
-    launch_energy_l<32>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
+  if (a.fine_energy)
+    launch_energy_fine(variant, P, s, cstart, cend, n, st, bv, split_bits, a.erec, n_dev);
+  else if (P.energy_unit)
+    launch_energy_u<true>(variant, P, s, a, cstart, cend, n, st, bv, split_bits, qbits, n_dev);
   else
-    launch_energy_l<16>(variant, P, s, cstart, cend, n, st, bv, split_bits, qbits, erec, n_dev);
+    launch_energy_u<false>(variant, P, s, a, cstart, cend, n, st, bv, split_bits, qbits, n_dev);
 }
 
 void launch_decide(int variant, const DevParams &P, DevState s, uint n, uint *split_bits, hipStream_t st) {
