@@ -1079,12 +1079,11 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
   }
   const size_t cap = a->cap;
   const size_t nth = (size_t)std::max(a->nf, 2) * std::max(a->nf, 2) * std::max(a->nf, 2) * 3;
-  const size_t scan_n = std::max<size_t>(cap, sph_sort_hist_elems(cap));
   const size_t iblocks = (cap + IBLK - 1) / IBLK;
   bool ok = a->alloc_state(a->cur) && a->alloc_state(a->scratch) && a->alloc_state(a->state0) &&
             a->alloc(a->keys, cap) && a->alloc(a->vals, cap) && a->alloc(a->sc.keys_alt, cap) &&
             a->alloc(a->sc.vals_alt, cap) && a->alloc(a->sc.tile_hist, sph_sort_hist_elems(cap)) &&
-            a->alloc(a->sc.len_dev, 1) && a->alloc(a->scan_tmp, sph_scan_tmp_elems(scan_n)) &&
+            a->alloc(a->scan_tmp, sph_scan_tmp_elems(cap)) &&
             a->alloc(a->s2p_hash, cap) && a->alloc(a->s2p_cell, cap) &&
             a->alloc(a->cs_scr, a->cells) && a->alloc(a->ce_scr, a->cells) &&
             a->alloc(a->sb.split, sph_bit_words(cap)) && a->alloc(a->sb.dead, sph_bit_words(cap)) &&
@@ -1102,8 +1101,7 @@ int sph_adj_create(const void *sysparam, uint32_t n, uint32_t field_nodes, uint3
             a->alloc(a->aos_dev, cap * sizeof(SphParticle3D));
   a->aux.nbl_stride = (uint)cap;
   a->aux.choose_forms(SPH_V3D2, false, flags & SPH_STEP_SPLIT ? 2 * n : n);
-  a->sc.scan_tmp = a->sb.scan_tmp = a->scan_tmp;
-  a->sc.max_tiles = sph_sort_tiles(cap);
+  a->sb.scan_tmp = a->scan_tmp;
   if (ok && sph_use_bins(a->cells, cap)) {
     a->bins.hkey = a->keys;
     a->bins.rank = a->vals;

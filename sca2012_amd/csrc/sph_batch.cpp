@@ -628,7 +628,6 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
     return SPH_EHIP;
   }
   const size_t cap = b->phys_cap;
-  const size_t scan_n = std::max<size_t>(cap, sph_sort_hist_elems(cap));
   bool ok = b->alloc_state(b->cur) && b->alloc_state(b->alt) && b->alloc(b->keys, cap) &&
             b->alloc(b->vals, cap) && b->alloc(b->sc.keys_alt, cap) && b->alloc(b->sc.vals_alt, cap) &&
             b->alloc(b->sc.tile_hist, sph_sort_hist_elems(cap)) &&
@@ -640,9 +639,9 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
             b->alloc(b->Ptab, n_scenes) && b->alloc(b->aos_dev, (size_t)b->max_cap * b->rec) &&
             b->alloc(b->aux.frec, 3 * cap) && b->alloc(b->aux.erec, cap) && b->alloc(b->aux.ez, cap) && b->alloc(b->aux.qpos, cap) &&
             b->alloc(b->aux.nbl, (size_t)SPH_NBL_K * cap) && b->alloc(b->aux.nbl_cnt, cap) &&
-            b->alloc(b->scan_tmp, sph_scan_tmp_elems(scan_n)) && b->alloc(b->sc.len_dev, 1);
+            b->alloc(b->scan_tmp, sph_scan_tmp_elems(cap));
   b->aux.nbl_stride = (uint)cap;
-  b->sc.scan_tmp = b->sb.scan_tmp = b->scan_tmp;
+  b->sb.scan_tmp = b->scan_tmp;
   if (ok && sph_use_bins(b->total_cell, cap)) {
     b->bins.hkey = b->keys;
     b->bins.rank = b->vals;
@@ -650,7 +649,6 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
     ok = b->alloc(b->bins.ccount, b->total_cell) && b->alloc(b->bins.tmp, sph_bin_tiles(b->total_cell));
     if (ok) sph_fill_u32(b->bins.ccount, 0u, b->total_cell, b->st);
   }
-  b->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && hipHostMalloc((void **)&b->cnt_host, sizeof(Counters), hipHostMallocDefault) != hipSuccess)
     ok = false;
   if (ok && hipHostMalloc((void **)&b->scn_host, sizeof(SceneCnt) * n_scenes,

@@ -859,7 +859,6 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
     return SPH_EHIP;
   }
   const size_t cap = capacity;
-  const size_t scan_n = std::max<size_t>(cap, sph_sort_hist_elems(cap));
   bool ok = c->alloc_state(c->cur) && c->alloc_state(c->alt) && c->alloc(c->keys, cap) &&
             c->alloc(c->vals, cap) && c->alloc(c->sc.keys_alt, cap) && c->alloc(c->sc.vals_alt, cap) &&
             c->alloc(c->sc.tile_hist, sph_sort_hist_elems(cap)) &&
@@ -881,9 +880,9 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
          c->alloc(c->tris, (size_t)std::max<uint32_t>(max_triangles, 1) * 18);
     if (ok) ok = c->alloc(c->occ, 2 * sph_occ_words(c->P.total_cell));
   }
-  size_t scan_elems = sph_scan_tmp_elems(std::max(scan_n, c->ncube));
+  size_t scan_elems = sph_scan_tmp_elems(std::max(cap, c->ncube));
   ok = ok && c->alloc(c->scan_tmp, scan_elems);
-  c->sc.scan_tmp = c->sb.scan_tmp = c->scan_tmp;
+  c->sb.scan_tmp = c->scan_tmp;
   if (ok && sph_use_bins(c->P.total_cell, cap)) {
     c->bins.hkey = c->keys;
     c->bins.rank = c->vals;
@@ -892,7 +891,6 @@ int sph_ctx_create(int variant, const void *sysparam, uint32_t capacity, uint32_
          c->alloc(c->bins.tmp, sph_bin_tiles(c->P.total_cell));
     if (ok) sph_fill_u32(c->bins.ccount, 0u, c->P.total_cell, c->st);
   }
-  c->sc.max_tiles = sph_sort_tiles(cap);
   if (ok && (hipHostMalloc((void **)&c->rep, sizeof(Report), hipHostMallocDefault) != hipSuccess ||
              hipHostGetDevicePointer((void **)&c->rep_dev, c->rep, 0) != hipSuccess))
     ok = false;

@@ -404,22 +404,18 @@ __host__ __device__ inline float sph_wavelet(float x) {
 // ---------------------------------------------------------------------------------------
 struct SortScratch {
   uint *keys_alt, *vals_alt;  // ping-pong partners
-  uint *tile_hist;            // RADIX * max_tiles
-  uint *scan_tmp;             // block sums for the scan
-  size_t max_tiles;
-  uint *len_dev;              // one device word: histogram length of a sort by device count
+  uint *tile_hist;            // sph_sort_hist_elems(n)
 };
 
 size_t sph_scan_tmp_elems(size_t n);
-size_t sph_sort_tiles(size_t n);
-size_t sph_sort_hist_elems(size_t n);  // tile histogram entries for a sort of n keys
+size_t sph_sort_hist_elems(size_t n);  // histogram entries for a sort of n keys
 
 // Exclusive scan of in[0..*n_dev) (host upper bound n_max) into out; total -> *total_dev.
 void sph_exclusive_scan(const uint *in, uint *out, const uint *n_dev, uint n_max, uint *total_dev,
                         uint *tmp, hipStream_t st);
 // Stable LSD radix sort of keys[0..n) (values = slot index 0..n-1, generated) by the low
 // `bits` bits. Result (keys, vals) ends in (*keys_out, *vals_out), which point into
-// {keys, vals} or {sc.keys_alt, sc.vals_alt}. n_dev (optional, needs sc.len_dev): the key
+// {keys, vals} or {sc.keys_alt, sc.vals_alt}. n_dev (optional): the key
 // count in device memory, n bounding it; grid (optional): persistent histogram and scatter
 // launches of that many workgroups.
 void sph_radix_sort(uint *keys, uint *vals, uint n, int bits, SortScratch &sc, uint **keys_out,

@@ -4,9 +4,10 @@
 //     adds the sums of the tiles before it, which it reads itself when there are at most
 //     1024 tiles and otherwise takes from a single-block scan of the sums);
 //   * stable LSD radix sort of (cell hash, slot) with digits of up to 9 bits (an 18-bit key,
-//     64^3 cells, takes two passes); each pass is a per-tile LDS histogram, a scan of the
-//     digit-major tile histograms, and a scatter whose stable in-tile rank comes from
-//     64-lane ballot matching plus per-wave digit counts in LDS.
+//     64^3 cells, takes two passes). A pass is two launches: LDS histograms per tile and per
+//     group of tiles, and a scatter whose stable in-tile rank comes from 64-lane ballot matching
+//     and per-wave digit counts in LDS, and which adds up the groups before its own; above 128
+//     groups a third launch between them does that.
 // All integer work, no floating point, results independent of scheduling.
 #include <mutex>
 
@@ -20,11 +21,15 @@ constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;  // 2048
 constexpr uint SCAN_FUSED_TILES = 4 * SCAN_THREADS;     // two-kernel scan up to 1024 tiles
 
 constexpr int RADIX_BITS = 9;           // widest digit
-constexpr int RADIX = 1 << RADIX_BITS;  // 512 bins, two per thread
-constexpr int SORT_THREADS = 256;
-constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ITEMS = 4;
-constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;  // 1024 keys per tile (more tiles fill the GPU)
+constexpr int RADIX = 1 << RADIX_BITS;  // 512 bins
+constexpr int SORT_ITEMS = 4;        // keys of a thread
+constexpr int GROUP_TILES = 4;
+constexpr int SORT_TILE_MIN = 256 * SORT_ITEMS;
+constexpr uint BASE_GROUPS = 128;    // more groups are added up by a launch of their own
+
+// Waves of a tile for n keys: enough workgroups for the GPU, and few enough groups for a workgroup to
+// add up. Beyond 1M keys the groups have their own launch and a tile is 4096 keys, eight of a digit.
+inline int sort_waves(size_t n) { return n <= 131072 ? 4 : (n <= 1048576 ? 8 : 16); }
 
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const uint *__restrict__ in,
                                                               const uint *n_dev, uint n_host,
@@ -139,93 +144,219 @@ __device__ inline uint sort_count(const uint *n_dev, uint n_host) {
   return n_dev ? min(*n_dev, n_host) : n_host;
 }
 
-// Per-tile digit histogram, stored digit-major: hist[d * ntiles + tile], d < 2^width,
-// ntiles = ceil(n / SORT_TILE). Workgroup b takes tiles b, b + gridDim.x, ... (one tile each
-// in a plain launch). scan_len (optional): receives the histogram's length, 2^width * ntiles.
-__global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint *__restrict__ keys,
+// Bins of a digit: whole 16-byte groups (the first pass over one bit has two that stay empty).
+__device__ __host__ inline uint radix_bins(int width) { return width < 2 ? 4u : 1u << width; }
+
+// Histograms of a pass: workgroup b takes groups b, b + gridDim.x, ... of GROUP_TILES tiles.
+// pre[tile * bins + d]: keys of digit d in the group's tiles before this one; gsum[group *
+// bins + d]: in the whole group.
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_radix_hist(const uint *__restrict__ keys,
                                                              const uint *n_dev, uint n_host,
                                                              int shift, int width,
-                                                             uint *__restrict__ hist,
-                                                             uint *scan_len) {
-  __shared__ uint h[RADIX];
-  const int t = threadIdx.x;
-  const int nbin = 1 << width;
-  const uint mask = (uint)nbin - 1u;
+                                                             uint *__restrict__ pre,
+                                                             uint *__restrict__ gsum) {
+  constexpr uint SORT_THREADS = 64 * W, SORT_TILE = SORT_THREADS * SORT_ITEMS;
+  constexpr int PER_WAVE = GROUP_TILES * SORT_TILE / W;  // keys of a wave
+  constexpr int TILE_WAVES = W / GROUP_TILES;
+  __shared__ uint h[GROUP_TILES][RADIX];
+  const uint t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  const uint nbin = radix_bins(width), mask = (1u << width) - 1u;
   const uint n = sort_count(n_dev, n_host);
   const uint ntiles = (n + SORT_TILE - 1) / SORT_TILE;
-  if (scan_len && blockIdx.x == 0 && t == 0) *scan_len = (uint)nbin * ntiles;
-  for (uint tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    for (int d = t; d < nbin; d += SORT_THREADS) h[d] = 0;
+  const uint ngroups = (ntiles + GROUP_TILES - 1) / GROUP_TILES;
+  for (uint g = blockIdx.x; g < ngroups; g += gridDim.x) {
+    for (uint x = t; x < GROUP_TILES * RADIX; x += SORT_THREADS) (&h[0][0])[x] = 0u;
     __syncthreads();
-    const size_t base = (size_t)tile * SORT_TILE;
-#pragma unroll 4
-    for (int j = 0; j < SORT_ITEMS; j++) {
-      size_t i = base + (size_t)j * SORT_THREADS + t;
-      if (i < n) atomicAdd(&h[(keys[i] >> shift) & mask], 1u);
+    const size_t base = (size_t)g * GROUP_TILES * SORT_TILE + w * PER_WAVE + lane;
+    uint *const hw = h[w / TILE_WAVES];
+#pragma unroll
+    for (int j = 0; j < PER_WAVE / 64; j++) {
+      const size_t i = base + 64 * j;
+      if (i < n) atomicAdd(&hw[(keys[i] >> shift) & mask], 1u);
     }
     __syncthreads();
-    for (int d = t; d < nbin; d += SORT_THREADS) hist[(size_t)d * ntiles + tile] = h[d];
-    __syncthreads();  // h is cleared for the next tile
+    for (uint d = t; d < nbin; d += SORT_THREADS) {
+      uint a = 0;
+#pragma unroll
+      for (int k = 0; k < GROUP_TILES; k++) {
+        const uint tile = g * GROUP_TILES + k;
+        if (tile < ntiles) pre[(size_t)tile * nbin + d] = a;
+        a += h[k][d];
+      }
+      gsum[(size_t)g * nbin + d] = a;
+    }
+    __syncthreads();  // h is cleared for the next group
   }
 }
 
-// Stable scatter. Items of a tile are taken in index order (round j, then thread t); the
-// rank of an item among equal digits = digits seen in earlier rounds of this tile (run)
-// + equal digits in earlier waves of this round (wcnt) + equal digits in lower lanes of
-// its own wave (ballot match).
-__global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(
+// gsum[group][d] becomes the sum over the groups before, total[d] the sum over all. A workgroup
+// takes BASE_DIGITS digits; a thread sums a run of groups, the runs are scanned in LDS.
+constexpr int BASE_THREADS = 1024, BASE_DIGITS = 32, BASE_ROWS = BASE_THREADS / BASE_DIGITS;
+__global__ __launch_bounds__(BASE_THREADS) void k_radix_base(const uint *n_dev, uint n_host, int width,
+                                                             uint group_keys,
+                                                             uint *__restrict__ gsum,
+                                                             uint *__restrict__ total) {
+  __shared__ uint s[BASE_ROWS][BASE_DIGITS];
+  const uint nbin = radix_bins(width);
+  const uint n = sort_count(n_dev, n_host);
+  const uint ngroups = (n + group_keys - 1) / group_keys;
+  const uint x = threadIdx.x % BASE_DIGITS, r = threadIdx.x / BASE_DIGITS;
+  const uint d = blockIdx.x * BASE_DIGITS + x;
+  const uint len = (ngroups + BASE_ROWS - 1) / BASE_ROWS, g0 = min(r * len, ngroups), g1 = min(g0 + len, ngroups);
+  uint sum = 0;
+  if (d < nbin)
+    for (uint g = g0; g < g1; g++) sum += gsum[(size_t)g * nbin + d];
+  s[r][x] = sum;
+  __syncthreads();
+  uint run = 0, all = 0;
+  for (uint k = 0; k < BASE_ROWS; k++) {
+    run += k < r ? s[k][x] : 0u;
+    all += s[k][x];
+  }
+  if (d >= nbin) return;
+  for (uint g = g0; g < g1; g++) {
+    const uint v = gsum[(size_t)g * nbin + d];
+    gsum[(size_t)g * nbin + d] = run;
+    run += v;
+  }
+  if (r == 0) total[d] = all;
+}
+
+// Stable scatter. A wave takes SORT_ITEMS rounds of 64 consecutive keys and counts its digits in
+// its own row of LDS, so no round needs a block barrier: the rank of a key among equal digits is
+// the row's count from earlier rounds plus the equal digits in lower lanes (ballot match). Then
+// each digit's row counts become places: the smaller digits of all keys, this digit's of the
+// groups before (both from k_radix_base, or added up here when total is null), of the group's
+// tiles before and of the tile's waves before. The tile is put in order in LDS first, so that its
+// stores go out in runs of a digit (700k keys, a digit of 9 bits: 22.6 -> 17.5 us). Bound: the
+// scattered stores and, up to some 100k keys, the chain of loads. Against a digit-major histogram,
+// its scan in two launches and a scatter with three barriers per round, us per call of
+// sph_sort_noalloc: 700k keys of 27 bits 110 -> 77, 1M 145 -> 91, 100k 60 -> 56, 1000 40 -> 35;
+// 700k of 18 bits 71 -> 49, of 32 bits 110 -> 80.
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_radix_scatter(
     const uint *__restrict__ keys_in, const uint *__restrict__ vals_in, const uint *n_dev,
-    uint n_host, int shift, int width, const uint *__restrict__ offs,
-    uint *__restrict__ keys_out, uint *__restrict__ vals_out) {
-  __shared__ uint run[RADIX];
-  __shared__ uint wcnt[SORT_WAVES][RADIX];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int nbin = 1 << width;
-  const uint mask = (uint)nbin - 1u;
+    uint n_host, int shift, int width, const uint *__restrict__ pre, const uint *__restrict__ gsum,
+    const uint *__restrict__ total, uint *__restrict__ keys_out, uint *__restrict__ vals_out) {
+  constexpr uint SORT_THREADS = 64 * W, SORT_TILE = SORT_THREADS * SORT_ITEMS;
+  constexpr uint DP = RADIX > SORT_THREADS ? RADIX / SORT_THREADS : 1;  // a thread's digits
+  __shared__ uint cnt[W][RADIX];
+  __shared__ uint all[RADIX], before[RADIX];
+  __shared__ uint skey[SORT_TILE], sval[SORT_TILE];
+  __shared__ uint lw[W];
+  const uint t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  const uint nbin = radix_bins(width), mask = (1u << width) - 1u;
   const uint n = sort_count(n_dev, n_host);
   const uint ntiles = (n + SORT_TILE - 1) / SORT_TILE;
-  for (uint tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-  for (int d = t; d < nbin; d += SORT_THREADS) {
-    run[d] = offs[(size_t)d * ntiles + tile];
-#pragma unroll
-    for (int k = 0; k < SORT_WAVES; k++) wcnt[k][d] = 0;
-  }
-  __syncthreads();
-  const size_t base = (size_t)tile * SORT_TILE;
+  const uint ngroups = (ntiles + GROUP_TILES - 1) / GROUP_TILES;
   const unsigned long long lt = (1ull << lane) - 1ull;
-  for (int j = 0; j < SORT_ITEMS; j++) {
-    const size_t i = base + (size_t)j * SORT_THREADS + t;
-    const bool valid = i < n;
-    uint key = valid ? keys_in[i] : 0u;
-    uint val = valid ? (vals_in ? vals_in[i] : (uint)i) : 0u;
-    uint d = (key >> shift) & mask;
-    unsigned long long peers = __ballot(valid);
-    for (int b = 0; b < width; b++) {  // width is uniform: the ballots stay wave-wide
-      unsigned long long bb = __ballot((d >> b) & 1u);
-      peers &= ((d >> b) & 1u) ? bb : ~bb;
-    }
-    uint rank = (uint)__popcll(peers & lt);
-    if (valid && rank == 0) wcnt[w][d] = (uint)__popcll(peers);
-    __syncthreads();
-    if (valid) {
-      uint pos = run[d] + rank;
-      for (int k = 0; k < w; k++) pos += wcnt[k][d];
-      keys_out[pos] = key;
-      vals_out[pos] = val;
-    }
-    __syncthreads();
-    for (int dd = t; dd < nbin; dd += SORT_THREADS) {
-      uint add = 0;
+  for (uint tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const uint g = tile / GROUP_TILES;
+    const size_t base = (size_t)tile * SORT_TILE + w * (64 * SORT_ITEMS) + lane;
+    uint key[SORT_ITEMS], val[SORT_ITEMS], rank[SORT_ITEMS], mine[DP];
 #pragma unroll
-      for (int k = 0; k < SORT_WAVES; k++) {
-        add += wcnt[k][dd];
-        wcnt[k][dd] = 0;
+    for (int j = 0; j < SORT_ITEMS; j++) {
+      const size_t i = base + 64 * j;
+      key[j] = i < n ? keys_in[i] : 0u;
+      val[j] = i < n ? (vals_in ? vals_in[i] : (uint)i) : 0u;
+    }
+#pragma unroll
+    for (uint k = 0; k < DP; k++) mine[k] = t * DP + k < nbin ? pre[(size_t)tile * nbin + t * DP + k] : 0u;
+    for (uint x = t; x < W * RADIX; x += SORT_THREADS) (&cnt[0][0])[x] = 0u;
+    for (uint x = t; x < RADIX; x += SORT_THREADS) all[x] = before[x] = 0u;
+    __syncthreads();
+    if (total) {
+      for (uint d = t; d < nbin; d += SORT_THREADS) {
+        all[d] = total[d];
+        before[d] = gsum[(size_t)g * nbin + d];
       }
-      run[dd] += add;
+    } else {  // four digits of every few groups
+      const uint quads = nbin / 4u, q = t & (quads - 1u), rows = SORT_THREADS / quads;
+      uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+#pragma unroll 8
+      for (uint r = t / quads; r < ngroups; r += rows) {
+        const uint4 v = reinterpret_cast<const uint4 *>(gsum)[(size_t)r * quads + q];
+        const uint m = r < g ? 0xffffffffu : 0u;
+        a = make_uint4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
+        b = make_uint4(b.x + (v.x & m), b.y + (v.y & m), b.z + (v.z & m), b.w + (v.w & m));
+      }
+      atomicAdd(&all[4 * q], a.x), atomicAdd(&all[4 * q + 1], a.y);
+      atomicAdd(&all[4 * q + 2], a.z), atomicAdd(&all[4 * q + 3], a.w);
+      atomicAdd(&before[4 * q], b.x), atomicAdd(&before[4 * q + 1], b.y);
+      atomicAdd(&before[4 * q + 2], b.z), atomicAdd(&before[4 * q + 3], b.w);
+    }
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; j++) {
+      const bool valid = base + 64 * j < n;
+      const uint d = (key[j] >> shift) & mask;
+      unsigned long long peers = __ballot(valid);
+      for (int b = 0; b < width; b++) {  // width is uniform: the ballots stay wave-wide
+        const unsigned long long bb = __ballot((d >> b) & 1u);
+        peers &= ((d >> b) & 1u) ? bb : ~bb;
+      }
+      const uint lower = (uint)__popcll(peers & lt);
+      const uint seen = cnt[w][d];
+      rank[j] = seen + lower;
+      // the row is read by every lane before its digits' first lanes write it, and written
+      // before the next round reads it
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (valid && lower == 0u) cnt[w][d] = seen + (uint)__popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
+    uint tot, sum = 0, here = 0, local[DP];
+#pragma unroll
+    for (uint k = 0; k < DP; k++) {
+      const uint d = t * DP + k;
+      local[k] = 0u;
+      if (d < nbin) {
+        sum += all[d];
+#pragma unroll
+        for (int x = 0; x < W; x++) local[k] += cnt[x][d];
+        here += local[k];
+      }
+    }
+    uint smaller = block_excl_scan(sum, lw, tot);  // keys of smaller digits: in all
+    uint at = block_excl_scan(here, lw, tot);      // and in this tile
+#pragma unroll
+    for (uint k = 0; k < DP; k++) {
+      const uint d = t * DP + k;
+      if (d < nbin) {
+        before[d] = smaller + before[d] + mine[k] - at;  // place of a key - its place in the tile
+        uint q = at;
+#pragma unroll
+        for (int x = 0; x < W; x++) {
+          const uint c = cnt[x][d];
+          cnt[x][d] = q;
+          q += c;
+        }
+        smaller += all[d];
+        at += local[k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; j++)
+      if (base + 64 * j < n) {
+        const uint q = cnt[w][(key[j] >> shift) & mask] + rank[j];
+        skey[q] = key[j];
+        sval[q] = val[j];
+      }
+    __syncthreads();
+#pragma unroll
+    for (uint j = 0; j < SORT_ITEMS; j++) {  // a digit's keys side by side
+      const uint q = j * SORT_THREADS + t;
+      if (q < tot) {
+        const uint k = skey[q], to = before[(k >> shift) & mask] + q;
+        keys_out[to] = k;
+        vals_out[to] = sval[q];
+      }
+    }
+    __syncthreads();  // the counts start over
   }
-  }  // tile
 }
 
 inline uint blocks_for(size_t n, size_t per) { return (uint)((n + per - 1) / per); }
@@ -233,8 +364,11 @@ inline uint blocks_for(size_t n, size_t per) { return (uint)((n + per - 1) / per
 }  // namespace
 
 size_t sph_scan_tmp_elems(size_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
-size_t sph_sort_tiles(size_t n) { return (n + SORT_TILE - 1) / SORT_TILE; }
-size_t sph_sort_hist_elems(size_t n) { return (size_t)RADIX * sph_sort_tiles(n); }
+// per tile, per group and one row of totals, for any tile size
+size_t sph_sort_hist_elems(size_t n) {
+  const size_t tiles = (n + SORT_TILE_MIN - 1) / SORT_TILE_MIN;
+  return (size_t)RADIX * (tiles + (tiles + GROUP_TILES - 1) / GROUP_TILES + 1);
+}
 
 void sph_exclusive_scan(const uint *in, uint *out, const uint *n_dev, uint n_max, uint *total_dev,
                         uint *tmp, hipStream_t st) {
@@ -293,28 +427,37 @@ namespace {
 // and writes the other pair, (vbuf0 standing in as v0's storage). The result ends in
 // (*keys_out, *vals_out).
 // n_dev (optional): a device word holding the key count, n only bounding it; grid
-// (optional): a persistent grid for the histogram and scatter kernels; len_dev: a device word
-// for the histogram length when n_dev is given.
+// (optional): a persistent grid for the histogram and scatter kernels.
 void radix_passes(uint *k0, const uint *v0, uint *vbuf0, uint *k1, uint *v1, uint n, int bits,
-                  uint *tile_hist, uint *scan_tmp, uint **keys_out, uint **vals_out,
-                  hipStream_t st, const uint *n_dev = nullptr, uint grid = 0,
-                  uint *len_dev = nullptr) {
+                  uint *tile_hist, uint **keys_out, uint **vals_out, hipStream_t st,
+                  const uint *n_dev = nullptr, uint grid = 0) {
   const uint *kin = k0, *vin = v0;
   uint *kout = k1, *vout = v1;
-  const uint ntiles = (uint)sph_sort_tiles(n);
-  const uint tiles_grid = grid ? grid : ntiles;
+  const int waves = sort_waves(n);
+  const uint threads = 64u * waves, tile_keys = threads * SORT_ITEMS;
+  const uint ntiles = blocks_for(n, tile_keys), ngroups = blocks_for(ntiles, GROUP_TILES);
+  const bool based = ngroups > BASE_GROUPS;
   if (bits < 1) bits = 1;
   // fewest passes of at most RADIX_BITS bits, the digit width spread evenly over them
   const int passes = (bits + RADIX_BITS - 1) / RADIX_BITS;
   const int width = (bits + passes - 1) / passes;
-  for (int p = 0; p < passes; p++) {
+  uint *const gsum = tile_hist + (size_t)RADIX * ntiles, *const total = gsum + (size_t)RADIX * ngroups;
+  for (int p = 0; p < passes && n > 0; p++) {
     const int shift = p * width;
-    hipLaunchKernelGGL(k_radix_hist, dim3(tiles_grid), dim3(SORT_THREADS), 0, st, kin, n_dev, n,
-                       shift, width, tile_hist, n_dev ? len_dev : nullptr);
-    sph_exclusive_scan(tile_hist, tile_hist, n_dev ? len_dev : nullptr,
-                       (uint)((1u << width) * ntiles), nullptr, scan_tmp, st);
-    hipLaunchKernelGGL(k_radix_scatter, dim3(tiles_grid), dim3(SORT_THREADS), 0, st, kin, vin,
-                       n_dev, n, shift, width, tile_hist, kout, vout);
+#define SPH_RADIX(KERNEL, blocks, ...)                                                       \
+  do {                                                                                       \
+    const dim3 g(grid ? grid : (blocks)), b(threads);                                        \
+    if (waves == 4) KERNEL<4><<<g, b, 0, st>>>(__VA_ARGS__);                                  \
+    else if (waves == 8) KERNEL<8><<<g, b, 0, st>>>(__VA_ARGS__);                             \
+    else KERNEL<16><<<g, b, 0, st>>>(__VA_ARGS__);                                            \
+  } while (0)
+    SPH_RADIX(k_radix_hist, ngroups, kin, n_dev, n, shift, width, tile_hist, gsum);
+    if (based)
+      hipLaunchKernelGGL(k_radix_base, dim3(blocks_for(radix_bins(width), BASE_DIGITS)), dim3(BASE_THREADS),
+                         0, st, n_dev, n, width, GROUP_TILES * tile_keys, gsum, total);
+    SPH_RADIX(k_radix_scatter, ntiles, kin, vin, n_dev, n, shift, width, tile_hist, gsum,
+              based ? total : nullptr, kout, vout);
+#undef SPH_RADIX
     // next pass reads what this one wrote
     uint *nk = kout, *nv = vout;
     if (kout == k1) {
@@ -335,13 +478,12 @@ void radix_passes(uint *k0, const uint *v0, uint *vbuf0, uint *k1, uint *v1, uin
 
 void sph_radix_sort(uint *keys, uint *vals, uint n, int bits, SortScratch &sc, uint **keys_out,
                     uint **vals_out, hipStream_t st, const uint *n_dev, uint grid) {
-  radix_passes(keys, nullptr, vals, sc.keys_alt, sc.vals_alt, n, bits, sc.tile_hist, sc.scan_tmp,
-               keys_out, vals_out, st, n_dev, grid, sc.len_dev);
+  radix_passes(keys, nullptr, vals, sc.keys_alt, sc.vals_alt, n, bits, sc.tile_hist, keys_out,
+               vals_out, st, n_dev, grid);
 }
 
 // ---------------------------------------------------------------------------------------
-// Sort without allocation. The sort's working memory (ping-pong partners, tile histograms,
-// scan block sums) is one static device array instead of buffers a context allocates, so
+// Sort without allocation. The sort's working memory (ping-pong partners, histograms) is one static device array instead of buffers a context allocates, so
 // the call makes no hipMalloc/hipFree: for callers that cannot allocate (code under stream
 // capture into a graph, serving loops that forbid allocation). Each GPU holds its own copy
 // of the array for the life of the process; every call on one GPU shares it, so calls that
@@ -350,15 +492,14 @@ void sph_radix_sort(uint *keys, uint *vals, uint n, int bits, SortScratch &sc, u
 // ---------------------------------------------------------------------------------------
 namespace {
 constexpr uint kNoAllocMaxKeys = 1u << 20;
-constexpr size_t kNoAllocHist = (size_t)RADIX * ((kNoAllocMaxKeys + SORT_TILE - 1) / SORT_TILE);
-constexpr size_t kNoAllocScanTmp = (kNoAllocHist + SCAN_TILE - 1) / SCAN_TILE + 1;
-// [keys_alt | vals_alt | tile histograms | scan block sums], every part 256-byte aligned
+constexpr size_t kNoAllocTiles = (kNoAllocMaxKeys + SORT_TILE_MIN - 1) / SORT_TILE_MIN;
+constexpr size_t kNoAllocHist = (size_t)RADIX * (kNoAllocTiles + (kNoAllocTiles + GROUP_TILES - 1) / GROUP_TILES + 1);
+// [keys_alt | vals_alt | histograms], every part 256-byte aligned
 constexpr size_t kNoAllocKeysAlt = 0;
 constexpr size_t kNoAllocValsAlt = kNoAllocKeysAlt + kNoAllocMaxKeys;
 constexpr size_t kNoAllocHistOff = kNoAllocValsAlt + kNoAllocMaxKeys;
-constexpr size_t kNoAllocScanOff = kNoAllocHistOff + kNoAllocHist;
-constexpr size_t kNoAllocWords = kNoAllocScanOff + (kNoAllocScanTmp + 63) / 64 * 64;
-static_assert(kNoAllocHistOff % 64 == 0 && kNoAllocScanOff % 64 == 0, "scratch part alignment");
+constexpr size_t kNoAllocWords = kNoAllocHistOff + kNoAllocHist;
+static_assert(kNoAllocHistOff % 64 == 0, "scratch part alignment");
 static_assert(SPH_SORT_NOALLOC_MAX_KEYS == kNoAllocMaxKeys, "header limit");
 }  // namespace
 
@@ -407,8 +548,7 @@ extern "C" int sph_sort_noalloc(uint32_t *hash, uint32_t *index, uint32_t n, uin
   hipStream_t st = (hipStream_t)stream;
   uint *ko = nullptr, *vo = nullptr;
   radix_passes(hash, index, index, base + kNoAllocKeysAlt, base + kNoAllocValsAlt, n,
-               key_bits ? (int)key_bits : 32, base + kNoAllocHistOff, base + kNoAllocScanOff, &ko,
-               &vo, st);
+               key_bits ? (int)key_bits : 32, base + kNoAllocHistOff, &ko, &vo, st);
   if (ko != hash)  // an odd number of passes ends in the scratch pair
     hipLaunchKernelGGL(k_copy_pairs, dim3((n + 255) / 256), dim3(256), 0, st, ko, vo, hash, index, n);
   return hipGetLastError() == hipSuccess ? SPH_OK : SPH_EHIP;
