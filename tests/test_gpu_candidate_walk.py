@@ -65,17 +65,27 @@ def edges(p, a, r):
     a["pos"][m:2 * m] = q
 
 
+def brisk(p, a, r):
+    """Steps of up to one and a half cells."""
+    a["vel"] = r.uniform(-15.0, 15.0, a["vel"].shape)
+
+
 def fast(p, a, r):
     """Steps of up to 40 cells."""
     a["vel"] = r.uniform(-400.0, 400.0, a["vel"].shape)
 
 
 @pytest.mark.parametrize("variant", [sa.V2D, sa.V3D2, sa.V3D4])
-@pytest.mark.parametrize("kind", ["crowd", "edges", "fast", "swap"])
+@pytest.mark.parametrize("kind", ["crowd", "edges", "brisk", "fast", "swap", "nan"])
 def test_one_step(variant, kind):
     p, a, r = base(variant, 7, kind == "swap")
-    if kind != "swap":
-        {"crowd": crowd, "edges": edges, "fast": fast}[kind](p, a, r)
+    if kind in ("crowd", "edges", "swap"):  # the energy sees small steps, or the same edges again
+        p["time_step"] = 0.0 if kind == "edges" else 0.001
+    if kind == "nan":  # a few particles whose velocity is not finite
+        a["vel"][::9001] = np.nan
+        a["vel"][5::9001, -1] = np.inf
+    elif kind != "swap":
+        {"crowd": crowd, "edges": edges, "brisk": brisk, "fast": fast}[kind](p, a, r)
     print("variant", variant, kind, flush=True)
     o = orc.Oracle(variant, p, len(a))
     o.upload(a)
