@@ -340,7 +340,8 @@ struct SphCtx {
   uint n_sorted = 0, n_flagged = 0, n_status = 0;
   bool hashed = false, sorted = false, lists_valid = false, merged = false, compacted = false;
   bool qual_ready = false;  // the step's energy kernel wrote sb.qual
-  bool erec_ok = false;  // aux.erec holds the current positions and velocities
+  // aux.erec, ez and qpos hold the current positions and velocities, in the current parameters' steps
+  bool erec_ok = false;
   // aux.nbl holds the force pairs of the current state, cell lists and parameters (the
   // density kernel writes them; anything else that runs invalidates them)
   bool nbl_ok = false;
@@ -925,7 +926,8 @@ int sph_set_params(SphCtx *ctx, const void *sysparam) {
   std::memcpy(ctx->raw, sysparam, ctx->raw_size);
   if (std::memcmp(&P, &ctx->P, sizeof(P)) != 0) ctx->drop_graphs();  // they hold the parameters
   ctx->P = P;
-  ctx->nbl_ok = false;  // the pair lists were made with the old kernel radii
+  ctx->nbl_ok = false;   // the pair lists were made with the old kernel radii
+  ctx->erec_ok = false;  // and the quantised positions with the old steps and marks
   return SPH_OK;
 }
 
