@@ -648,7 +648,8 @@ struct SphCtx {
     erec_ok = false;
     pbegin(SPH_P_MERGE);
     if (variant == SPH_V2D) launch_merge_q2d(P, cur, s2p_cell, cnt, cstart, cend, q2d, st);
-    if (!in_step) sph_fill_u32(sb.dead, 0u, sph_bit_words(m), st);
+    // all of them: a split may still come before compact, and its children's slots follow
+    if (!in_step) sph_fill_u32(sb.dead, 0u, sph_bit_words(cap), st);
     // a step in several lanes per particle leaves the qualification to each cell's walk
     launch_merge(variant, P, cur, cstart, cend, q2d, sb.dead, cnt, st, nullptr, skeys, n_sorted,
                  nd, nullptr, in_step && !qual_ready ? nullptr : sb.qual, in_step);

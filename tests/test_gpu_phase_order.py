@@ -1,6 +1,6 @@
 """Phase calls in orders other than a step's: parameters changed between integrate (or a step)
-and energy, above the counts from which the energy kernel reads quantised positions. Against the
-CPU oracle, bit for bit."""
+and energy, above the counts from which the energy kernel reads quantised positions; a split
+between merge and compact. Against the CPU oracle, bit for bit."""
 import numpy as np
 import pytest
 
@@ -70,4 +70,48 @@ def test_energy_after_other_radii(variant, n, before):
             o.energy()
             assert_particles_equal(g.download(), o.download(), ["pos", "vel", "energy", "level"],
                                    what="radii %d" % k)
+            o.close()
+
+
+def merge_split_scene(variant, n, seed, n_small, large_splits):
+    """Small particles that merge in pairs (or fours) and large ones that split or not."""
+    p = sa.param_defaults(variant)
+    r = np.random.default_rng(seed)
+    names = ("thresh_split", "thresh_merge") if variant == sa.V2D else ("split_criteria", "merge_criteria")
+    p[names[0]], p[names[1]] = 10.0, 1.0
+    p["co_energy"], p["co_surface"] = 1.0, 0.0
+    a = np.zeros(n, dtype=sa.particle_dtype(variant))
+    a["pos"] = 2.0 + r.uniform(0.0, 12.0 if variant == sa.V2D else 5.0, a["pos"].shape)
+    for f in ("vel", "ev", "acc"):
+        a[f] = r.uniform(-1.0, 1.0, a[f].shape)
+    a["dens"] = 1.0
+    a["level"] = 1 + (r.permutation(n) < n_small)
+    a["energy"] = np.where(a["level"] == 2, 0.5, 20.0 if large_splits else 5.0)
+    return p, a
+
+
+@pytest.mark.parametrize("variant", [sa.V2D, sa.V3D2, sa.V3D4])
+@pytest.mark.parametrize("n", [700, 1024, 1500, 2300])
+def test_split_between_merge_and_compact(variant, n):
+    """The children's slots lie past those that the merge saw, in words and 1024-slot tiles that an
+    earlier, larger merge has used."""
+    cap = 12000
+    print("variant", variant, "n", n, flush=True)
+    with sa.SPHContext(variant, sa.param_defaults(variant), cap, max_triangles=1) as g:
+        for count, small, splits in ((8000, 8000, False), (n, n // 3, True)):
+            p, a = merge_split_scene(variant, count, count, small, splits)
+            o = orc.Oracle(variant, p, cap)
+            g.set_params(p)
+            for x in (g, o):
+                x.upload(a)
+                for phase in ("calc_hash", "sort", "cell_ranges"):
+                    getattr(x, phase)()
+            groups = g.merge()
+            assert groups == o.merge() and groups > 0
+            assert g.split() == o.split()
+            g.compact()
+            o.compact()
+            assert not splits or g.num_particles() > n  # more children than removed particles
+            assert_particles_equal(g.download(), o.download(), what="%d particles" % count)
+            assert np.array_equal(g.get_u32(sa._abi.Q_STATUS)[:count], o.get_u32(orc.STATUS)[:count])
             o.close()
