@@ -326,7 +326,7 @@ struct SphCtx {
   uint *rep_seq = nullptr;       // reports made, on the device
   Report *rep = nullptr;         // the last report (pinned host memory) and its device address
   Report *rep_dev = nullptr;
-  uint rep_want = 0;             // reports launched
+  uint rep_want = 0;             // reports that were launched
   float *dgrid = nullptr, *normal3 = nullptr, *tris = nullptr;
   uint *cube_count = nullptr, *cube_off = nullptr;  // per z-segment: triangles, their offsets
   uint *seg_cube = nullptr, *seg_coff = nullptr;    // per z-segment: non-empty cubes, offsets
@@ -454,43 +454,49 @@ struct SphCtx {
     last_err = e;
     return SPH_EHIP;
   }
-  // Wait for the stream's work; the counters stay as the host knows them.
+  // Wait for the stream's work; the counters stay as the host knows them. An error that was there
+  // before (of a launch, or left in this thread by other code) is returned, but not before the
+  // work is done: copies to or from the caller's memory may be among it.
   int drain() {
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return fail(e);
+    hipError_t err = hipGetLastError();
+    const hipError_t e = hipStreamSynchronize(st);
+    if (err == hipSuccess) err = e;
+    if (err != hipSuccess) return fail(err);
     collect();
     return SPH_OK;
   }
   // Read the counters once the stream's work is done, collect timings. Returns an SPH status.
-  // reported: the work ended with a report kernel. The host polls the report's number for a
-  // while, about what a small scene's step takes, and then waits for the stream; a stream that
-  // fails, or ends without the report, ends the wait there.
+  // reported: the work ended with a report kernel, counted in rep_want where it was launched. The
+  // host polls the report's number for a while, about what a small scene's step takes, and then
+  // waits for the stream; a stream that fails, or ends without the report, ends the wait there.
+  // An error that was there before is returned after the counters are read, so that they and the
+  // number of reports stay those of the device.
   int sync(bool reported = false) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(e);
-    if (!reported) launch_report(cnt, rep_seq, rep_dev, st);
-    rep_want++;
+    hipError_t err = hipGetLastError();
+    if (!reported) {
+      launch_report(cnt, rep_seq, rep_dev, st);
+      const hipError_t e = hipGetLastError();
+      if (e == hipSuccess) rep_want++;
+      else if (err == hipSuccess) err = e;
+    }
     const bool events = !pending.empty() || tune.pending;  // read below or by the caller
     auto there = [&] { return __atomic_load_n(&rep->seq, __ATOMIC_ACQUIRE) == rep_want; };
     bool done = false;
-    for (uint k = 0; !events && !done && k < kReportPolls; k++) {
+    for (uint k = 0; !events && err == hipSuccess && !done && k < kReportPolls; k++) {
       done = there();
       __builtin_ia32_pause();
     }
     if (!done) {
-      e = hipGetLastError();
-      if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e != hipSuccess) return fail(e);
-      if (!there()) {  // a launch that failed
+      const hipError_t e = hipStreamSynchronize(st);
+      if (e != hipSuccess || !there()) {  // the work failed
         rep_want = rep->seq;
-        return fail(hipErrorUnknown);
+        return fail(err != hipSuccess ? err : e != hipSuccess ? e : hipErrorUnknown);
       }
     }
     collect();
     n = rep->c.n;
     m = rep->c.m;
-    return SPH_OK;
+    return err == hipSuccess ? SPH_OK : fail(err);
   }
 
   // ---- enqueue-only phase bodies ----
@@ -779,6 +785,7 @@ struct SphCtx {
       (void)hipGetLastError();
       return false;
     }
+    rep_want++;
     // the host's state after q_step
     std::swap(cur, alt);
     flipped = !flipped;

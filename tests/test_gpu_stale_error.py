@@ -1,0 +1,42 @@
+"""An error that other code left in the calling thread: the call that finds it says so, and the
+calls after it answer as if it had not been there. Steps launched one by one and as a captured
+graph, against the CPU oracle."""
+import numpy as np
+import pytest
+
+import sca2012_amd as sa
+from oracle import orc
+from sca2012_amd import scenes
+
+from helpers import assert_particles_equal
+
+pytestmark = pytest.mark.gpu
+SM = sa.STEP_SPLIT | sa.STEP_MERGE
+
+
+def leave_error(lib):
+    assert lib.hipSetDevice(1 << 20) != 0  # no such device: refused on the host
+
+
+@pytest.mark.parametrize("variant, flags", [(sa.V2D, SM), (sa.V3D2, SM), (sa.V3D2, 0)])
+def test_context_step(variant, flags):
+    p, a = scenes.reference_scene(variant)
+    cap = 8 * len(a)
+    o = orc.Oracle(variant, p, cap)
+    o.upload(a)
+    with sa.SPHContext(variant, p, cap, max_triangles=1) as g:
+        g.autotune(0)  # steps that repeat are captured after three launches of a buffer parity
+        g.upload(a)
+        for k in range(24):
+            fault = k in (1, 12, 17, 18)
+            if fault:
+                leave_error(g.lib)
+                with pytest.raises(sa.SphError) as e:
+                    g.step(flags)
+                assert e.value.code == sa._abi.EHIP
+            else:
+                g.step(flags)
+            assert o.step(flags) == 0
+            assert g.num_particles() == o.num_particles() == g.counters()["n"], k
+            if fault or k == 23:
+                assert_particles_equal(g.download(), o.download(), what="step %d" % k)
