@@ -1159,15 +1159,15 @@ int sph_get_u32(SphCtx *ctx, int which, uint32_t *out, size_t n) {
     case SPH_Q_COUNTERS: src = (const uint *)ctx->cnt; break;
     default: return SPH_EINVAL;
   }
+  // bits arrive in the first words of out and are spread from the last entry down (word k / 32 is
+  // still there when entry k is written)
   const bool bits = which == SPH_Q_SPLITFLAG || which == SPH_Q_STATUS;
-  std::vector<uint32_t> w(bits ? (n + 31) / 32 : 0);
-  if (hipMemcpyAsync(bits ? w.data() : out, src, (bits ? w.size() : n) * 4, hipMemcpyDeviceToHost,
-                     ctx->st) != hipSuccess)
+  if (hipMemcpyAsync(out, src, (bits ? (n + 31) / 32 : n) * 4, hipMemcpyDeviceToHost, ctx->st) != hipSuccess)
     return SPH_EHIP;
   int rc = ctx->drain();
   if (rc) return rc;
-  for (size_t k = 0; bits && k < n; k++)
-    out[k] = ((w[k >> 5] >> (k & 31)) & 1u) ^ (which == SPH_Q_SPLITFLAG ? 1u : 0u);
+  for (size_t k = bits ? n : 0; k-- > 0;)
+    out[k] = ((out[k >> 5] >> (k & 31)) & 1u) ^ (which == SPH_Q_SPLITFLAG ? 1u : 0u);
   return SPH_OK;
 }
 

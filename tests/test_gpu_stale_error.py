@@ -40,3 +40,25 @@ def test_context_step(variant, flags):
             assert g.num_particles() == o.num_particles() == g.counters()["n"], k
             if fault or k == 23:
                 assert_particles_equal(g.download(), o.download(), what="step %d" % k)
+
+
+def test_flags_read_in_part():
+    """Split flags and statuses, kept as bits, read for any number of slots, also right after a
+    refused read."""
+    p, a = scenes.reference_scene(sa.V3D2)
+    cap = 4 * len(a)
+    o = orc.Oracle(sa.V3D2, p, cap)
+    o.upload(a)
+    with sa.SPHContext(sa.V3D2, p, cap, max_triangles=1) as g:
+        g.upload(a)
+        for _ in range(3):
+            g.step(SM)
+            assert o.step(SM) == 0
+        for q, r in ((sa._abi.Q_SPLITFLAG, orc.SPLITFLAG), (sa._abi.Q_STATUS, orc.STATUS)):
+            ref = o.get_u32(r)
+            for n in (1, 2, 31, 32, 33, 63, 64, 65, 1023, 1025, len(ref) - 1, len(ref)):
+                leave_error(g.lib)
+                with pytest.raises(sa.SphError) as e:
+                    g.get_u32(q, n)
+                assert e.value.code == sa._abi.EHIP
+                assert np.array_equal(g.get_u32(q, n), ref[:n]), (q, n)
