@@ -329,34 +329,37 @@ struct SphBatch {
     return SPH_OK;
   }
 
-  // wait for the stream's work; the counters stay as the host knows them
+  int fail(hipError_t e) {
+    last_err = e;
+    return SPH_EHIP;
+  }
+  // Wait for the stream's work; the counters stay as the host knows them. An error that was there
+  // before (of a launch, or left in this thread by other code) is returned, but not before the
+  // work is done: copies to or from the caller's memory may be among it.
   int drain() {
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-      last_err = e;
-      return SPH_EHIP;
-    }
+    hipError_t err = hipGetLastError();
+    const hipError_t e = hipStreamSynchronize(st);
+    if (err == hipSuccess) err = e;
+    if (err != hipSuccess) return fail(err);
     collect();
     return SPH_OK;
   }
 
-  // synchronise and read every counter back
-  int sync() {
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(cnt_host, cnt, sizeof(Counters), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(scn_host, scn, sizeof(SceneCnt) * ns, hipMemcpyDeviceToHost, st);
+  // Wait and read every counter back; stepped: a step ran last, so the scenes' entries move too.
+  // An error that was there before is returned after that, so that counters and entries stay
+  // those of the device.
+  int sync(bool stepped = false) {
+    const hipError_t err = hipGetLastError();
+    hipError_t e = hipMemcpyAsync(cnt_host, cnt, sizeof(Counters), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(scn_host, scn, sizeof(SceneCnt) * ns, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) {
-      last_err = e;
-      return SPH_EHIP;
-    }
+    if (e != hipSuccess) return fail(err != hipSuccess ? err : e);
     collect();
     M = cnt_host->n;
     m = cnt_host->m;
     for (uint s = 0; s < ns; s++) n_host[s] = scn_host[s].n;
-    return SPH_OK;
+    if (stepped) spans_after_step();
+    return err == hipSuccess ? SPH_OK : fail(err);
   }
   // where a step left the scenes: their particles before the split in cell order, scene after
   // scene, then the children, scene after scene
@@ -539,21 +542,22 @@ struct SphBatch {
       int shape[3];
       ltune.next(shape);
       hipGraphExec_t ex = graph_for(flags, shape);
-      if (!ex) return SPH_EHIP;
       hipEvent_t a = nullptr;
-      ltune.before(st, shape, a);
-      if (hipGraphLaunch(ex, st) != hipSuccess) return SPH_EHIP;
+      if (ex) ltune.before(st, shape, a);
+      if (!ex || hipGraphLaunch(ex, st) != hipSuccess) {  // the steps before it count
+        (void)sync(k > 0);
+        return SPH_EHIP;
+      }
       ltune.after_launch(st, a);
       swap_state();  // the step's reorder moved the state to the other buffer
       if (pushes) {
-        const int rc = sync();
+        const int rc = sync(true);
         clear_pushes();
         if (rc) return rc;
       }
     }
-    const int rc = sync();
+    const int rc = sync(true);
     ltune.collect();
-    if (rc == SPH_OK) spans_after_step();
     return rc;
   }
 
@@ -774,10 +778,9 @@ int sph_batch_step(SphBatch *b, uint32_t flags, uint32_t steps, uint32_t *n_tota
   for (uint32_t k = 0; k < steps; k++) {
     if (b->M == 0) return SPH_EEMPTY;
     b->enqueue_step(flags);
-    rc = b->sync();
+    rc = b->sync(true);
     b->clear_pushes();
     if (rc) return rc;
-    b->spans_after_step();
     b->tune.end_step();
     if (b->cnt_host->err) rc = SPH_EDOMAIN;
   }

@@ -62,3 +62,41 @@ def test_flags_read_in_part():
                     g.get_u32(q, n)
                 assert e.value.code == sa._abi.EHIP
                 assert np.array_equal(g.get_u32(q, n), ref[:n]), (q, n)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_step(graph):
+    """Also the places of the scenes' particles, which every step moves: they are read right after
+    the refused call."""
+    sizes = [300, 1200, 77, 2500]
+    tanks = [scenes.tank_3d2(int(n), scenes.SEED_BASE + 50, s) for s, n in enumerate(sizes)]
+    caps = [4 * n + 8 for n in sizes]
+    b = sa.SPHBatch(sa.V3D2, [p for p, _ in tanks], caps)
+    b.set_graph(graph)
+    oracles = []
+    for s, (p, a) in enumerate(tanks):
+        o = orc.Oracle(sa.V3D2, p, caps[s])
+        o.upload(a)
+        b.upload(s, a)
+        oracles.append(o)
+    for k in range(8):
+        fault = k in (0, 3, 6, 7)
+        if fault:
+            leave_error(b.lib)
+            assert b.step_raw(SM, 2 if graph else 1)[0] == sa._abi.EHIP
+        else:
+            b.step(SM, 2 if graph else 1)
+        for o in oracles:
+            for _ in range(2 if graph else 1):
+                assert o.step(SM) == 0
+        assert list(b.num_particles()) == [o.num_particles() for o in oracles]
+        for s, o in enumerate(oracles):
+            assert_particles_equal(b.download(s), o.download(), what="call %d scene %d" % (k, s))
+        if k == 5:  # an upload that follows refused calls
+            leave_error(b.lib)
+            with pytest.raises(sa.SphError):
+                b.upload(1, tanks[1][1])
+            b.upload(2, tanks[2][1])
+            for s in (1, 2):
+                oracles[s].upload(tanks[s][1])
+    b.close()
