@@ -379,7 +379,8 @@ struct SphCtx {
     uint64_t last;
     hipGraphExec_t exec;  // null until the step has run kGraphAfter times
   };
-  std::vector<StepGraph> graphs;
+  StepGraph graphs[kGraphsMax];  // the first n_graphs
+  size_t n_graphs = 0;
   uint64_t graph_clock = 0;
   bool graphs_work = true;    // false once a capture has failed
   bool flipped = false;       // cur is the second state buffer
@@ -394,8 +395,8 @@ struct SphCtx {
     }
     for (auto e : ev_pool) (void)hipEventDestroy(e);
     for (void *p : allocs) (void)hipFree(p);
-    for (auto &g : graphs)
-      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    for (size_t k = 0; k < n_graphs; k++)
+      if (graphs[k].exec) (void)hipGraphExecDestroy(graphs[k].exec);
     if (rep) (void)hipHostFree(rep);
     if (st) (void)hipStreamDestroy(st);
   }
@@ -709,11 +710,11 @@ struct SphCtx {
   }
 
   void drop_graphs() {
-    if (graphs.empty()) return;
+    if (n_graphs == 0) return;
     (void)hipStreamSynchronize(st);
-    for (auto &g : graphs)
-      if (g.exec) (void)hipGraphExecDestroy(g.exec);
-    graphs.clear();
+    for (size_t k = 0; k < n_graphs; k++)
+      if (graphs[k].exec) (void)hipGraphExecDestroy(graphs[k].exec);
+    n_graphs = 0;
   }
   // The step as one captured graph, its report included, when it has run kGraphAfter times with
   // the same launches (a capture takes longer than a step; a scene that is stepped a few times
@@ -730,19 +731,19 @@ struct SphCtx {
     aux.choose_forms(variant, false, n);
     const StepKey key{bound, flags & 7u, aux.forms(), (uint)tune.force | (uint)tune.energy << 8,
                       (flipped ? 1u : 0u) | (par ? 2u : 0u)};
-    auto g = std::find_if(graphs.begin(), graphs.end(), [&](const StepGraph &x) { return x.key == key; });
-    if (g == graphs.end()) {
-      if (graphs.size() >= kGraphsMax) {  // the one unused for longest goes
-        g = std::min_element(graphs.begin(), graphs.end(),
-                             [](const StepGraph &a, const StepGraph &b) { return a.last < b.last; });
+    StepGraph *const all = graphs, *end = all + n_graphs;
+    StepGraph *g = std::find_if(all, end, [&](const StepGraph &x) { return x.key == key; });
+    if (g == end) {
+      if (n_graphs < kGraphsMax) {
+        n_graphs++;
+      } else {  // the one unused for longest goes
+        g = std::min_element(all, end, [](const StepGraph &a, const StepGraph &b) { return a.last < b.last; });
         if (g->exec) {
           (void)hipStreamSynchronize(st);
           (void)hipGraphExecDestroy(g->exec);
         }
-        graphs.erase(g);
       }
-      graphs.push_back({key, 0u, 0u, nullptr});
-      g = graphs.end() - 1;
+      *g = StepGraph{key, 0u, 0u, nullptr};
     }
     g->last = ++graph_clock;
     if (!g->exec) {
