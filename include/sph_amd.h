@@ -245,22 +245,26 @@ int sph_prof_enable(SphCtx *ctx, int on);
 int sph_prof_phases(SphCtx *ctx, uint32_t phase_mask);
 
 /* ---- autotuning of the pair-list lengths (no counterpart in the reference) ----
- * The force and energy kernels queue interacting pairs in per-thread LDS lists; the list
- * length (force 24/32/48, energy 16/24/32 entries) changes only where the lists are
+ * Where the force kernel runs one thread per particle (3D: above 6,000,000 particles, a
+ * batch's scenes together above 150,000; 2D: above 100,000) it queues interacting pairs in
+ * per-thread LDS lists; the list length (24/32/48 entries) changes only where the lists are
  * drained, never the order in which a particle's terms are summed, so every length gives
- * the same bits. A context tunes itself in rounds of 12 steps (the first round of a tuning
- * run: 6): each step of a round runs both kernels with one candidate length, the
- * candidates taking turns in the order 0 1 2 2 1 0 0 1 2 2 1 0 so that a cost drifting
- * from step to step weighs on all alike, timed with events; after the round each kernel
- * switches to the length with the lowest mean time if it beats the length in use by more
- * than 5% (10% in the later rounds). The first round starts after 8 steps, the next ones
- * every 128 steps (the best length drifts with a scene's neighbour counts).
+ * the same bits. The energy kernel has one form: its lengths (16/24/32) can be set and are
+ * reported, and select nothing. A context tunes itself in rounds of 12 steps (the first
+ * round of a tuning run: 6): each step of a round runs the force kernel with one candidate
+ * length, the candidates taking turns in the order 0 1 2 2 1 0 0 1 2 2 1 0 so that a cost
+ * drifting from step to step weighs on all alike, timed with events; after the round the
+ * force kernel switches to the length with the lowest mean time if it beats the length in
+ * use by more than 5% (10% in the later rounds). The first round starts after 8 steps, the
+ * next ones every 128 steps (the best length drifts with a scene's neighbour counts). While
+ * the force kernel has no lists, one step of the first round is timed, whose times stand
+ * for every length, and nothing is tried.
  * sph_autotune(rounds, after_steps, every_steps) restarts that: `rounds` rounds (0 stops
  * tuning and keeps the current lengths), the first after `after_steps` more steps, then one
  * every `every_steps` steps (at least 12). sph_tuned_lists reports the lengths in use and,
  * in best_ms (6 floats, may be NULL), the mean time per candidate in the last round
- * (force 24/32/48, energy 16/24/32; -1 = not measured). The phase calls (sph_force,
- * sph_energy) use the current lengths. */
+ * (force 24/32/48, energy 16/24/32; -1 = not measured). The phase call sph_force uses the
+ * current length. */
 int sph_autotune(SphCtx *ctx, uint32_t rounds, uint32_t after_steps, uint32_t every_steps);
 int sph_tuned_lists(SphCtx *ctx, uint32_t *force_list, uint32_t *energy_list, float *best_ms);
 /* pins the lengths and stops tuning; SPH_EINVAL for a length that is not a candidate */

@@ -57,7 +57,10 @@ constexpr int kGridDefault = 0;
 // call's synchronisation) the dimension takes the candidate with the lowest mean step time
 // if it beats the current one by more than kTuneMargin. Rounds follow one another from
 // `after` steps on; a cycle over the three dimensions repeats every `every` steps (a
-// scene's neighbour counts, and with them the best lengths, drift).
+// scene's neighbour counts, and with them the best lengths, drift). A length that no kernel
+// of the step reads (the energy kernel's; the force kernel's while it runs in several lanes
+// per particle) runs the same graph for every candidate: the mean of the round's steps
+// stands for each, and the choice stays.
 struct LaunchTuner {
   static constexpr int kDims = 3;
   static constexpr int kCands[kDims] = {4, 3, 3};
@@ -72,7 +75,8 @@ struct LaunchTuner {
   float sum[kDims][4];
   int cnt[kDims][4];
   float best[kDims][4];  // mean ms per candidate in the last finished round of each dimension
-  struct Pending { int dim, cand; uint rid; hipEvent_t a, b; };
+  bool same[kDims] = {false, false, false};  // some step of the gathered round had equal candidates
+  struct Pending { int dim, cand; uint rid; bool same; hipEvent_t a, b; };
   std::vector<Pending> pending;
   std::vector<hipEvent_t> pool;
 
@@ -85,6 +89,7 @@ struct LaunchTuner {
   }
   void clear_sums(int d) {
     acc_n[d] = 0;
+    same[d] = false;
     for (int c = 0; c < 4; c++) {
       sum[d][c] = 0.0f;
       cnt[d][c] = 0;
@@ -122,13 +127,13 @@ struct LaunchTuner {
     (void)hipEventCreate(&e);
     return e;
   }
-  // around the graph launch of a step with `shape`
-  void before(hipStream_t st, const int shape[kDims], hipEvent_t &a) {
+  // around the graph launch of a step with `shape`; force_counts: its force kernel has lists
+  void before(hipStream_t st, const int shape[kDims], bool force_counts, hipEvent_t &a) {
     a = nullptr;
     if (!tuning()) return;
     a = take();
     (void)hipEventRecord(a, st);
-    pending.push_back({dim, shape[dim], rid, a, nullptr});
+    pending.push_back({dim, shape[dim], rid, dim == 2 || (dim == 1 && !force_counts), a, nullptr});
   }
   void after_launch(hipStream_t st, hipEvent_t a) {
     if (a) {
@@ -152,6 +157,17 @@ struct LaunchTuner {
   }
   void finish(int d) {
     const int k = kCands[d];
+    if (same[d]) {
+      float s = 0.0f;
+      int n = 0;
+      for (int c = 0; c < k; c++) {
+        s += sum[d][c];
+        n += cnt[d][c];
+      }
+      for (int c = 0; c < k; c++) best[d][c] = n ? s / (float)n : -1.0f;
+      clear_sums(d);
+      return;
+    }
     for (int c = 0; c < k; c++) best[d][c] = cnt[d][c] ? sum[d][c] / (float)cnt[d][c] : -1.0f;
     int pick = cur[d];
     for (int c = 0; c < k; c++)
@@ -175,6 +191,7 @@ struct LaunchTuner {
         sum[d][p.cand] += ms;
         cnt[d][p.cand] += 1;
       }
+      same[d] = same[d] || p.same;
       if (++acc_n[d] == round_len(d)) finish(d);
       pool.push_back(p.a);
       if (p.b) pool.push_back(p.b);
@@ -230,7 +247,7 @@ struct SphBatch {
   int open_phase = -1;
   hipEvent_t open_ev = nullptr;
 
-  ListTuner tune;  // pair-list lengths of the force and energy kernels (stream steps)
+  ListTuner tune;  // pair-list length of the force kernel (stream steps)
 
   // graph steps
   bool use_graph = true;
@@ -397,10 +414,10 @@ struct SphBatch {
 
   // One step of every scene.
   //   stream step (grid == 0): launches sized by M (live) and m (entries), which the host
-  //     read at the end of the previous step; the list tuner picks the pair-list lengths.
+  //     read at the end of the previous step; the list tuner picks the pair-list length.
   //   graph step (dev): launches that read every count on the device (the host bounds are
   //     the buffers' size), sized by those bounds (grid == 0) or persistent over `grid`
-  //     workgroups, with list lengths lf, le; no events, so the enqueued work can be
+  //     workgroups, with force list length lf; no events, so the enqueued work can be
   //     captured into a graph.
   bool energy_unit_all() const {
     for (const DevParams &p : P)
@@ -408,7 +425,7 @@ struct SphBatch {
     return true;
   }
 
-  void enqueue_step(uint flags, bool dev = false, uint grid = 0, int lf = -1, int le = -1) {
+  void enqueue_step(uint flags, bool dev = false, uint grid = 0, int lf = -1) {
     const BatchView bv = view();
     const DevParams &P0 = P[0];
     const int v = variant;
@@ -421,6 +438,7 @@ struct SphBatch {
     const uint *n_live = dev ? &cnt->n : nullptr;   // live entries at the start of the step
     const uint *n_pre = dev ? &cnt->n_pre : nullptr;  // the same, once split has moved n
     aux.choose_forms(v, true, M);  // M: the live count at the call's start, also for a graph
+    tune.force_counts = !aux.fine_force;
     launch_batch_begin(bv, cnt, st);
     if (bins.ccount) {
       skeys = sc.keys_alt;
@@ -480,7 +498,7 @@ struct SphBatch {
     auto energy = [&](int) {
       launch_energy(v, Pe, cur, aux, cstart, cend, Mb, st, &bv, split_bits, qual, n_live);
     };
-    if (dev) energy(le);
+    if (dev) energy(tune.energy);
     else tune.run(1, st, energy);
     pend();
     pbegin(SPH_P_SPLIT);
@@ -500,12 +518,11 @@ struct SphBatch {
   }
 
   // The graph of one step with this shape, flags and state-buffer parity (captured on first
-  // use). Returns nullptr if capture or instantiation failed.
+  // use; lengths that no kernel reads share one). Returns nullptr if capture or instantiation failed.
   hipGraphExec_t graph_for(uint flags, const int shape[3]) {
     aux.choose_forms(variant, true, M);
-    const uint key = (flags & 3u) | ((uint)shape[0] << 2) | ((uint)shape[1] << 4) |
-                     ((uint)shape[2] << 6) | ((parity ? 1u : 0u) << 8) |
-                     ((energy_unit_all() ? 1u : 0u) << 9) | (aux.forms() << 10);
+    const uint key = (flags & 3u) | ((uint)shape[0] << 2) | ((aux.fine_force ? 0u : (uint)shape[1]) << 4) |
+                     ((parity ? 1u : 0u) << 8) | ((energy_unit_all() ? 1u : 0u) << 9) | (aux.forms() << 10);
     for (auto &g : graphs)
       if (g.key == key) return g.exec;
     const uint grid = kGridPerCU[shape[0]] * num_cu;
@@ -517,7 +534,7 @@ struct SphBatch {
     hipGraphExec_t ex = nullptr;
     hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
-      enqueue_step(flags, true, grid, shape[1], shape[2]);
+      enqueue_step(flags, true, grid, shape[1]);
       e = hipStreamEndCapture(st, &g);
     }
     // capture only recorded the step: the host's view of the buffers stays as it was
@@ -543,7 +560,7 @@ struct SphBatch {
       ltune.next(shape);
       hipGraphExec_t ex = graph_for(flags, shape);
       hipEvent_t a = nullptr;
-      if (ex) ltune.before(st, shape, a);
+      if (ex) ltune.before(st, shape, !aux.fine_force, a);
       if (!ex || hipGraphLaunch(ex, st) != hipSuccess) {  // the steps before it count
         (void)sync(k > 0);
         return SPH_EHIP;

@@ -363,13 +363,13 @@ struct SphCtx {
   int open_phase = -1;
   hipEvent_t open_ev = nullptr;
 
-  ListTuner tune;  // pair-list lengths of the force and energy kernels
+  ListTuner tune;  // pair-list length of the force kernel
 
   // Captured steps (graph_step): everything a step's launches depend on but the device's state
   struct StepKey {
-    uint bound, flags, forms, lists, buffers;
+    uint bound, flags, forms, list, buffers;
     bool operator==(const StepKey &o) const {
-      return bound == o.bound && flags == o.flags && forms == o.forms && lists == o.lists &&
+      return bound == o.bound && flags == o.flags && forms == o.forms && list == o.list &&
              buffers == o.buffers;
     }
   };
@@ -728,8 +728,7 @@ struct SphCtx {
     uint bound = 1024;
     while (bound < std::max(n, m) && bound < cap) bound *= 2;
     bound = std::min(bound, cap);
-    aux.choose_forms(variant, false, n);
-    const StepKey key{bound, flags & 7u, aux.forms(), (uint)tune.force | (uint)tune.energy << 8,
+    const StepKey key{bound, flags & 7u, aux.forms(), tune.force_counts ? (uint)tune.force : 0u,
                       (flipped ? 1u : 0u) | (par ? 2u : 0u)};
     StepGraph *const all = graphs, *end = all + n_graphs;
     StepGraph *g = std::find_if(all, end, [&](const StepGraph &x) { return x.key == key; });
@@ -1103,6 +1102,8 @@ int sph_marching_cubes(SphCtx *ctx, uint32_t *n_tri) {
 int sph_step(SphCtx *ctx, uint32_t flags, uint32_t *n_out) {
   CHECK_CTX(ctx);
   if (ctx->n == 0) return SPH_EEMPTY;
+  ctx->aux.choose_forms(ctx->variant, false, ctx->n);
+  ctx->tune.force_counts = !ctx->aux.fine_force;
   const bool reported = ctx->graph_step(flags);
   if (!reported) ctx->q_step(flags);
   // the cell-range phase made physical == live before split appended children

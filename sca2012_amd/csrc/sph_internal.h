@@ -597,25 +597,29 @@ void launch_download(int variant, DevState s, Span at, uint n, void *aos_dev, hi
                      uint scene = 0u);
 void launch_slot2phys(DevState s, uint m, uint *slot2phys, hipStream_t st);
 
-// Online autotuner of the pair-list lengths of the force and energy kernels, shared by
-// the single-scene context and the batch. The length never changes the order in which a
-// particle's terms are summed, so the results do not depend on tuning. Tuning starts after
-// `after` steps (a scene's first steps are not representative: cold caches, and an
-// adaptive scene grows over its first few steps). A round is 12 tuning steps (the first
-// round of a tuning run 6); each runs each kernel once, with one candidate length,
-// bracketed by events; the candidates take turns in the order 0 1 2 2 1 0 0 1 2 2 1 0, so
-// a cost that drifts linearly from step to step (a scene's neighbour counts keep changing)
-// weighs on every candidate alike. The first round decides between lengths that differ by
-// 20% or more at a scene's start; the later ones compare lengths within a few percent, so
-// each candidate's mean is over four launches (with two, launch-to-launch noise made a
-// later round pick a length 9% slower than the one in use). After a round
-// each kernel switches to the candidate with the lowest mean time if it beats the length
-// in use by more than kTuneMargin. Rounds repeat every `every` steps, as the best length
-// drifts with the neighbour counts (shorter lists win while a scene is sparse).
+// Online autotuner of the force kernel's pair-list length, shared by the single-scene context
+// and the batch. The length never changes the order in which a particle's terms are summed, so
+// the results do not depend on tuning. Tuning starts after `after` steps (a scene's first steps
+// are not representative: cold caches, and an adaptive scene grows over its first few steps). A
+// round is 12 tuning steps (the first round of a tuning run 6); each runs the force and energy
+// kernels once, the force kernel with one candidate length, bracketed by events; the candidates
+// take turns in the order 0 1 2 2 1 0 0 1 2 2 1 0, so a cost that drifts linearly from step to
+// step (a scene's neighbour counts keep changing) weighs on every candidate alike. The first
+// round decides between lengths that differ by 20% or more at a scene's start; the later ones
+// compare lengths within a few percent, so each candidate's mean is over four launches (with
+// two, launch-to-launch noise made a later round pick a length 9% slower than the one in use).
+// After a round the force kernel switches to the candidate with the lowest mean time if it beats
+// the length in use by more than kTuneMargin. Rounds repeat every `every` steps, as the best
+// length drifts with the neighbour counts (shorter lists win while a scene is sparse).
+// What has one form has nothing to choose: the energy kernel at every length, and the force
+// kernel while it runs in several lanes per particle (force_counts is false), which keeps no such
+// list. Their time stands for every length, and a round without a choice is one timed step if
+// no times are there yet, else none, so that steps stay captured.
 struct ListTuner {
   static constexpr int kRound = 12;
   static constexpr int kOrder[kRound] = {0, 1, 2, 2, 1, 0, 0, 1, 2, 2, 1, 0};
   int force = kForceListDefault, energy = kEnergyListDefault;
+  bool force_counts = true;     // the next step's force kernel has lists (set before each step)
   uint rounds_left = 0, skip = 0, every = 0;
   int steps_left = 0, pos = 0, round_len = 0;
   bool pending = false;         // a tuning step's events are not read yet
@@ -643,17 +647,19 @@ struct ListTuner {
     every = every_steps > (uint)kRound ? every_steps : (uint)kRound;
     pos = 0;
     pending = false;
-    clear();
+    clear_sums();
+    for (auto &k : best)
+      for (float &b : k) b = -1.0f;
   }
-  void clear() {
+  void clear_sums() {
     for (int k = 0; k < 2; k++)
       for (int c = 0; c < 3; c++) {
         sum[k][c] = 0.0f;
         cnt[k][c] = 0;
-        best[k][c] = -1.0f;
       }
   }
-  bool tuning() const { return steps_left > 0 && skip == 0; }
+  // the next step is a tuning step
+  bool tuning() const { return steps_left > 0 && skip == 0 && (force_counts || best[0][0] < 0.0f); }
   bool active() const { return steps_left > 0; }
   // pin the lengths (stops tuning); false if a length is not a candidate
   bool set(uint force_len, uint energy_len) {
@@ -671,7 +677,7 @@ struct ListTuner {
     pending = false;
     return true;
   }
-  // kernel 0 = force, 1 = energy; launch(cfg) enqueues one run with that candidate
+  // kernel 0 = force, 1 = energy; launch(cfg) enqueues one run (of the force kernel with that candidate)
   template <class F> void run(int kernel, hipStream_t st, F launch) {
     if (!tuning()) {
       launch(kernel == 0 ? force : energy);
@@ -689,42 +695,41 @@ struct ListTuner {
       skip--;
       return;
     }
-    if (!pending) return;
+    if (!pending && force_counts) return;
     const int c = kOrder[pos % kRound];
-    for (int k = 0; k < 2; k++) {
-      float ms = 0.0f;
-      if (hipEventElapsedTime(&ms, ev[k][0], ev[k][1]) == hipSuccess) {
-        sum[k][c] += ms;
-        cnt[k][c] += 1;
-      }
-    }
-    pending = false;
-    pos++;
-    if (--steps_left == 0) {
-      const int cur[2] = {force, energy};
-      int pick[2] = {cur[0], cur[1]};
-      const float margin = round_len < kRound ? kTuneMargin : kTuneMarginLater;
+    if (pending)
       for (int k = 0; k < 2; k++) {
-        for (int j = 0; j < 3; j++) best[k][j] = cnt[k][j] ? sum[k][j] / (float)cnt[k][j] : -1.0f;
+        float ms = 0.0f;
+        if (hipEventElapsedTime(&ms, ev[k][0], ev[k][1]) != hipSuccess) continue;
         for (int j = 0; j < 3; j++)
-          if (best[k][j] >= 0.0f && best[k][cur[k]] >= 0.0f &&
-              best[k][j] < best[k][cur[k]] * (1.0f - margin) && best[k][j] < best[k][pick[k]])
-            pick[k] = j;
-      }
-      force = pick[0];
-      energy = pick[1];
-      rounds_left--;
-      if (rounds_left > 0) {  // the next round, `every` steps after this one started
-        skip = every - round_len;
-        round_len = kRound;
-        steps_left = kRound;
-        pos = 0;
-        for (int k = 0; k < 2; k++)
-          for (int j = 0; j < 3; j++) {
-            sum[k][j] = 0.0f;
-            cnt[k][j] = 0;
+          if (j == c || k == 1 || !force_counts) {
+            sum[k][j] += ms;
+            cnt[k][j] += 1;
           }
       }
+    pending = false;
+    pos++;
+    steps_left = force_counts ? steps_left - 1 : 0;
+    if (steps_left > 0) return;
+    for (int k = 0; k < 2; k++)
+      for (int j = 0; j < 3; j++)
+        if (cnt[k][j]) best[k][j] = sum[k][j] / (float)cnt[k][j];
+    if (force_counts) {
+      const float margin = round_len < kRound ? kTuneMargin : kTuneMarginLater;
+      int pick = force;
+      for (int j = 0; j < 3; j++)
+        if (best[0][j] >= 0.0f && best[0][force] >= 0.0f && best[0][j] < best[0][force] * (1.0f - margin) &&
+            best[0][j] < best[0][pick])
+          pick = j;
+      force = pick;
+    }
+    rounds_left--;
+    if (rounds_left > 0) {  // the next round, `every` steps after this one started
+      skip = every - (uint)pos;
+      round_len = kRound;
+      steps_left = kRound;
+      pos = 0;
+      clear_sums();
     }
   }
 };
