@@ -228,7 +228,7 @@ struct SphBatch {
   uint *s2p_hash = nullptr, *s2p_cell = nullptr;
   uint *cstart = nullptr, *cend = nullptr;
   SlotBits sb{};
-  uint *newslot = nullptr, *scan_tmp = nullptr;
+  uint *scan_tmp = nullptr;
   unsigned char *aos_dev = nullptr;
   int kbits = 1;
   uint M = 0;      // live particles of all scenes
@@ -656,7 +656,7 @@ int sph_batch_create(int variant, uint32_t n_scenes, const void *sysparams,
             b->alloc(b->cstart, b->total_cell) && b->alloc(b->cend, b->total_cell) &&
             b->alloc(b->sb.split, sph_bit_words(cap)) && b->alloc(b->sb.dead, sph_bit_words(cap)) &&
             b->alloc(b->sb.qual, sph_bit_words(cap)) && b->alloc(b->sb.toff, sph_bit_tiles(cap)) &&
-            b->alloc(b->newslot, cap) && b->alloc(b->cnt, 1) && b->alloc(b->scn, n_scenes) &&
+            b->alloc(b->cnt, 1) && b->alloc(b->scn, n_scenes) &&
             b->alloc(b->Ptab, n_scenes) && b->alloc(b->aos_dev, (size_t)b->max_cap * b->rec) &&
             b->alloc(b->aux.frec, 3 * cap) && b->alloc(b->aux.erec, cap) && b->alloc(b->aux.ez, cap) && b->alloc(b->aux.qpos, cap) &&
             b->alloc(b->aux.nbl, (size_t)SPH_NBL_K * cap) && b->alloc(b->aux.nbl_cnt, cap) &&
