@@ -105,16 +105,36 @@ __global__ __launch_bounds__(BLK) void k_reorder(DevState src, DevState dst,
 // The ring lets lanes with few pairs in one cell go on to the next while others catch up: in a
 // falling dam break (20 pairs) a wave takes 29 rounds of step 2, 41 when rings are emptied after
 // each layer of nine cells and 84 when after each cell; rings of 16 cells take 26 and twice the LDS.
-// From the first cells on of which some lane has a run above 32, step 1 is left out.
+// From the first cells on of which some lane has a run above 32, a cell is looked up at a time and its
+// run taken in parts of 31, each a word in the ring (3D: one pair a round there, or it spills).
 // Bound: VALU issue in the crowded waves, whose chain ends the launch when every wave is resident
 // (dam break), and the L1 misses of the scattered pairs (energy: 2400 lines of 64 bytes per wave).
 // Against a fp32 test of every candidate, us per launch: density 3D-2 500k 133 -> 111, 3D-4 2 to 4M
 // 1105 -> 743, a batch of 3.2M 362 -> 271, of 240k 70 -> 48; energy 176 -> 172, 1700 -> 1114, 492 ->
 // 357, 102 -> 81. One pair per round instead of two: energy 192, 1186, 409 and 83. Emptying the
-// rings after each layer: density 101, 797, 278 and 50, energy 194, 1271, 407 and 88.
+// rings after each layer: density 101, 797, 278 and 50, energy 194, 1271, 407 and 88. Crowded, against
+// the fp32 test and against candidates one by one from the first long run on: still clouds of 45 per
+// cell, density 3D-2 200k 271, 385 -> 246, 3D-4 1M 948, 1168 -> 771, 2D 250k 135, 243 -> 147; energy
+// 306, 388 -> 269, 1240, 1835 -> 1028, 280, 341 -> 204; the falling dam of 262k has such cells too,
+// 21.2 -> 19.3 ms per pass.
 // ---------------------------------------------------------------------------------------
 constexpr int QC = 3;    // cells looked up together
 constexpr uint QR = 8;   // cells of a lane's ring
+
+// Bit 32 - c + x of the word: candidate x of the run [s, e) of c <= 32 may interact; QG in flight.
+template <int QG>
+__device__ inline uint near_bits(const QSelf &qi, const __amdgpu_buffer_rsrc_t qrs, uint s, uint e) {
+  uint w = 0;
+  for (uint j = s; j < e; j += QG) {
+#pragma unroll
+    for (int x = 0; x < QG; x += 2) {
+      const auto q = __builtin_amdgcn_raw_buffer_load_b128(qrs, j * 8u + 8u * x, 0, 0);
+      w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[0], q[1]), 31);
+      w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[2], q[3]), 31);
+    }
+  }
+  return __builtin_bitreverse32(w >> ((s - e) & (QG - 1)));  // the last group's places past the run go
+}
 
 template <int V, bool TWO, class LOAD, class NEAR, class CELL>
 __device__ inline void walk_near(const DevParams &P, const uint c[3], bool valid, const QSelf &qi,
@@ -130,24 +150,26 @@ __device__ inline void walk_near(const DevParams &P, const uint c[3], bool valid
   const bool z0 = c[2] != 0u, z1 = c[2] != nz - 1u;
   uint head = 0, tail = 0;  // cells taken from and put into the ring
   uint m = 0, base = 0;     // the current cell: bits left, entry of bit 0
-  auto take = [&](uint &ent) -> bool {
-    const bool fresh = !m;
+  // the next pair; true when it is a cell's first (parts: of words that hold a part of a cell)
+  auto take = [&](bool parts, uint &ent) -> bool {
+    bool fresh = !m;
     if (fresh) {
       const uint2 w = sh[head++ % QR][t];
-      m = w.x;
+      m = parts ? w.x & ~1u : w.x;
       base = w.y;
+      if (parts) fresh = (w.x & 1u) != 0u;
     }
     ent = base + (uint)__builtin_ctz(m);
     m &= m - 1u;
     return fresh;
   };
-  auto step = [&]() {  // up to two pairs, both loaded before the first is evaluated
+  auto step = [&](bool parts) {  // up to two pairs, both loaded before the first is evaluated
     uint e0, e1;
-    const bool f0 = take(e0);
-    const bool two = TWO && (m | (tail ^ head)) != 0u;
+    const bool f0 = take(parts, e0);
+    const bool two = TWO && !(parts && VT<V>::dim == 3) && (m | (tail ^ head)) != 0u;
     bool f1 = false;
     e1 = e0;
-    if (two) f1 = take(e1);
+    if (two) f1 = take(parts, e1);
     const auto d0 = load(e0), d1 = load(e1);
     if (f0) next_cell();
     near(e0, d0);
@@ -180,7 +202,7 @@ __device__ inline void walk_near(const DevParams &P, const uint c[3], bool valid
     }
     if (it > 1)  // (the lookups are in flight)
       while (__any(tail - head > QR - QC))
-        if (m | (tail ^ head)) step();
+        if (m | (tail ^ head)) step(false);
 #pragma unroll
     for (int k = 0; k < QC; k++) {
       if (s[k] == SPH_EMPTY) s[k] = e[k];
@@ -192,30 +214,34 @@ __device__ inline void walk_near(const DevParams &P, const uint c[3], bool valid
     }
 #pragma unroll
     for (int k = 0; k < QC; k++) {
-      uint w = 0;
-      for (uint j = s[k]; j < e[k]; j += QG) {
-#pragma unroll
-        for (int x = 0; x < QG; x += 2) {
-          const auto q = __builtin_amdgcn_raw_buffer_load_b128(qrs, j * 8u + 8u * x, 0, 0);
-          w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[0], q[1]), 31);
-          w = __builtin_amdgcn_alignbit(w, (uint)sph_near_q(qi, q[2], q[3]), 31);
-        }
-      }
-      // the last group's places past the run go; candidate x of c is then bit 32 - c + x
-      w = __builtin_bitreverse32(w >> ((s[k] - e[k]) & (QG - 1)));
+      const uint w = near_bits<QG>(qi, qrs, s[k], e[k]);
       if (w) sh[tail++ % QR][t] = make_uint2(w, pack_entry(it * QC + k, 0u) + e[k] - 32u);
     }
   }
-  while (m | (tail ^ head)) step();
+  while (m | (tail ^ head)) step(false);
+  if (done == NT) return;
+  // Crowded cells: the run of one cell at a time, in parts of 31 candidates. A word's bit 0, free
+  // then, tells that it holds the cell's first pair.
 #pragma unroll 1
-  for (int o = done * QC; o < VT<V>::nnb; o++) {
-    uint s0 = 0, e0 = 0;
-    if (valid) nb_range<V>(P, o, c, cstart, cend, s0, e0);
-    next_cell();
-    for (uint j = s0; j < e0; j++) {
-      const uint ent = pack_entry(o, j);
-      near(ent, load(ent));
-    }
+  for (int o = done * QC; o <= VT<V>::nnb; o++) {  // past the last cell: what is left in the rings
+    const bool last = o == VT<V>::nnb;
+    uint s0 = 0, e0 = 0, first = 1u;
+    if (valid && !last) nb_range<V>(P, o, c, cstart, cend, s0, e0);
+#pragma unroll 1
+    do {
+      if (s0 < e0) {
+        const uint end = min(e0, s0 + 31u);
+        const uint w = near_bits<QG>(qi, qrs, s0, end);
+        if (w) {
+          sh[tail++ % QR][t] = make_uint2(w | first, pack_entry(o, 0u) + end - 32u);
+          first = 0u;
+        }
+        s0 = end;
+      }
+#pragma unroll 1
+      while (__any(last ? (m | (tail ^ head)) != 0u : tail - head == QR))
+        if (m | (tail ^ head)) step(true);
+    } while (__any(s0 < e0));
   }
 }
 
