@@ -425,6 +425,10 @@ struct SphBatch {
     return true;
   }
 
+  // not after a step that found particles outside their grids: they all go to one cell, and an
+  // entry's place in its cell costs a pass over the cell (sph_bins.hip)
+  bool by_counting() const { return bins.ccount && !cnt_host->err; }
+
   void enqueue_step(uint flags, bool dev = false, uint grid = 0, int lf = -1) {
     const BatchView bv = view();
     const DevParams &P0 = P[0];
@@ -440,7 +444,7 @@ struct SphBatch {
     aux.choose_forms(v, true, M);  // M: the live count at the call's start, also for a graph
     tune.force_counts = !aux.fine_force;
     launch_batch_begin(bv, cnt, st);
-    if (bins.ccount) {
+    if (by_counting()) {
       skeys = sc.keys_alt;
       svals = sc.vals_alt;
       pbegin(SPH_P_HASH);
@@ -522,7 +526,8 @@ struct SphBatch {
   hipGraphExec_t graph_for(uint flags, const int shape[3]) {
     aux.choose_forms(variant, true, M);
     const uint key = (flags & 3u) | ((uint)shape[0] << 2) | ((aux.fine_force ? 0u : (uint)shape[1]) << 4) |
-                     ((parity ? 1u : 0u) << 8) | ((energy_unit_all() ? 1u : 0u) << 9) | (aux.forms() << 10);
+                     ((parity ? 1u : 0u) << 8) | ((energy_unit_all() ? 1u : 0u) << 9) | (aux.forms() << 10) |
+                     ((by_counting() ? 1u : 0u) << 13);
     for (auto &g : graphs)
       if (g.key == key) return g.exec;
     const uint grid = kGridPerCU[shape[0]] * num_cu;

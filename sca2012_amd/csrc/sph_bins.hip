@@ -12,7 +12,9 @@
 //                  record goes there
 // The arrival order differs from run to run, the places do not. Bound: launches and latency up
 // to some 100k particles, HBM beyond (the records move once: 52 bytes read, 64 written).
-// Counting needs a scan over all cells, so a sparse grid keeps the radix sort (sph_use_bins).
+// Counting needs a scan over all cells, so a sparse grid keeps the radix sort (sph_use_bins); so
+// does the step after one that found particles outside the grid, which share a cell however many
+// they are (k_bin_reorder reads a cell once per entry).
 #include <algorithm>
 
 #include "sph_device.h"

@@ -548,7 +548,9 @@ struct SphCtx {
   }
   // hash, sort, cell ranges and reorder of a step: by counting where the grid suits it. The bits
   // that the step's split and merge set start clear.
-  bool by_counting() const { return bins.ccount && sph_use_bins(P.total_cell, n); }
+  // After a step that found particles outside the grid the sort takes over: those particles go to
+  // cell 0, and an entry's place in its cell costs a pass over the cell (sph_bins.hip).
+  bool by_counting() const { return bins.ccount && !rep->c.err && sph_use_bins(P.total_cell, n); }
   void q_bin_step(bool do_split, bool do_merge) {
     if (!nd && !by_counting()) {
       q_hash();
