@@ -14,9 +14,11 @@ against the 8 TB/s HBM peak. roofline.traffic is the HBM bytes per launch of tha
 measured by rocprofv3 PMC runs (FETCH_SIZE, WRITE_SIZE), scaled by what the same counters
 read for a plain device copy of known size (--copy-calibration-mib), read from
 profiles/<kernel>_<workload>_traffic.json. roofline.valu_frac is the fraction of the VALU
-issue peak (one wave64 instruction per SIMD per 4 cycles) that the kernel's VALU
+issue peak (one wave64 instruction per SIMD per 2 cycles) that the kernel's VALU
 instructions (SQ_INSTS_VALU per live particle, profiles/<kernel>_<workload>_valu.json)
-take of its measured launch time -- the neighbour kernels' secondary bound.
+take of its measured launch time -- the neighbour kernels' secondary bound. The counters
+are of certain steps of the workload (the default run's timed ones); a run that times
+others reports null.
 full_run: the workload's whole configured step count (2000 steps for the 3D-2 dam break)
 from the seeded start on a fresh context, beside the K-step window.
 cpu_baseline: the fp32 CPU oracle (a restatement of the reference kernels, OpenMP over
@@ -153,10 +155,11 @@ def measured_traffic(kernel, workload):
     return t["fetch_bytes_per_launch"] + t["write_bytes_per_launch"]
 
 
-# MI355X VALU issue peak: 256 CUs x 4 SIMDs, one wave64 VALU instruction per SIMD every 4
-# cycles (16 lanes per SIMD) at 2.4 GHz = 614.4e9 wave-instructions/s, i.e. 78.6 TFLOP/s
-# of non-packed fp32 FMA.
-VALU_PEAK_WAVE_INST_S = 256 * 4 * 2.4e9 / 4
+# MI355X VALU issue peak: 256 CUs x 4 SIMDs, one wave64 VALU instruction per SIMD every 2
+# cycles at 2.4 GHz = 1228.8e9 wave-instructions/s, i.e. 157.3 TFLOP/s of fp32 FMA. Measured
+# with independent chains in every wave: v_fma, v_add, v_mul_f32, v_add_u32, v_and_b32 and
+# v_mov_b32 0.98e12 to 1.07e12 per second, v_max_f32 and v_dot2_i32_i16 0.6e12 (4 cycles).
+VALU_PEAK_WAVE_INST_S = 256 * 4 * 2.4e9 / 2
 
 
 def measured_valu(kernel, workload):
@@ -169,21 +172,23 @@ def measured_valu(kernel, workload):
         return json.load(f)
 
 
-def valu_fraction(kernel, workload, mean_live, mean_launch_ms):
+def valu_fraction(kernel, workload, mean_live, mean_launch_ms, steps):
     """Fraction of the VALU issue peak: the profiled VALU instructions per live particle x the
-    live particles of the timed steps, over the launch time measured live."""
+    live particles of the timed steps, over the launch time measured live. `steps`: first and
+    last timed step, counted from 1; None unless they are the profiled ones (a particle's
+    neighbours, and with them its instructions, differ from step to step)."""
     v = measured_valu(kernel, workload)
-    if not v or not mean_launch_ms:
+    if not v or not mean_launch_ms or v.get("steps") != list(steps):
         return None, None
     insts = v["valu_insts_per_particle"] * mean_live
     return insts / (mean_launch_ms * 1e-3) / VALU_PEAK_WAVE_INST_S, insts
 
 
 def tune_in_warmup(obj, warmup, lists=None):
-    """Place the pair-list autotuner's first round (six tuning steps) at the end of the
-    warm-up; its later rounds (twelve steps, every 128 steps) fall in the timed steps, as in
-    any long run (fewer than 7 warm-up steps: the library's own schedule). `lists` = "F,E"
-    pins the lengths instead."""
+    """Place the pair-list autotuner's first round (six tuning steps; one where the force
+    kernel has no lists) at the end of the warm-up; its later rounds (twelve steps, every 128
+    steps, where there are lists) fall in the timed steps, as in any long run (fewer than 7
+    warm-up steps: the library's own schedule). `lists` = "F,E" pins the lengths instead."""
     if lists:
         f, e = (int(x) for x in lists.split(","))
         obj.set_lists(f, e)
@@ -253,7 +258,7 @@ def run_batched(args, w):
     if args.groups_per_cu >= 0:
         b.set_launch(args.groups_per_cu)
     if not args.lists and args.groups_per_cu < 0 and args.warmup >= 24:
-        # one round of each tuned dimension (grid, force list, energy list) in the warm-up
+        # one round of each dimension (grid, force list, energy list) in the warm-up
         b.autotune(0xffffffff, after=args.warmup - 20, every=128)
     for s_, (_, a) in enumerate(tanks):
         b.upload(s_, a)
@@ -564,7 +569,8 @@ def main():
 
     traffic = measured_traffic(dominant, args.workload)
     mean_launch_ms = dom_ms / dom_launches if dom_launches else None
-    valu_frac, valu_insts = valu_fraction(dominant, args.workload, mean_n, mean_launch_ms)
+    valu_frac, valu_insts = valu_fraction(dominant, args.workload, mean_n, mean_launch_ms,
+                                            (args.warmup + 1, args.warmup + args.steps))
 
     # the whole configured run (all of its steps, from the seeded start) on a fresh context:
     # the rate over the full trajectory, beside the rate of the timed window

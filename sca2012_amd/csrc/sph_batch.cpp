@@ -6,24 +6,25 @@
 //
 // Layout of a batch of S scenes:
 //   cells     scene s owns the global cells [cell_base_s, cell_base_s + total_cell_s);
-//             a particle's sort key is cell_base_s + its reference hash, so one radix sort
-//             orders all scenes, scene after scene, cells ascending within a scene.
-//   slots     the slot word of a particle is s << 24 | its slot within scene s. The sort
-//             input packs the scenes densely (scene s at [first_s, first_s + n_s)), so ties
-//             stay in ascending slot within each scene, as in the single-scene sort.
+//             a particle's cell is cell_base_s + its reference hash, so one ordering by cell (by
+//             counting, sph_bins.hip, or on sparse grids a radix sort) orders all scenes, scene
+//             after scene, cells ascending within a scene.
+//   slots     the slot word of a particle is s << 24 | its slot within scene s. Slots are also
+//             numbered densely over the scenes (scene s at [first_s, first_s + n_s)), so ties
+//             stay in ascending slot within each scene, as in a single scene.
 //   entries   the SoA state arrays hold live entries [0, M) in cell order after the
 //             reorder, then the split children of all scenes (scene by scene, in parent
-//             rank order); merge victims stay as removed entries until the next sort.
+//             rank order); merge victims stay as removed entries until the next step's order.
 // Split capacity (floor((cap_s - n_s)/(n_split - 1)) parents) and merge groups are decided
 // per scene, so each scene evolves exactly as it would in its own SphCtx.
 //
 // Two ways to run a step:
-//   graph     (default) the whole step is one captured hipGraph: every per-item phase is a
-//             persistent launch (a fixed grid of workgroups per CU, each looping over blocks
-//             of 256 items) that reads its item count from the device counters, so nothing
-//             in the step depends on the host's view of the counts and the host launches
-//             step after step without waiting. A launch tuner picks the workgroups per CU
-//             and the pair-list lengths by timing whole steps.
+//   graph     (default) the whole step is one captured hipGraph: every launch reads its item
+//             count from the device counters, so nothing in the step depends on the host's view
+//             of the counts and the host launches step after step without waiting. Launches are
+//             sized by their buffers' bounds; a launch tuner, timing whole steps, also tries
+//             persistent ones (a fixed grid of workgroups per CU, each looping over blocks of
+//             256 items) and the force kernel's pair-list lengths.
 //   stream    the kernels launched one by one per step, sized by the counts the host read
 //             at the end of the previous step (one synchronisation per step).
 // Both give the same bits for every scene: the launch shape never changes what an item

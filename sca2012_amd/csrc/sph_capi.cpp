@@ -2,11 +2,14 @@
 // that owns every device buffer, the phase entry points and the whole step.
 //
 // Per-step device work (one HIP stream, no host round trip until the end of the step):
-//   hash -> radix sort -> cell ranges + reorder into cell order -> density -> force ->
-//   integrate -> [density grid -> normals -> marching cubes] -> energy ->
-//   [split] -> [merge -> renumber survivors]
+//   particles counted into cells -> cell table -> place -> reorder into cell order
+//   (sph_bins.hip; a sparse grid, and the phase calls: hash -> radix sort -> cell ranges +
+//   reorder) -> density -> force -> integrate -> [density grid -> normals -> marching cubes] ->
+//   energy -> [split] -> [merge -> renumber survivors]
 // Counts that change inside the step (after split and merge) stay on the device; kernels
-// read them and are launched over host-side upper bounds.
+// read them and are launched over host-side upper bounds. A step that repeats is launched as one
+// captured graph, and a kernel at its end reports the counters into pinned memory that the host
+// polls (graph_step, sync).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

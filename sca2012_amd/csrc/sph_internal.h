@@ -110,15 +110,19 @@ struct Aux {
   // For n live particles of a scene or of a batch's scenes together. Several lanes per
   // particle shorten the chain of dependent loads and cost more instructions, so density and
   // energy are chosen by whether n threads fill the GPU. Measured (one thread -> several
-  // lanes, us): density, a falling dam 3D-2 27k 40 -> 32, 43k 44 -> 44, 65k 51 -> 59, 93k 61 -> 78;
-  // a collision 3D-4 27k 44 -> 32, 76k 52 -> 73; the line lies above 65k because sparse scenes
-  // keep several lanes longer (a calm 3D-2 block of 33k to 65k: 14). 2D 20k 14 -> 12, 37k
+  // lanes, us): density, a falling dam 3D-2 36k 28.9 -> 24.5, 47k 29.2 -> 27.6, 55k 29.2 -> 29.6,
+  // 64k 29.2 -> 32.0, an adaptive one 24k 35.0 -> 25.0, 45k 38.3 -> 34.3; a collision 3D-4 43k
+  // 49.3 -> 54.5, 53k 66.7 -> 62.5, 64k 61.6 -> 73.7. The two meet near 53k; the line lies at 66k
+  // because a rollout chooses by its bound, 65,536 entries for 32^3 particles of which half live
+  // at first (36k still: 28.1 -> 24.0). 2D 20k 14 -> 12, 37k
   // 15 -> 15. Energy 3D-2 65k 63 -> 53, 93k 78 -> 69, 128k 101 -> 91, 330k 112 -> 123; 3D-4 76k
   // 108 -> 73, 124k 124 -> 103; 2D 67k 19 -> 16. Force evaluates the same pairs either way, with
   // one pair's registers instead of
   // four: 3D-2 25k 36 -> 15, 498k 107 -> 91; 3D-4 506k 219 -> 134, 1.7M 501 -> 392, 4.2M
   // shrinking to 2M 732 -> 717; 2D 66k 15 -> 13, 264k 24 -> 30; in a batch, whose lanes each
-  // load their scene's parameters, 126k 49 -> 39, 400k 41 -> 52.
+  // load their scene's parameters, 126k 49 -> 39, 400k 41 -> 52. Above the 3D line of a single
+  // scene either is the faster: a young dam 6.9M 475 -> 534, falling 8.6M 1118 -> 1039, adaptive
+  // 12.0M 1332 -> 1198, a collision 3D-4 6.7M 1509 -> 1419, 9.0M 2212 -> 1798.
   void choose_forms(int variant, bool batch, uint n) {
     const bool d3 = variant != SPH_V2D;
     fine_density = n <= (d3 ? 66000u : 32000u);
