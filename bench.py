@@ -239,11 +239,35 @@ def batch_stream_run(args, w, tanks, caps, flags):
                 phase_ms=phase_ms, phase_steps=phase_steps, lists=tuned[:2])
 
 
+def batch_one_by_one(args, variant, tanks, caps, flags):
+    """The same tanks, one context each, stepped one after another (same warm-up)."""
+    ctxs = []
+    for (p, a), c in zip(tanks, caps):
+        g = sa.SPHContext(variant, p, c, max_triangles=1)
+        tune_in_warmup(g, args.warmup, args.lists)
+        g.upload(a)
+        ctxs.append(g)
+    for g in ctxs:
+        for _ in range(args.warmup):
+            g.step(flags)
+    steps = max(1, min(args.steps, 20))
+    t0 = time.perf_counter()
+    for k in range(steps):
+        for g in ctxs:
+            g.step(flags)
+    wall = time.perf_counter() - t0
+    value = len(tanks) * steps / wall
+    log("one by one: %.4g scene-steps/s (%d steps)" % (value, steps))
+    for g in ctxs:
+        g.close()
+    return value, steps
+
+
 def run_batched(args, w):
     """Batched tanks: scene-steps/s of graph steps over all tanks (each step one captured
-    hipGraph of persistent launches, the host launching step after step), beside the same
-    batch with stream steps (kernels launched one by one, one synchronisation per step) and
-    the same tanks stepped one after another through their own single-scene contexts."""
+    hipGraph, the host launching step after step), beside the same batch with stream steps
+    (kernels launched one by one, one synchronisation per step) and the same tanks stepped one
+    after another through their own single-scene contexts."""
     variant, flags = w["variant"], w["flags"]
     sizes, tanks = w["build"]()
     caps = [int(w["capacity_factor"] * n) for n in sizes]
@@ -287,26 +311,11 @@ def run_batched(args, w):
     log("stream steps: %.4g scene-steps/s, phases over %d further steps (ms/step): %s" % (
         stream_value, phase_steps, phase_ms))
 
-    # the same tanks, one context each, stepped one after another (same warm-up)
-    ctxs = []
-    for (p, a), c in zip(tanks, caps):
-        g = sa.SPHContext(variant, p, c, max_triangles=1)
-        tune_in_warmup(g, args.warmup, args.lists)
-        g.upload(a)
-        ctxs.append(g)
-    for g in ctxs:
-        for _ in range(args.warmup):
-            g.step(flags)
-    seq_steps = max(1, min(args.steps, 20))
-    t0 = time.perf_counter()
-    for k in range(seq_steps):
-        for g in ctxs:
-            g.step(flags)
-    seq_wall = time.perf_counter() - t0
-    seq_value = ns * seq_steps / seq_wall
-    log("one by one: %.4g scene-steps/s (%d steps)" % (seq_value, seq_steps))
-    for g in ctxs:
-        g.close()
+    one_by_one = None
+    if args.one_by_one:
+        seq_value, seq_steps = batch_one_by_one(args, variant, tanks, caps, flags)
+        one_by_one = {"value": seq_value, "unit": "scene-steps/s", "steps": seq_steps,
+                      "speedup_batched": value / seq_value}
 
     cpu = None
     if not args.no_cpu:
@@ -356,8 +365,7 @@ def run_batched(args, w):
             "particle_steps_per_s_approx": mean_n * args.steps / wall,
             "parallelism": "single-gpu",
         },
-        "one_by_one": {"value": seq_value, "unit": "scene-steps/s", "steps": seq_steps,
-                       "speedup_batched": value / seq_value},
+        "one_by_one": one_by_one,
         "stream_steps": {"value": stream_value, "unit": "scene-steps/s",
                          "ms_per_step": stream["wall"] * 1e3 / args.steps,
                          "note": "the same batch with the kernels launched one by one, one "
@@ -485,6 +493,8 @@ def main():
                          "sized by the buffers' bounds; 4, 8, 16: persistent) instead of autotuning")
     ap.add_argument("--no-full-run", dest="full_run", action="store_false",
                     help="skip the run over all of the workload's configured steps")
+    ap.add_argument("--no-one-by-one", dest="one_by_one", action="store_false",
+                    help="batched workload: without the leg that steps every tank in a context of its own")
     ap.add_argument("--copy-calibration-mib", type=int, default=0,
                     help="after the run, copy a buffer of this many MiB 5 times on the device "
                          "(the plain copy kernel that scales the PMC byte counters)")
